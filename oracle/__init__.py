@@ -40,7 +40,7 @@ def build(ref: bool | None = None) -> None:
     """Compile liboracle.so and, when the reference tree is present, _ref."""
     subprocess.run(["make", "-s", "-C", HERE, "liboracle.so"], check=True)
     if ref is None:
-        ref = os.path.isdir(REFERENCE_TREE)
+        ref = os.path.isdir(os.path.join(REFERENCE_TREE, "src"))  # an empty mount point is no tree
     if ref:
         subprocess.run(["make", "-s", "-j8", "-C", HERE, "ref", f"REF={REFERENCE_TREE}"],
                        check=True)
