@@ -17,6 +17,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "liboracle.so")
 REF_PATH = os.path.join(HERE, "_ref", "libhyref.so")
 REFERENCE_TREE = "/root/reference"
+if not os.path.isdir(os.path.join(REFERENCE_TREE, "src")):
+    REFERENCE_TREE = os.path.join(REFERENCE_TREE, "absent")  # an empty mount point is no tree
 
 _d = C.c_double
 _u64 = C.c_uint64
@@ -40,7 +42,7 @@ def build(ref: bool | None = None) -> None:
     """Compile liboracle.so and, when the reference tree is present, _ref."""
     subprocess.run(["make", "-s", "-C", HERE, "liboracle.so"], check=True)
     if ref is None:
-        ref = os.path.isdir(os.path.join(REFERENCE_TREE, "src"))  # an empty mount point is no tree
+        ref = os.path.isdir(REFERENCE_TREE)
     if ref:
         subprocess.run(["make", "-s", "-j8", "-C", HERE, "ref", f"REF={REFERENCE_TREE}"],
                        check=True)
