@@ -144,6 +144,8 @@ struct hy_pm_ctx {
     uint32_t* xcounts = nullptr;   // x-plane bins (N)
     uint32_t* xoffsets = nullptr;  // N+1
     unsigned long long* mass_digits = nullptr;  // per box: exact deposited-mass digit counters
+    uint64_t* dense_list = nullptr;             // binary64 deposit jobs of the tiles above its LDS capacity
+    uint64_t even_cap = 0, plan_cap = 0;        // evenly cut and planned jobs the list holds
     unsigned long long* mass_waves = nullptr;   // per deposit wave: its exact mass (binary64: digit window,
                                                 // binary32: two digit sums of its 32.32 cells)
     double* mass_total = nullptr;
@@ -265,7 +267,7 @@ void raise_errors(uint32_t e) {
     if (e & ERR_MASS_INVALID) fail(HY_EINVAL, "CIC masses must be finite and non-negative");
     if (e & ERR_STALE_KEYS) fail(HY_ELOGIC, "reused bucket keys do not match the input positions");
     if (e & ERR_COORDINATE) fail(HY_ELOGIC, "CIC bounded coordinate escaped the mesh domain");
-    if (e & ERR_SCRATCH) fail(HY_ERUNTIME, "deposit fallback scratch exhausted");
+    if (e & ERR_SCRATCH) fail(HY_ERUNTIME, "bucket sort scratch exhausted");
     if (e & ERR_FIELD_NONFINITE) fail(HY_EINVAL, "CIC centered-gradient potential must be finite");
     if (e & ERR_FORCE_NONFINITE) fail(HY_EOVERFLOW, "CIC centered-gradient gathered acceleration is non-finite");
     if (e & ERR_MOMENTUM_NONFINITE) fail(HY_EOVERFLOW, "Leapfrog kick input is not finite");
@@ -392,6 +394,26 @@ struct DepositPlan {
     hy::DepParams P;
 };
 
+// Quanta of the exact cell-mass sum (SaQuanta): q3 is the digit boundary at or
+// above 2^-112 of the mass unit's power of two.
+hy::SaQuanta sa_quanta(double unit) {
+    hy::SaQuanta q{};
+    q.max = -1.0;
+    const int e = std::isfinite(unit) && unit > 0.0 ? std::ilogb(unit) : -1024;
+    if (e < -700 || e > 700) return q;  // every mass to the counters
+    q.base = (e - 112 + 1074 + 31) / 32;
+    const int e3 = 32 * q.base - 1074;
+    auto splitter = [](int x) { return std::ldexp(1.5, 52 + x); };
+    q.c1 = splitter(e3 + 80);
+    q.c2 = splitter(e3 + 40);
+    q.c3 = splitter(e3);
+    q.i1 = std::ldexp(1.0, -(e3 + 80));
+    q.i2 = std::ldexp(1.0, -(e3 + 40));
+    q.i3 = std::ldexp(1.0, -e3);
+    q.max = std::ldexp(1.0, 40 + e3 + 80);
+    return q;
+}
+
 DepositPlan plan_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const double* z,
                          const double* masses, double uniform, double Min, double shift = 0.0) {
     const double dx = c->geom.dx;
@@ -428,11 +450,16 @@ DepositPlan plan_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double
         P.norm_exp = e - 64;
     }
     P.direct = (exact_mean && std::isfinite(inv_volume) && inv_volume > 0.0) ? 1 : 0;
-    P.mass_digits = c->mass_digits;
-    P.mass_waves = c->mass_waves;
+    P.sa = sa_quanta(c->mass_unit);
+    P.dense_count = c->mass_digits + (uint64_t)hy::SA_WORDS * c->nbox;
+    P.dense_list = c->dense_list;
     P.scratch = c->scratch;
     P.scratch_cap = c->scratch_cap;
-    P.scratch_cursor = c->scratch_cursor;
+    P.even_cap = (uint32_t)c->even_cap;
+    P.plan_cap = (uint32_t)c->plan_cap;
+    P.scratch_cursor = P.dense_count + 2;
+    P.mass_digits = c->mass_digits;
+    P.mass_waves = c->mass_waves;
     P.err = c->err;
     (void)n;
     return {Min, P};
@@ -457,12 +484,23 @@ long double mass_tol_factor(const hy_pm_ctx* c, uint64_t n) {
 // carried in a capacity layout, whose overflow prefix is ovf).
 void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, bool status_check = true,
                     const uint32_t* start = nullptr, const uint32_t* ovf = nullptr) {
-    fill_u32(c, c->mass_digits, (uint64_t)hy::SA_WORDS * c->nbox * 2);
-    if (c->prec == HY_PREC_FP64)
-        hipLaunchKernelGGL((c->geom.T == 16 ? hy::k_deposit<double, 16> : hy::k_deposit<double, 0>),
-                           dim3(c->ntiles * c->nbox), dim3(hy::DEP_THREADS), 0, c->stream, P,
-                           static_cast<double*>(c->R));
-    else {
+    // with the two job counts and the scratch cursor of the deposit behind them
+    fill_u32(c, c->mass_digits, ((uint64_t)hy::SA_WORDS * c->nbox + 3) * 2);
+    if (c->prec == HY_PREC_FP64) {
+        auto launch = [&](auto kern, uint64_t blocks) {
+            hipLaunchKernelGGL(kern, dim3((uint32_t)blocks), dim3(hy::DEP_THREADS), 0, c->stream, P,
+                               static_cast<double*>(c->R));
+        };
+        const uint64_t tiles = c->ntiles * c->nbox, jobs = std::min<uint64_t>(c->even_cap, 512);
+        const bool t16 = c->geom.T == 16;
+        if (P.masses) {
+            launch(t16 ? hy::k_deposit<16, true, false> : hy::k_deposit<0, true, false>, tiles);
+            launch(t16 ? hy::k_deposit<16, true, true> : hy::k_deposit<0, true, true>, jobs);
+        } else {
+            launch(t16 ? hy::k_deposit<16, false, false> : hy::k_deposit<0, false, false>, tiles);
+            launch(t16 ? hy::k_deposit<16, false, true> : hy::k_deposit<0, false, true>, jobs);
+        }
+    } else {
         hy::DepFxParams Q{P, c->mass_unit, std::ldexp(c->mass_unit, -32), c->rec,
                           P.masses ? c->rec_mass : nullptr, start ? start : c->offsets, c->counts, ovf,
                           c->nball};
@@ -730,7 +768,7 @@ void check_mass(hy_pm_ctx* c, double input, double deposited, uint64_t n) {
         fail(HY_ERUNTIME, "CIC deposited mass violates the forward-error bound");
 }
 
-// Deposit stage: bucketize, deposit (+ retry with a larger fallback scratch).
+// Deposit stage: bucketize, deposit.
 // carried_rec (binary32, asynchronous): deposit the records the previous
 // fused step wrote into its capacity layout for these positions.  rec_out:
 // also lay out the capacities of the records this step's gather writes.
@@ -767,31 +805,15 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
     mark(c, HY_STAGE_DEPOSIT + 1);
     c->last_input_mass = Min;
     if (!sync) return;
-    for (int attempt = 0;; ++attempt) {
+    for (;;) {
         const auto st = fetch_status(c);
         if (carried && (st.err & hy::ERR_STALE_KEYS)) {
             // the positions changed since the keys were made: route them afresh
-            // (coordinate and scratch errors of the stale routing are its artefacts)
+            // (coordinate errors of the stale routing are its artefacts)
             raise_errors(st.err & (hy::ERR_POSITION_NONFINITE | hy::ERR_MASS_INVALID));
             carried = false;
             reset_status(c);
             bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, false, masses, nullptr, shift);
-            plan = plan_deposit(c, n, x, y, z, masses, uniform, Min, shift);
-            launch_deposit(c, plan.P);
-            continue;
-        }
-        if ((st.err & hy::ERR_SCRATCH) && attempt < 3) {
-            // grow the fallback scratch (records of the hot tiles) and redo the
-            // deposit; errors the retry would clear are raised first
-            raise_errors(st.err & ~(hy::ERR_SCRATCH | hy::ERR_MASS_CONSERVATION | hy::ERR_ROUTING));
-            const uint64_t grow = c->scratch_cap * 2;
-            void* p = nullptr;
-            hip_check(hipMalloc(&p, grow * sizeof(uint64_t)), "hipMalloc scratch");
-            c->allocations.push_back(p);
-            c->device_bytes += grow * sizeof(uint64_t);
-            c->scratch = static_cast<uint64_t*>(p);
-            c->scratch_cap = grow;
-            reset_status(c);
             plan = plan_deposit(c, n, x, y, z, masses, uniform, Min, shift);
             launch_deposit(c, plan.P);
             continue;
@@ -1052,7 +1074,15 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         c->grand_total = (uint32_t*)c->alloc(16);
         c->xcounts = (uint32_t*)c->alloc((size_t)N * 4);
         c->xoffsets = (uint32_t*)c->alloc(((size_t)N + 1) * 4);
-        c->mass_digits = (unsigned long long*)c->alloc((uint64_t)hy::SA_WORDS * c->nbox * 8);
+        c->mass_digits = (unsigned long long*)c->alloc(((uint64_t)hy::SA_WORDS * c->nbox + 3) * 8);
+        if (c->prec == HY_PREC_FP64) {
+            // one job per tile, or at most 64 and one per DEP_JOB_RECORDS records
+            // of the tile; a record lies in at most eight tiles
+            const uint64_t tiles = c->ntiles * c->nbox;
+            c->even_cap = std::min<uint64_t>(64 * tiles, tiles + 8 * cap / hy::DEP_JOB_RECORDS);
+            c->plan_cap = 64 * tiles < cap / 16 + 4096 ? 64 * tiles : cap / 16 + 4096;
+            c->dense_list = (uint64_t*)c->alloc((c->even_cap + c->plan_cap) * 8);
+        }
         const uint64_t wave_words = c->prec == HY_PREC_FP64 ? hy::SA_WAVE_WORDS : 2;  // window, or digit-sum pair
         c->mass_waves = (unsigned long long*)c->alloc(wave_words * hy::SA_WAVES_PER_TILE * c->ntiles * c->nbox * 8);
         c->mass_total = (double*)c->alloc(std::max<uint64_t>(2, c->nbox) * 8);

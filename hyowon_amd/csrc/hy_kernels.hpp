@@ -499,13 +499,6 @@ constexpr int DEP_MAX_T = 16;
 constexpr int DEP_EXT = (DEP_MAX_T + 1) * (DEP_MAX_T + 1) * (DEP_MAX_T + 1);  // 4913
 constexpr int DEP_NRANGES = 20;
 
-template <typename T>
-struct DepCfg;
-template <>
-struct DepCfg<float> { static constexpr int CAP = 2048; };
-template <>
-struct DepCfg<double> { static constexpr int CAP = 1024; };
-
 // ---------------------------------------------------------------------------
 // Exact deposited mass: the reference sums every cell's mass with
 // ExactPositiveDoubleSum (src/gravity/pm_solver.cpp:132-180).  Here each box
@@ -570,30 +563,9 @@ __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
     return v + (row > 0 ? r0 : 0u) + (row > 1 ? r1 : 0u) + (row > 2 ? r2 : 0u);
 }
 
-__device__ __forceinline__ int wave_min_i32(int v) {
-    constexpr uint32_t big = 0x7fffffffu;
-    v = min(v, (int)dpp_u32<0x111>((uint32_t)v, big));
-    v = min(v, (int)dpp_u32<0x112>((uint32_t)v, big));
-    v = min(v, (int)dpp_u32<0x114>((uint32_t)v, big));
-    v = min(v, (int)dpp_u32<0x118>((uint32_t)v, big));
-    int m = __builtin_amdgcn_readlane(v, 15);
-#pragma unroll
-    for (int r = 31; r < 64; r += 16) m = min(m, __builtin_amdgcn_readlane(v, r));
-    return m;
-}
-
-// A lane's running sum of cell masses: a 192-bit integer (a2:a1:a0) in
-// units of the binary position 32*base (base < 0: empty), base one digit
-// below the first mass it took.  A mass m 2^s (s its bit position, 53-bit m)
-// is added exactly when 0 <= s - 32 base <= 127; others go to the counters d
-// directly.  sa_acc_flush reduces the wave's sums (DPP wave sums) into the
-// wave's digit window.
-struct SaAcc {
-    int base = -1;
-    uint64_t a0 = 0, a1 = 0, a2 = 0;
-};
-
-__device__ __forceinline__ void sa_acc_add(SaAcc& a, unsigned long long* d, double x) {
+// Adds x exactly to the counters d (flagging a value that is not finite and
+// non-negative).
+__device__ __forceinline__ void sa_add_direct(unsigned long long* d, double x) {
     if (x == 0.0) return;
     if (!(x > 0.0) || !isfinite(x)) {
         atomicOr(&d[SA_DIGITS], 1ull);
@@ -604,66 +576,93 @@ __device__ __forceinline__ void sa_acc_add(SaAcc& a, unsigned long long* d, doub
     const uint64_t frac = bits & ((1ull << 52) - 1ull);
     const uint64_t mant = e ? (frac | (1ull << 52)) : frac;
     const int shift = e ? e - 1 : 0;
-    if (a.base < 0) a.base = (shift >> 5) > 0 ? (shift >> 5) - 1 : 0;
-    const int s = shift - 32 * a.base;
-    if (s >= 0 && s <= 127) {
-        const int off = s & 63;
-        const uint64_t lo = mant << off;
-        const uint64_t hi = off ? mant >> (64 - off) : 0ull;
-        if (s < 64) {
-            a.a0 += lo;
-            const uint64_t c0 = a.a0 < lo ? 1ull : 0ull;
-            const uint64_t t = a.a1 + hi;
-            const uint64_t c1 = t < hi ? 1ull : 0ull;
-            a.a1 = t + c0;
-            a.a2 += c1 + (a.a1 < c0 ? 1ull : 0ull);
-        } else {
-            a.a1 += lo;
-            a.a2 += hi + (a.a1 < lo ? 1ull : 0ull);
-        }
+    const int limb = shift >> 5, o = shift & 31;
+    const uint64_t l = mant << o, h = o ? mant >> (64 - o) : 0ull;
+    if ((uint32_t)l) atomicAdd(&d[limb], (unsigned long long)(uint32_t)l);
+    if ((uint32_t)(l >> 32) && limb + 1 < SA_DIGITS) atomicAdd(&d[limb + 1], (unsigned long long)(uint32_t)(l >> 32));
+    if (h && limb + 2 < SA_DIGITS) atomicAdd(&d[limb + 2], (unsigned long long)h);
+}
+
+// A lane's running sum of cell masses as three binary64 sums of multiples of
+// q1 = 2^80 q3, q2 = 2^40 q3 and q3 = 2^(32 base - 1074): adding and
+// subtracting 1.5 2^52 q rounds a value to a multiple of q, so a mass splits
+// into three parts whose sums stay exact integers of their quantum (parts of at
+// most 2^40 quanta, at most 4096 cells per wave).  Fifteen additions per cell
+// instead of the 60-odd integer instructions of a 192-bit accumulator.  A
+// mass above 2^40 q1 or with bits below q3 (the host places q3 so that this
+// leaves at least 2^-29 .. 2^8 mass units) goes to the box's counters.
+struct SaQuanta {
+    double c1, c2, c3;     // 1.5 2^52 q
+    double i1, i2, i3;     // 1 / q
+    double max;            // 2^40 q1; negative: every mass goes to the counters
+    int base;              // digit of q3
+};
+
+struct SaAcc {
+    double s1 = 0.0, s2 = 0.0, s3 = 0.0;
+};
+
+__device__ __forceinline__ void sa_acc_add(SaAcc& a, const SaQuanta& q, unsigned long long* d, double x) {
+    const double t1 = (x + q.c1) - q.c1, r1 = x - t1;
+    const double t2 = (r1 + q.c2) - q.c2, r2 = r1 - t2;
+    const double t3 = (r2 + q.c3) - q.c3;
+    if (x >= 0.0 && x <= q.max && r2 == t3) {
+        a.s1 += t1;
+        a.s2 += t2;
+        a.s3 += t3;
     } else {
-        const int limb = shift >> 5, o = shift & 31;
-        const uint64_t l = mant << o, h = o ? mant >> (64 - o) : 0ull;
-        if ((uint32_t)l) atomicAdd(&d[limb], (unsigned long long)(uint32_t)l);
-        if ((uint32_t)(l >> 32) && limb + 1 < SA_DIGITS) atomicAdd(&d[limb + 1], (unsigned long long)(uint32_t)(l >> 32));
-        if (h && limb + 2 < SA_DIGITS) atomicAdd(&d[limb + 2], (unsigned long long)h);
+        sa_add_direct(d, x);
     }
 }
 
-// Every lane of the wave calls this (the wave reductions need all lanes): the
-// wave's window (base, SA_WAVE_WIN digits) goes to out from lanes
-// 0..SA_WAVE_WIN; lanes whose sums start more than 2 digits above the wave's
-// lowest add theirs to d directly.
-__device__ __forceinline__ void sa_acc_flush(const SaAcc& a, unsigned long long* d, unsigned long long* out) {
-    const int b0 = wave_min_i32(a.base < 0 ? 0x7fffffff : a.base);
+// Wave-wide sum of binary64 values whose sums are exact (integers of one
+// quantum below 2^53), the same in every lane; DPP as wave_sum_u64.
+__device__ __forceinline__ double wave_sum_exact(double x) {
+    auto shifted = [](uint64_t v, auto ctrl) { return __longlong_as_double((long long)dpp_u64<decltype(ctrl)::value>(v)); };
+    auto bits = [](double v) { return (uint64_t)__double_as_longlong(v); };
+    x += shifted(bits(x), std::integral_constant<int, 0x111>{});
+    x += shifted(bits(x), std::integral_constant<int, 0x112>{});
+    x += shifted(bits(x), std::integral_constant<int, 0x114>{});
+    x += shifted(bits(x), std::integral_constant<int, 0x118>{});
+    const int lo = (int)(uint32_t)bits(x), hi = (int)(uint32_t)(bits(x) >> 32);
+    double s = 0.0;
+#pragma unroll
+    for (int r = 15; r < 64; r += 16)
+        s += __longlong_as_double((long long)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, r) << 32) |
+                                              (uint32_t)__builtin_amdgcn_readlane(lo, r)));
+    return s;
+}
+
+// The wave's sum as six 32-bit digits from q.base, the same in every lane;
+// every lane of the wave calls this.
+__device__ __forceinline__ void sa_acc_digits(const SaAcc& a, const SaQuanta& q, uint64_t (&v)[6]) {
+    // s1 2^80 + s2 2^40 + s3 in units of q3: parts may be negative, the sum is not
+    const double s1 = wave_sum_exact(a.s1), s2 = wave_sum_exact(a.s2), s3 = wave_sum_exact(a.s3);
+    const __int128 low = (__int128)(long long)(s3 * q.i3) + ((__int128)(long long)(s2 * q.i2) << 40);
+    const __int128 mid = ((__int128)(long long)(s1 * q.i1) << 16) + (low >> 64);
+    const uint64_t a0 = (uint64_t)low, a1 = (uint64_t)mid, a2 = (uint64_t)(mid >> 64);
+    v[0] = (uint32_t)a0;
+    v[1] = a0 >> 32;
+    v[2] = (uint32_t)a1;
+    v[3] = a1 >> 32;
+    v[4] = (uint32_t)a2;
+    v[5] = a2 >> 32;
+}
+
+// The wave's window (base, SA_WAVE_WIN digits; base -1: no mass) to out, from
+// lanes 0..SA_WAVE_WIN.
+__device__ __forceinline__ void sa_acc_flush(const SaAcc& a, const SaQuanta& q, unsigned long long* out) {
+    uint64_t v[6];
+    sa_acc_digits(a, q, v);
     const uint32_t lane = lane_id();
-    if (b0 == 0x7fffffff) {  // no lane holds a mass
-        if (lane == 0) out[0] = ~0ull;
-        return;
-    }
-    const uint32_t w[6] = {(uint32_t)a.a0, (uint32_t)(a.a0 >> 32), (uint32_t)a.a1, (uint32_t)(a.a1 >> 32),
-                           (uint32_t)a.a2, (uint32_t)(a.a2 >> 32)};
-    // lanes whose base is within 2 digits of the wave's lowest share an
-    // 8-digit window; the others add their own digits directly
-    const int k = a.base - b0;
-    const bool shared = a.base >= 0 && k <= 2;
-    if (a.base >= 0 && !shared) {
-        for (int j = 0; j < 6; ++j)
-            if (w[j] && a.base + j < SA_DIGITS) atomicAdd(&d[a.base + j], (unsigned long long)w[j]);
-    }
-    static_assert(SA_WAVE_WIN == 8, "window of the 6-digit lane sums at offsets 0..2");
-    uint64_t word = (uint64_t)b0;
+    uint64_t word = 0ull;
+    bool any = false;
 #pragma unroll
-    for (int j = 0; j < SA_WAVE_WIN; ++j) {
-        uint64_t v = 0;
-        if (shared) {
-#pragma unroll
-            for (int t = 0; t < 6; ++t)
-                if (t + k == j) v = w[t];
-        }
-        v = wave_sum_u64(v);
-        if (lane == (uint32_t)j + 1) word = b0 + j < SA_DIGITS ? v : 0ull;
+    for (int j = 0; j < 6; ++j) {
+        any = any || v[j] != 0ull;
+        if (lane == (uint32_t)j + 1) word = q.base + j < SA_DIGITS ? v[j] : 0ull;
     }
+    if (lane == 0) word = any ? (uint64_t)q.base : ~0ull;
     if (lane <= (uint32_t)SA_WAVE_WIN) out[lane] = word;
 }
 
@@ -719,19 +718,19 @@ struct DepParams {
     int norm_exp;             // ... times 2^norm_exp (the reference holds it in long double)
     int direct;               // 1: (m - mean) * inv_volume ; 0: fma-centred path
     int raw;                  // 1: write the deposited sum itself (adjoint deposits of signed values)
+    SaQuanta sa;                      // splitting of the cell masses (binary64)
     unsigned long long* mass_digits;  // per box SA_WORDS counters of the exact deposited mass
     unsigned long long* mass_waves;   // per tile and wave: binary64 its digit window (SA_WAVE_WORDS),
                                       // binary32 the two digit sums of its cells
-    uint64_t* scratch;        // global fallback keys
+    unsigned long long* dense_count;  // binary64 jobs of tiles beyond one workgroup's LDS: evenly cut, planned
+    uint64_t* dense_list;             // box of the tile (dep_box) << 32 | box-major tile index: even_cap evenly
+                                      // cut jobs, then plan_cap planned ones
+    uint32_t even_cap, plan_cap;
+    uint64_t* scratch;                // record lists of dense jobs (as far as it reaches)
     uint64_t scratch_cap;
     unsigned long long* scratch_cursor;
     uint32_t* err;
 };
-
-// Key layout: ext cell (13 bits) << 51 | particle index (32 bits) << 19 | slot (19 bits)
-__device__ __forceinline__ uint32_t key_cell(uint64_t k) { return (uint32_t)(k >> 51); }
-__device__ __forceinline__ uint32_t key_index(uint64_t k) { return (uint32_t)((k >> 19) & 0xffffffffull); }
-__device__ __forceinline__ uint32_t key_slot(uint64_t k) { return (uint32_t)(k & 0x7ffffull); }
 
 // |c| * S with S = s_mant * 2^s_exp (64-bit mantissa), rounded first to a
 // 64-bit significand and then to binary64: the x87 long-double product and cast
@@ -781,124 +780,6 @@ __device__ __forceinline__ T contrast_of(T sum, const DepParams& P) {
 __device__ __forceinline__ float contrast_fp32(double m, const DepParams& P) {
     if (P.raw) return (float)m;
     return (float)((m - P.mean_mass) * P.inv_volume);
-}
-
-template <typename T, bool LDS_PAYLOAD, int TE, typename KP, typename FP>
-__device__ __forceinline__ void deposit_cells(const DepParams& P, T* __restrict__ mesh, int tx,
-                                              int ty, int tz, KP keys, uint32_t M,
-                                              const uint32_t* start, FP fx, FP fy, FP fz, FP fm,
-                                              unsigned long long* sa, unsigned long long* wave_out) {
-    const Geom& g = P.g;
-    const int TT = TE > 0 ? TE : g.T;
-    const int Te = TT + 1;
-    const int cells = TT * TT * TT;
-    SaAcc win;
-    for (int c = threadIdx.x; c < cells; c += blockDim.x) {
-        const int lz = c % TT, ly = (c / TT) % TT, lx = c / (TT * TT);
-        T sum = (T)0;
-        for (int phase = 0; phase < 2; ++phase) {
-            const int ex = lx + 1 - phase;  // phase 0: base x == cell x; phase 1: base x == cell x - 1
-            uint32_t cur[4], end[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int oy = q >> 1, oz = q & 1;
-                const int cell = (ex * Te + (ly + 1 - oy)) * Te + (lz + 1 - oz);
-                cur[q] = start[cell];
-                end[q] = start[cell + 1];
-            }
-            if constexpr (LDS_PAYLOAD) {
-                // at most one record per source cell (the common case): order the
-                // up to four contributions by particle index with a sorting network
-                // and add them in that order
-                bool simple = true;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) simple = simple && end[q] - cur[q] <= 1u;
-                if (simple) {
-                    uint32_t idx[4], slot[4];
-                    int src[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const bool have = cur[q] < end[q];
-                        const uint64_t k = have ? keys[cur[q]] : 0ull;
-                        idx[q] = have ? key_index(k) : 0xffffffffu;  // empty lists sort last
-                        slot[q] = key_slot(k);
-                        src[q] = q;
-                    }
-                    auto cswap = [&](int i, int j) {
-                        if (idx[j] < idx[i]) {
-                            const uint32_t ti = idx[i], ts = slot[i];
-                            const int tq = src[i];
-                            idx[i] = idx[j]; slot[i] = slot[j]; src[i] = src[j];
-                            idx[j] = ti; slot[j] = ts; src[j] = tq;
-                        }
-                    };
-                    cswap(0, 1); cswap(2, 3); cswap(0, 2); cswap(1, 3); cswap(1, 2);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (idx[i] == 0xffffffffu) break;  // the rest are empty too
-                        const uint32_t sl = slot[i];
-                        const T ffx = fx[sl], ffy = fy[sl], ffz = fz[sl];
-                        const T mm = P.masses ? fm[sl] : (T)P.uniform_mass;
-                        const int oy = src[i] >> 1, oz = src[i] & 1;
-                        const T xw = phase == 0 ? (T)1 - ffx : ffx;
-                        const T wy = oy ? ffy : (T)1 - ffy;
-                        const T wz = oz ? ffz : (T)1 - ffz;
-                        sum += mm * xw * wy * wz;
-                    }
-                    continue;
-                }
-            }
-            // merge the four source cells by particle index
-            while (true) {
-                int best = -1;
-                uint32_t best_idx = 0xffffffffu;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (cur[q] < end[q]) {
-                        const uint32_t idx = key_index(keys[cur[q]]);
-                        if (best < 0 || idx < best_idx) { best = q; best_idx = idx; }
-                    }
-                }
-                if (best < 0) break;
-                const uint64_t k = keys[cur[best]];
-                ++cur[best];
-                T ffx, ffy, ffz, mm;
-                if constexpr (LDS_PAYLOAD) {
-                    const uint32_t s = key_slot(k);
-                    ffx = fx[s]; ffy = fy[s]; ffz = fz[s];
-                    mm = P.masses ? fm[s] : (T)P.uniform_mass;
-                } else {
-                    const uint32_t pidx = key_index(k);
-                    int b; double f;
-                    cic_axis(P.x[pidx] - P.pos_shift, g, b, f); ffx = (T)f;
-                    cic_axis(P.y[pidx] - P.pos_shift, g, b, f); ffy = (T)f;
-                    cic_axis(P.z[pidx] - P.pos_shift, g, b, f); ffz = (T)f;
-                    mm = P.masses ? (T)P.masses[pidx] : (T)P.uniform_mass;
-                }
-                const int oy = best >> 1, oz = best & 1;
-                const T xw = phase == 0 ? (T)1 - ffx : ffx;
-                const T wy = oy ? ffy : (T)1 - ffy;
-                const T wz = oz ? ffz : (T)1 - ffz;
-                sum += mm * xw * wy * wz;
-            }
-        }
-        if (!P.raw) sa_acc_add(win, sa, (double)sum);
-        const uint64_t gx = (uint64_t)(tx * g.T + lx), gy = (uint64_t)(ty * g.T + ly),
-                       gz = (uint64_t)(tz * g.T + lz);
-        mesh[(gx * g.N + gy) * g.N + gz] = contrast_of(sum, P);
-    }
-    sa_acc_flush(win, sa, wave_out);
-}
-
-// Build start[0..Te^3] (prefix positions per ext cell) from sorted keys.
-template <typename KP>
-__device__ __forceinline__ void build_cell_starts(KP keys, uint32_t M, uint32_t* start, int ncell) {
-    for (uint32_t i = threadIdx.x; i <= M; i += blockDim.x) {
-        const int c = i < M ? (int)key_cell(keys[i]) : ncell;
-        const int prev = i == 0 ? -1 : (int)key_cell(keys[i - 1]);
-        for (int q = prev + 1; q <= c; ++q) start[q] = i;
-    }
-    __syncthreads();
 }
 
 // Source ranges of a destination tile: range 0 is the own tile (all eight
@@ -968,143 +849,826 @@ __device__ __forceinline__ void wg_exclusive_scan_lds(uint32_t* a, int count, ui
     __syncthreads();
 }
 
-template <typename T, int TE = 0>
-__global__ void __launch_bounds__(DEP_THREADS) k_deposit(DepParams P, T* __restrict__ mesh) {
-    using Cfg = DepCfg<T>;
-    constexpr int CAP = Cfg::CAP;
-    constexpr int PER = CAP / DEP_THREADS;  // records per thread on the LDS path
-    static_assert(CAP % DEP_THREADS == 0, "LDS capacity must be a multiple of the workgroup size");
-    __shared__ uint64_t sh_keys[CAP];
-    __shared__ T sh_fx[CAP], sh_fy[CAP], sh_fz[CAP], sh_m[CAP];
-    __shared__ uint32_t sh_start[DEP_EXT + 1];
+// ---------------------------------------------------------------------------
+// Binary64 deposit in the reference's summation order.
+//
+// One workgroup per destination tile.  The tile's records (own bucket and the
+// boundary classes of the seven lower neighbours) go to LDS, then a counting
+// sort by DESTINATION cell gives every cell the list of its contributions
+// (record slot, corner): eight LDS counter atomics and eight 2-byte stores per
+// record.  A cell's list is put into the reference's order (base x == cell x
+// first, then base x == cell x - 1, each by particle index) and summed:
+//   - short lists by one thread (a sorting network in registers, for two
+//     neighbouring cells at once while they hold at most 8; at 1/8 to 1
+//     particle per cell a list holds 1 to 8 entries);
+//   - longer lists by one wave: with the records' ranks by particle index, a
+//     list is sorted through a bitmap of its (offset, rank) pairs and a prefix of
+//     its word counts, in time linear in its length; then the terms are formed
+//     64 at a time and added in order with lane reads, so a dense cell costs
+//     one addition latency per entry.
+// A tile with more than DEP_CAP records, or with a list for a wave, becomes 1 to
+// 64 jobs (boxes of the tile, one workgroup each) of a second launch; a job that still exceeds the
+// LDS lists its records in the scratch (when it has room) and halves its box
+// along the longest edge until the records fit.  A single cell with more than
+// DEP_CAP sources sorts its particle indices by themselves, in index ranges
+// that fit the LDS.
+//
+// Bound by LDS latency (the chain counter -> scan -> entry -> record) and by
+// the 150 or so instructions per cell; DEP_CAP = 736 records (the 1/8
+// particles per cell of a mesh twice the lattice give about 614) keep the
+// workgroup's LDS at 53 KB, three per CU.  Measured against one thread per cell
+// merging four index-sorted source lists (and a whole-tile sort in global
+// memory above 1024 records): 16.8M lattice particles on 512^3 1.33 -> 0.85 ms,
+// 3M clustered particles with masses on 192^3 16.8 -> 2.2 ms, 8192 on 32^3
+// 162 -> 36 us.
+// ---------------------------------------------------------------------------
+constexpr int DEP_CAP = 736;
+constexpr int DEP_PER = (DEP_CAP + DEP_THREADS - 1) / DEP_THREADS;
+constexpr int DEP_SERIAL = 16;  // entries one thread sorts (its network's size) in the second launch ...
+constexpr int DEP_COMMON = 8;   // ... and in the first, whose 80 registers hold no larger network
+constexpr int DEP_JOB_RECORDS = 256;  // a tile of M records makes at most M / DEP_JOB_RECORDS jobs
+constexpr int DEP_MAX_CELLS = DEP_MAX_T * DEP_MAX_T * DEP_MAX_T;
+constexpr int DEP_HEAVY = 8 * DEP_CAP / (DEP_SERIAL + 1) + 1;  // most lists longer than DEP_SERIAL
+constexpr int DEP_STACK = 16;                                   // boxes waiting (at most one per halving, 12)
+constexpr int DEP_BITS = 2 * ((DEP_CAP + 31) / 32);  // words of a list's bitmap: both x offsets
+static_assert(8 * DEP_CAP <= 65535 && DEP_CAP <= 8192, "16-bit list entries");
+static_assert(DEP_BITS <= 64 && DEP_CAP % 16 == 0, "one lane per bitmap word; padded index scans");
+
+// LDS of the workgroup as one block (also the key array of a hot cell).
+struct DepLds {
+    double fx[DEP_CAP], fy[DEP_CAP], fz[DEP_CAP];
+    uint32_t start[DEP_MAX_CELLS + 1];
+    alignas(16) uint32_t idx[DEP_CAP];  // particle index
+    uint16_t ent[8 * DEP_CAP]; // slot * 8 + corner (ox, oy, oz bits 2, 1, 0)
+    uint16_t cell[DEP_CAP];    // base cell in the tile, each axis + 1 in 5 bits; then ranks by particle index
+};
+constexpr uint32_t DEP_HOT_LDS = sizeof(DepLds) / sizeof(uint64_t);
+
+// Halvings (x, y, z in turn) of a tile of M > DEP_CAP records: uniform boxes
+// then hold 340 to 750 records.
+__device__ __forceinline__ int dep_split(uint32_t M) {
+    return M <= 1400u ? 1 : M <= 2400u ? 2 : M <= 4096u ? 3 : M <= 8192u ? 4 : M <= 16384u ? 5 : 6;
+}
+
+// Box j of the 2^levels boxes of a tile of edge T: x0, y0, z0 and the edges
+// minus one, four bits each.
+__device__ __forceinline__ uint32_t dep_box(int T, int levels, uint32_t j) {
+    uint32_t code = 0;
+    for (int a = 0; a < 3; ++a) {
+        const int n = (levels + 2 - a) / 3;  // halvings of this axis
+        int lo = 0, e = T;
+        for (int l = 0; l < n; ++l) {
+            const int h = (e + 1) / 2;
+            if (j & 1u) {
+                lo += h;
+                e -= h;
+            } else {
+                e = h;
+            }
+            j >>= 1;
+        }
+        code |= ((uint32_t)lo << (4 * a)) | ((uint32_t)(e - 1) << (12 + 4 * a));
+    }
+    return code;
+}
+
+// Order of a list entry: the x offset (reference's phase), then the particle index.
+__device__ __forceinline__ uint64_t dep_entry_key(uint16_t e, const uint32_t* idx) {
+    return ((uint64_t)(e & 4u) << 30) | idx[e >> 3];
+}
+
+// Minimum and maximum of ordinary binary64 numbers as the bare instructions
+// (fmin and fmax quiet their operands first).
+__device__ __forceinline__ double min_f64(double x, double y) {
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+#else
+    return x < y ? x : y;
+#endif
+}
+__device__ __forceinline__ double max_f64(double x, double y) {
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+#else
+    return x < y ? y : x;
+#endif
+}
+
+// In-order sum of up to 64 terms held one per lane, added to sum: sum is
+// uniform, each step reads one lane's term.  Whole waves run unrolled, so the
+// lane reads go ahead of the additions and a term costs one addition latency.
+__device__ __forceinline__ double wave_ordered_add(double sum, double term, int count) {
+    const uint64_t b = (uint64_t)__double_as_longlong(term);
+    const int lo = (int)(uint32_t)b, hi = (int)(uint32_t)(b >> 32);
+    auto at = [&](int j) {
+        const uint64_t t = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, j) << 32) |
+                           (uint32_t)__builtin_amdgcn_readlane(lo, j);
+        return __longlong_as_double((long long)t);
+    };
+    int j = 0;
+    for (; j + 8 <= count; j += 8) {
+        double t[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t[k] = at(j + k);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += t[k];
+    }
+    for (; j < count; ++j) sum += at(j);
+    return sum;
+}
+
+// Jobs of a tile of M > DEP_CAP records: a histogram of the records' base cells
+// and its 3-D prefix sums give every box's record count in eight lookups; boxes
+// are halved level by level until they hold DEP_CAP records or one cell, so a
+// clump's core becomes many jobs and the rest of its tile few.  False (no job
+// made) when a level or the job count outgrows its LDS array, or the planned
+// jobs outgrow their part of the list: the caller then cuts the tile evenly.
+// lds: DEP_PLAN_LDS words; counter: one LDS word.  The whole workgroup calls it.
+constexpr int DEP_PLAN_EXT = (DEP_MAX_T + 1) * (DEP_MAX_T + 1) * (DEP_MAX_T + 1);
+constexpr uint32_t DEP_FRONTIER = 1024, DEP_LEAVES = 2048;
+constexpr int DEP_PLAN_LDS = DEP_PLAN_EXT + 2 * (int)DEP_FRONTIER + (int)DEP_LEAVES + 4;
+static_assert(DEP_PLAN_LDS * sizeof(uint32_t) <= sizeof(DepLds), "the plan fits the deposit's LDS");
+
+template <typename BaseCell, typename SlotOf>
+__device__ __forceinline__ bool dep_plan_jobs(const DepParams& P, int T, uint32_t M, uint32_t gtile,
+                                              BaseCell&& base_cell, SlotOf&& slot_of, uint32_t* lds,
+                                              uint32_t* reserved) {
+    const int tid = (int)threadIdx.x, E = T + 1;
+    uint32_t* hist = lds;
+    uint32_t* front = lds + DEP_PLAN_EXT;
+    uint32_t* next = front + DEP_FRONTIER;
+    uint32_t* leaves = next + DEP_FRONTIER;
+    uint32_t* counts = leaves + DEP_LEAVES;  // frontier, next frontier, leaves
+    for (int i = tid; i < E * E * E; i += DEP_THREADS) hist[i] = 0u;
+    if (tid == 0) {
+        front[0] = dep_box(T, 0, 0u);
+        counts[0] = 1u;
+        counts[1] = 0u;
+        counts[2] = 0u;
+    }
+    __syncthreads();
+    for (uint32_t v = (uint32_t)tid; v < M; v += DEP_THREADS) {
+        int d;
+        const uint32_t slot = slot_of(v, d);
+        const uint32_t c = base_cell(P.rec64[slot], d);
+        const int x = (int)(c >> 10), y = (int)((c >> 5) & 31u), z = (int)(c & 31u);
+        if (x < E && y < E && z < E) atomicAdd(&hist[(x * E + y) * E + z], 1u);
+    }
+    __syncthreads();
+    // inclusive sums along z, then y, then x: line l of each axis by one thread
+    for (int axis = 0; axis < 3; ++axis) {
+        const int step = axis == 0 ? 1 : (axis == 1 ? E : E * E);
+        for (int l = tid; l < E * E; l += DEP_THREADS) {
+            const int a = l / E, b = l % E;
+            int at = axis == 0 ? l * E : (axis == 1 ? a * E * E + b : l);
+            uint32_t s = 0;
+            for (int i = 0; i < E; ++i, at += step) {
+                s += hist[at];
+                hist[at] = s;
+            }
+        }
+        __syncthreads();
+    }
+    auto sum = [&](int x, int y, int z) -> uint32_t {  // records with base below (x, y, z)
+        return x > 0 && y > 0 && z > 0 ? hist[((x - 1) * E + (y - 1)) * E + (z - 1)] : 0u;
+    };
+    for (;;) {
+        const uint32_t nf = counts[0];
+        for (uint32_t i = (uint32_t)tid; i < nf; i += DEP_THREADS) {
+            const uint32_t code = front[i];
+            const int lo[3] = {(int)(code & 15u), (int)((code >> 4) & 15u), (int)((code >> 8) & 15u)};
+            const int e[3] = {(int)((code >> 12) & 15u) + 1, (int)((code >> 16) & 15u) + 1, (int)((code >> 20) & 15u) + 1};
+            // base cells lo - 1 .. lo + e - 1, stored one up: lo .. lo + e
+            const int hx = lo[0] + e[0] + 1, hy = lo[1] + e[1] + 1, hz = lo[2] + e[2] + 1;
+            const uint32_t m = sum(hx, hy, hz) - sum(lo[0], hy, hz) - sum(hx, lo[1], hz) - sum(hx, hy, lo[2]) +
+                               sum(lo[0], lo[1], hz) + sum(lo[0], hy, lo[2]) + sum(hx, lo[1], lo[2]) -
+                               sum(lo[0], lo[1], lo[2]);
+            if (m <= (uint32_t)DEP_CAP || e[0] * e[1] * e[2] == 1) {
+                const uint32_t at = atomicAdd(&counts[2], 1u);
+                if (at < DEP_LEAVES) leaves[at] = code;
+            } else {
+                const int ax = e[0] >= e[1] && e[0] >= e[2] ? 0 : (e[1] >= e[2] ? 1 : 2);
+                const int h = (e[ax] + 1) / 2;
+                const uint32_t keep = ~((15u << (4 * ax)) | (15u << (12 + 4 * ax)));
+                const uint32_t at = atomicAdd(&counts[1], 2u);
+                if (at + 1 < DEP_FRONTIER) {
+                    next[at] = (code & keep) | ((uint32_t)lo[ax] << (4 * ax)) | ((uint32_t)(h - 1) << (12 + 4 * ax));
+                    next[at + 1] = (code & keep) | ((uint32_t)(lo[ax] + h) << (4 * ax)) |
+                                   ((uint32_t)(e[ax] - h - 1) << (12 + 4 * ax));
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t nn = counts[1], nl = counts[2];
+        __syncthreads();
+        if (nn > DEP_FRONTIER || nl > DEP_LEAVES) return false;
+        if (nn == 0) break;
+        if (tid == 0) {
+            counts[0] = nn;
+            counts[1] = 0u;
+        }
+        uint32_t* t = front;
+        front = next;
+        next = t;
+        __syncthreads();
+    }
+    const uint32_t nl = counts[2];
+    if (tid == 0) *reserved = (uint32_t)atomicAdd(P.dense_count + 1, (unsigned long long)nl);
+    __syncthreads();
+    const uint32_t at = *reserved;
+    if (at + nl > P.plan_cap) {
+        // the tile's part of the list counts as used; jobs there are marked void
+        for (uint32_t i = (uint32_t)tid; i < nl && at + i < P.plan_cap; i += DEP_THREADS)
+            P.dense_list[P.even_cap + at + i] = ~0ull;
+        return false;
+    }
+    for (uint32_t i = (uint32_t)tid; i < nl; i += DEP_THREADS)
+        P.dense_list[P.even_cap + at + i] = ((uint64_t)leaves[i] << 32) | gtile;
+    return true;
+}
+
+// TE: compile-time tile edge (16) or 0; MASS: explicit (or signed adjoint) masses.
+// DENSE = false: one workgroup per tile; tiles that need more go to the job
+// list.  DENSE = true: the workgroups walk that list (the box
+// splitting and the hot cells in the common kernel would take its registers
+// from 80 to 145, three workgroups per CU to one).
+template <int TE, bool MASS, bool DENSE>
+__global__ void __launch_bounds__(DEP_THREADS) __attribute__((amdgpu_waves_per_eu(DENSE || MASS ? 4 : 6)))
+k_deposit(DepParams P, double* __restrict__ mesh0) {
+    __shared__ __align__(16) DepLds S;
+    __shared__ double sh_m[MASS ? DEP_CAP : 1];
     __shared__ uint32_t sh_rs[DEP_NRANGES], sh_rc[DEP_NRANGES + 1];
-    __shared__ uint8_t sh_rd[DEP_NRANGES];
-    __shared__ uint64_t sh_gbase;
+    __shared__ uint8_t sh_rd[DEP_NRANGES], sh_rcls[DEP_NRANGES];
     __shared__ uint32_t sh_part[DEP_THREADS / 64];
+    __shared__ uint16_t sh_heavy[DEP_HEAVY];
+    __shared__ uint32_t sh_bits[DEP_THREADS / 64][DEP_BITS];
+    __shared__ uint32_t sh_stack[DEP_STACK];  // boxes: x0, y0, z0 (4 bits each), edges - 1 (4 bits each)
+    __shared__ uint32_t sh_count, sh_nheavy;
+    __shared__ unsigned long long sh_list;
+    __shared__ unsigned long long sh_digits[6];  // DENSE: the workgroup's mass digits
 
     const Geom& g = P.g;
     const int nT = g.nT;
     const uint32_t ntiles = (uint32_t)nT * nT * nT;
-    const uint32_t gtile = xcd_block(blockIdx.x, gridDim.x);  // box-major tile index
-    if (gtile >= ntiles * g.nbox) return;
+    const int TT = TE > 0 ? TE : g.T;
+    const int tid = (int)threadIdx.x, lane = (int)lane_id(), wave = tid >> 6;
+    // DENSE: the planned jobs, then the evenly cut ones
+    const uint32_t planned = DENSE ? min((uint32_t)P.dense_count[1], P.plan_cap) : 0u;
+    const uint32_t jobs = DENSE ? planned + (uint32_t)P.dense_count[0] : gridDim.x;
+    for (uint32_t job = blockIdx.x; job < jobs; job += gridDim.x) {
+    if constexpr (DENSE) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the last tile's LDS
+        __syncthreads();
+    }
+    const uint64_t entry = DENSE ? P.dense_list[job < planned ? P.even_cap + job : job - planned]
+                                 : (uint64_t)xcd_block(job, jobs);
+    if (DENSE && entry == ~0ull) continue;
+    const uint32_t gtile = (uint32_t)entry;  // box-major tile index
     const uint32_t box = gtile / ntiles, tile = gtile % ntiles;
     const int tz = tile % nT, ty = (tile / nT) % nT, tx = tile / (nT * nT);
-    const int TT = TE > 0 ? TE : g.T;
-    const int Te = TT + 1;
-    const int ncell = Te * Te * Te;
-    mesh += (uint64_t)box * g.N * g.N * g.N;
+    double* mesh = mesh0 + (uint64_t)box * g.N * g.N * g.N;
     static_assert(DEP_THREADS / 64 == SA_WAVES_PER_TILE, "one mass window per wave");
     // exact cell-mass sum: each wave's window, plus the box's counters for the rest
     unsigned long long* box_digits = P.mass_digits + (uint64_t)box * SA_WORDS;
     unsigned long long* wave_out =
         P.mass_waves + ((uint64_t)gtile * SA_WAVES_PER_TILE + threadIdx.x / 64) * SA_WAVE_WORDS;
+    SaAcc win;
 
-    __shared__ uint8_t sh_rcls[DEP_NRANGES];
+    if (DENSE && tid == 0) sh_stack[0] = (uint32_t)(entry >> 32);
     load_source_ranges(P.offsets + (uint64_t)box * buckets_per_box(g), tx, ty, tz, nT, sh_rs, sh_rc, sh_rd,
                        sh_rcls);
     const uint32_t M = sh_rc[DEP_NRANGES];
-    const bool use_lds = M <= (uint32_t)CAP;
+    // !DENSE: leaves the tile to 2^levels equal jobs, which also add its mass
+    auto leave = [&](int levels) {
+        if (tid < 64) {
+            uint32_t at = 0;
+            if (lane == 0) at = (uint32_t)atomicAdd(P.dense_count, 1ull << levels);
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+            if (lane < (1 << levels))
+                P.dense_list[at + (uint32_t)lane] = ((uint64_t)dep_box(TT, levels, (uint32_t)lane) << 32) | gtile;
+        }
+        if (lane == 0) wave_out[0] = ~0ull;
+    };
+    // Writes the finished cell (tile coordinates) and adds its mass.
+    mesh += ((uint64_t)(tx * TT) * g.N + (uint64_t)(ty * TT)) * g.N + (uint64_t)(tz * TT);
+    auto finish = [&](int lx, int ly, int lz, double sum) {
+        if (!P.raw) sa_acc_add(win, P.sa, box_digits, sum);
+        mesh[(uint64_t)(uint32_t)(lx * g.N + ly) * (uint64_t)g.N + (uint32_t)lz] = contrast_of(sum, P);
+    };
 
-    uint64_t* gkeys = nullptr;
-    if (!use_lds) {
-        if (threadIdx.x == 0) sh_gbase = atomicAdd(P.scratch_cursor, (unsigned long long)M);
-        __syncthreads();
-        if (sh_gbase + M > P.scratch_cap) {
-            if (threadIdx.x == 0) atomicOr(P.err, ERR_SCRATCH);
-            if (lane_id() == 0) wave_out[0] = ~0ull;  // this tile's waves hold no mass
+    // Base cell of a record in the tile (-1 .. T-1 per axis, each + 1 in 5 bits);
+    // DEP_NOWHERE, outside every box, for a record that does not lie where its
+    // bucket says (ERR_COORDINATE; also a slot a failed scatter left unwritten).
+    constexpr uint32_t DEP_NOWHERE = 0x7fff;
+    auto base_cell = [&](const DepRecord64& rec, int d) -> uint32_t {
+        const uint32_t c = rec.cell;
+        const int cz = (int)(c % (uint32_t)TT), cy = (int)((c / (uint32_t)TT) % (uint32_t)TT),
+                  cx = (int)(c / (uint32_t)(TT * TT));
+        if (cx >= TT || ((d & 4) && cx != TT - 1) || ((d & 2) && cy != TT - 1) || ((d & 1) && cz != TT - 1) ||
+            rec.index >= P.n) {
+            atomicOr(P.err, ERR_COORDINATE);
+            return DEP_NOWHERE;
+        }
+        return (uint32_t)((((d & 4) ? 0 : cx + 1) << 10) | (((d & 2) ? 0 : cy + 1) << 5) | ((d & 1) ? 0 : cz + 1));
+    };
+    auto slot_of = [&](uint32_t v, int& d) -> uint32_t {  // record v of the tile: its slot and neighbour offset
+        int lo = 0, hi = DEP_NRANGES - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (sh_rc[mid] <= v) lo = mid;
+            else hi = mid - 1;
+        }
+        d = sh_rd[lo];
+        return sh_rs[lo] + (v - sh_rc[lo]);
+    };
+
+    if constexpr (!DENSE) {
+        if (M > (uint32_t)DEP_CAP) {
+            if (!dep_plan_jobs(P, TT, M, gtile, base_cell, slot_of, reinterpret_cast<uint32_t*>(&S), &sh_nheavy)) leave(dep_split(M));
+            if (lane == 0) wave_out[0] = ~0ull;
             return;
         }
-        gkeys = P.scratch + sh_gbase;
-    } else {
-        for (int i = threadIdx.x; i <= ncell; i += blockDim.x) sh_start[i] = 0u;
-        __syncthreads();
     }
 
-    // Load the records (read contiguously per source range): ext cell relative
-    // to this tile, particle index, binary64 fractions.  A neighbour record
-    // sits on the last cell of its tile along each shifted axis.  On the LDS
-    // path each thread keeps its keys in registers and counts them per cell.
-    uint64_t mykey[PER];
-    uint32_t myrank[PER];
-    auto load = [&](uint32_t v) -> uint64_t {
-        int r = 0;
-        while (sh_rc[r + 1] <= v) ++r;
-        const uint32_t slot = sh_rs[r] + (v - sh_rc[r]);
-        const DepRecord64 rc = P.rec64[slot];
-        const int d = sh_rd[r];
-        const int TL = g.T;
-        const uint32_t pidx = rc.index < P.n ? rc.index : 0u;  // guards a slot a failed scatter left unwritten
-        const int cz = (int)(rc.cell % (uint32_t)TL), cy = (int)((rc.cell / (uint32_t)TL) % (uint32_t)TL),
-                  cx = (int)(rc.cell / (uint32_t)(TL * TL));
-        int ex = (d & 4) ? 0 : cx + 1;
-        int ey = (d & 2) ? 0 : cy + 1;
-        int ez = (d & 1) ? 0 : cz + 1;
-        if (rc.index >= P.n || rc.cell >= (uint32_t)(TL * TL * TL) || ((d & 4) && cx != TL - 1) ||
-            ((d & 2) && cy != TL - 1) || ((d & 1) && cz != TL - 1)) {
-            atomicOr(P.err, ERR_COORDINATE);
-            ex = ex > TL ? TL : ex;
-            ey = ey > TL ? TL : ey;
-            ez = ez > TL ? TL : ez;
-        }
-        const uint32_t cell = (uint32_t)((ex * Te + ey) * Te + ez);
-        if (use_lds) {
-            sh_fx[v] = (T)rc.fx; sh_fy[v] = (T)rc.fy; sh_fz[v] = (T)rc.fz;
-            if (P.masses) sh_m[v] = (T)P.rec_mass64[slot];
-        }
-        return ((uint64_t)cell << 51) | ((uint64_t)pidx << 19) | (use_lds ? v : 0u);
-    };
-    if (use_lds) {
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const uint32_t v = threadIdx.x + (uint32_t)j * DEP_THREADS;
-            mykey[j] = 0;
-            myrank[j] = 0;
-            if (v < M) {
-                mykey[j] = load(v);
-                myrank[j] = atomicAdd(&sh_start[key_cell(mykey[j])], 1u);
-            }
-        }
-    } else {
-        for (uint32_t v = threadIdx.x; v < M; v += blockDim.x) gkeys[v] = load(v);
-    }
-    __threadfence_block();
-    __syncthreads();
-
-    if (use_lds) {
-        // counting sort by cell, then each cell's few records by particle index
-        wg_exclusive_scan_lds(sh_start, ncell + 1, sh_part);
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const uint32_t v = threadIdx.x + (uint32_t)j * DEP_THREADS;
-            if (v < M) sh_keys[sh_start[key_cell(mykey[j])] + myrank[j]] = mykey[j];
-        }
+    uint64_t* list = nullptr;  // this job's records: slot << 32 | base cell
+    uint32_t listed = 0;
+    int depth = 1;
+    while (depth > 0) {
+        // The box stack written at the end of the last trip, and that box's LDS
+        // reads.  The wait is explicit: at this loop header the compiler left
+        // the barrier's own lgkmcnt wait out, and a wave that read the stack
+        // ahead of its write went through other barriers than the rest.
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         __syncthreads();
-        for (int c = threadIdx.x; c < ncell; c += blockDim.x) {
-            const uint32_t b = sh_start[c], e = sh_start[c + 1];
-            for (uint32_t i = b + 1; i < e; ++i) {
-                const uint64_t k = sh_keys[i];
-                uint32_t j = i;
-                while (j > b && sh_keys[j - 1] > k) {
-                    sh_keys[j] = sh_keys[j - 1];
-                    --j;
+        --depth;
+        const uint32_t code = DENSE ? sh_stack[depth] : dep_box(TT, 0, 0u);
+        const int x0 = (int)(code & 15u), y0 = (int)((code >> 4) & 15u), z0 = (int)((code >> 8) & 15u);
+        const int ex = (int)((code >> 12) & 15u) + 1, ey = (int)((code >> 16) & 15u) + 1,
+                  ez = (int)((code >> 20) & 15u) + 1;
+        const int cells = ex * ey * ez;
+
+        auto in_box = [&](uint32_t bc) {
+            const uint32_t bx = bc >> 10, by = (bc >> 5) & 31u, bz = bc & 31u;
+            return bx - (uint32_t)x0 <= (uint32_t)ex && by - (uint32_t)y0 <= (uint32_t)ey &&
+                   bz - (uint32_t)z0 <= (uint32_t)ez;
+        };
+        // The records whose corners touch the box: use(s, base cell, slot) for
+        // those that want(base cell, slot) takes, s from a counter in LDS (one
+        // atomic per wave and four records per thread, their loads in flight
+        // together).
+        auto each_match = [&](auto&& want, auto&& use) {
+            const uint32_t count = list ? listed : M;
+            for (uint32_t v0 = 0; v0 < count; v0 += 4 * DEP_THREADS) {
+                uint32_t bc[4], slot[4], at[4];
+                bool live[4];
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const uint32_t v = v0 + (uint32_t)(h * DEP_THREADS + tid);
+                    bc[h] = DEP_NOWHERE;
+                    slot[h] = 0u;
+                    if (v < count) {
+                        if (list) {
+                            const uint64_t e = list[v];
+                            bc[h] = (uint32_t)e;
+                            slot[h] = (uint32_t)(e >> 32);
+                        } else {
+                            int d;
+                            slot[h] = slot_of(v, d);
+                            bc[h] = base_cell(P.rec64[slot[h]], d);
+                        }
+                    }
                 }
-                sh_keys[j] = k;
+                uint32_t total = 0;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    live[h] = in_box(bc[h]) && want(bc[h], slot[h]);
+                    const uint64_t mask = __ballot(live[h]);
+                    at[h] = total + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+                    total += (uint32_t)__popcll(mask);
+                }
+                uint32_t base = 0;
+                if (total) {  // uniform over the wave
+                    if (lane == 0) base = atomicAdd(&sh_count, total);
+                    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                }
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    if (live[h]) use(base + at[h], bc[h], slot[h]);
+            }
+        };
+        auto any = [](uint32_t, uint32_t) { return true; };
+        auto keep = [&](uint32_t s, uint32_t slot, const DepRecord64& rc, uint32_t bc) {
+            S.fx[s] = rc.fx;
+            S.fy[s] = rc.fy;
+            S.fz[s] = rc.fz;
+            S.idx[s] = rc.index;
+            S.cell[s] = (uint16_t)bc;
+            if constexpr (MASS) sh_m[s] = P.rec_mass64[slot];
+        };
+
+        uint32_t m = M;
+        {
+            if (tid == 0) {
+                sh_count = 0;
+                sh_nheavy = 0;
+            }
+            for (int i = tid; i <= cells; i += DEP_THREADS) S.start[i] = 0u;
+            if constexpr (!DENSE) {
+                // both records of a thread in flight together
+                DepRecord64 rec[DEP_PER];
+                uint32_t slot[DEP_PER];
+                int d[DEP_PER];
+#pragma unroll
+                for (int j = 0; j < DEP_PER; ++j) {
+                    const uint32_t v = (uint32_t)(tid + j * DEP_THREADS);
+                    if (v < M) {
+                        slot[j] = slot_of(v, d[j]);
+                        rec[j] = P.rec64[slot[j]];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < DEP_PER; ++j) {
+                    const uint32_t v = (uint32_t)(tid + j * DEP_THREADS);
+                    if (v < M) keep(v, slot[j], rec[j], base_cell(rec[j], d[j]));
+                }
+                __syncthreads();
+            } else {
+                __syncthreads();
+                each_match(any, [&](uint32_t s, uint32_t bc, uint32_t slot) {
+                    if (s < (uint32_t)DEP_CAP) keep(s, slot, P.rec64[slot], bc);
+                });
+                __syncthreads();
+                m = sh_count;
+            }
+        }
+        if (DENSE && m > (uint32_t)DEP_CAP) {
+            if (!list) {
+                // first box of the job: its records listed for the boxes inside it
+                __syncthreads();
+                if (tid == 0) {
+                    sh_list = atomicAdd(P.scratch_cursor, (unsigned long long)m);
+                    sh_count = 0;
+                }
+                __syncthreads();
+                if (sh_list + m <= P.scratch_cap) {
+                    uint64_t* out = P.scratch + sh_list;
+                    each_match(any, [&](uint32_t s, uint32_t bc, uint32_t slot) {
+                        if (s < m) out[s] = ((uint64_t)slot << 32) | bc;
+                    });
+                    __threadfence_block();
+                    list = out;
+                    listed = m;
+                }
+            }
+            if (cells > 1) {
+                // halve the longest edge (x first: its halves are contiguous in the mesh)
+                __syncthreads();
+                if (tid == 0) {
+                    const int hx = ex >= ey && ex >= ez ? (ex + 1) / 2 : 0, hy = !hx && ey >= ez ? (ey + 1) / 2 : 0;
+                    const int hz = !hx && !hy ? (ez + 1) / 2 : 0;
+                    auto enc = [](int a, int b, int c, int u, int v, int w) {
+                        return (uint32_t)(a | (b << 4) | (c << 8) | ((u - 1) << 12) | ((v - 1) << 16) | ((w - 1) << 20));
+                    };
+                    sh_stack[depth] = enc(x0, y0, z0, hx ? hx : ex, hy ? hy : ey, hz ? hz : ez);
+                    sh_stack[depth + 1] = enc(x0 + hx, y0 + hy, z0 + hz, hx ? ex - hx : ex, hy ? ey - hy : ey,
+                                              hz ? ez - hz : ez);
+                }
+                __syncthreads();
+                depth += 2;
+                continue;
+            }
+            // One cell with more than DEP_CAP sources: keys (phase, particle index,
+            // y and z offset) of the sources whose (phase, index) lies in
+            // [lo, hi), a range whose keys fit the LDS, sorted; the terms in
+            // place of the keys, then added in order by the first wave.  Range
+            // by range, the running sum carried on.
+            uint64_t* keys = reinterpret_cast<uint64_t*>(&S);
+            const uint64_t end = 2 * P.n;  // keys are phase * n + index
+            uint64_t lo = 0, width = m <= DEP_HOT_LDS ? end : (P.n / m + 1) * (DEP_HOT_LDS / 2);
+            double sum = 0.0;
+            while (lo < end) {
+                const uint64_t hi = lo + width;
+                __syncthreads();
+                if (tid == 0) sh_count = 0;
+                __syncthreads();
+                // offsets 1 where the base is one below the cell
+                auto key = [&](uint32_t bc, uint32_t slot) -> uint64_t {
+                    return (((bc >> 10) == (uint32_t)x0 ? P.n : 0ull) + P.rec64[slot].index);
+                };
+                each_match(
+                    [&](uint32_t bc, uint32_t slot) {
+                        const uint64_t k = key(bc, slot);
+                        return k >= lo && k < hi;
+                    },
+                    [&](uint32_t s, uint32_t bc, uint32_t slot) {
+                        const uint32_t oy = ((bc >> 5) & 31u) == (uint32_t)y0, oz = (bc & 31u) == (uint32_t)z0;
+                        if (s < DEP_HOT_LDS) keys[s] = (key(bc, slot) << 2) | (uint64_t)(oy << 1) | (uint64_t)oz;
+                    });
+                __syncthreads();
+                const uint32_t c = sh_count;
+                if (c > DEP_HOT_LDS) {
+                    width >>= 1;
+                    continue;
+                }
+                wg_sort_u64(keys, c);
+                __syncthreads();
+                for (uint32_t i = (uint32_t)tid; i < c; i += DEP_THREADS) {
+                    const uint64_t k = keys[i];
+                    const bool upper = (k >> 2) >= P.n;
+                    const uint32_t p = (uint32_t)((k >> 2) - (upper ? P.n : 0ull));
+                    int b;
+                    double fx, fy, fz;
+                    cic_axis(P.x[p] - P.pos_shift, g, b, fx);
+                    cic_axis(P.y[p] - P.pos_shift, g, b, fy);
+                    cic_axis(P.z[p] - P.pos_shift, g, b, fz);
+                    const double mm = MASS ? P.masses[p] : P.uniform_mass;
+                    const double term = mm * (upper ? fx : 1.0 - fx) * (k & 2u ? fy : 1.0 - fy) *
+                                        (k & 1u ? fz : 1.0 - fz);
+                    keys[i] = (uint64_t)__double_as_longlong(term);
+                }
+                __syncthreads();
+                if (wave == 0) {
+                    for (uint32_t c0 = 0; c0 < c; c0 += 64) {
+                        const double term =
+                            c0 + (uint32_t)lane < c ? __longlong_as_double((long long)keys[c0 + (uint32_t)lane]) : 0.0;
+                        sum = wave_ordered_add(sum, term, (int)(c - c0 < 64u ? c - c0 : 64u));
+                    }
+                }
+                lo = hi;
+                if (c < DEP_HOT_LDS / 4) width <<= 1;
+            }
+            if (tid == 0) finish(x0, y0, z0, sum);
+            continue;
+        }
+
+        // counting sort of the contributions by destination cell: corner o of a
+        // record is cell c0 + ox sx + oy ez + oz of the box where it lies in it
+        const int sx = ey * ez;
+        uint32_t rank[DEP_PER][4];  // two 16-bit ranks per word (a list holds at most DEP_CAP)
+        int cell0[DEP_PER];
+        uint32_t corners[DEP_PER];  // bit o: corner o lies in the box
+#pragma unroll
+        for (int j = 0; j < DEP_PER; ++j) {
+            const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
+            corners[j] = 0u;
+            cell0[j] = 0;
+            if (s < m) {
+                const uint32_t cc = S.cell[s];
+                const int cx = (int)(cc >> 10) - 1 - x0, cy = (int)((cc >> 5) & 31u) - 1 - y0,
+                          cz = (int)(cc & 31u) - 1 - z0;
+                cell0[j] = (cx * ey + cy) * ez + cz;
+                const uint32_t mx = (cx >= 0 && cx < ex ? 0x0fu : 0u) | (cx + 1 < ex ? 0xf0u : 0u),
+                               my = (cy >= 0 && cy < ey ? 0x33u : 0u) | (cy + 1 < ey ? 0xccu : 0u),
+                               mz = (cz >= 0 && cz < ez ? 0x55u : 0u) | (cz + 1 < ez ? 0xaau : 0u);
+                corners[j] = mx & my & mz;
+#pragma unroll
+                for (int o = 0; o < 8; ++o) {
+                    const int c = cell0[j] + (o >> 2) * sx + ((o >> 1) & 1) * ez + (o & 1);
+                    const uint32_t r = (corners[j] >> o) & 1u ? atomicAdd(&S.start[c], 1u) : 0u;
+                    if (!DENSE && r >= (uint32_t)DEP_COMMON) sh_nheavy = 1u;
+                    rank[j][o >> 1] = o & 1 ? rank[j][o >> 1] | (r << 16) : r;
+                }
             }
         }
         __syncthreads();
-        deposit_cells<T, true, TE>(P, mesh, tx, ty, tz, sh_keys, M, sh_start, sh_fx, sh_fy, sh_fz,
-                               sh_m, box_digits, wave_out);
-    } else {
-        wg_sort_u64(gkeys, M);
-        build_cell_starts(gkeys, M, sh_start, ncell);
-        deposit_cells<T, false, TE>(P, mesh, tx, ty, tz, gkeys, M, sh_start, sh_fx, sh_fy, sh_fz,
-                                sh_m, box_digits, wave_out);
+        if constexpr (!DENSE) {
+            if (sh_nheavy) {  // lists for whole waves
+                leave(0);
+                return;
+            }
+        }
+        wg_exclusive_scan_lds(S.start, cells + 1, sh_part);
+#pragma unroll
+        for (int j = 0; j < DEP_PER; ++j) {
+            const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
+#pragma unroll
+            for (int o = 0; o < 8; ++o) {
+                const int c = cell0[j] + (o >> 2) * sx + ((o >> 1) & 1) * ez + (o & 1);
+                if ((corners[j] >> o) & 1u)
+                    S.ent[S.start[c] + ((rank[j][o >> 1] >> (16 * (o & 1))) & 0xffffu)] =
+                        (uint16_t)(s * 8u + (uint32_t)o);
+            }
+        }
+        __syncthreads();
+        auto term_of = [&](uint16_t e) -> double {
+            const uint32_t s = min((uint32_t)e >> 3, (uint32_t)DEP_CAP - 1u);  // empty network entries: any record
+            const double fx = S.fx[s], fy = S.fy[s], fz = S.fz[s];
+            double mm = P.uniform_mass;
+            if constexpr (MASS) mm = sh_m[s];
+            // weight f or 1 - f as |c - f| with c = 0 or 1 (exact alike)
+            auto one_unless = [](uint32_t bit) {
+                return __longlong_as_double((long long)((uint64_t)((bit - 1u) & 0x3ff00000u) << 32));
+            };
+            return mm * fabs(one_unless((e >> 2) & 1u) - fx) * fabs(one_unless((e >> 1) & 1u) - fy) *
+                   fabs(one_unless(e & 1u) - fz);
+        };
+        // box cell -> tile coordinates (edges are powers of two when TE is)
+        const int lgz = __ffs(ez) - 1, lgy = __ffs(ey) - 1;
+        auto finish_cell = [&](int c, double sum) {
+            if constexpr (TE > 0 && (TE & (TE - 1)) == 0)
+                finish(x0 + (c >> (lgz + lgy)), y0 + ((c >> lgz) & (ey - 1)), z0 + (c & (ez - 1)), sum);
+            else
+                finish(x0 + c / (ey * ez), y0 + (c / ez) % ey, z0 + c % ez, sum);
+        };
+        // Two neighbouring cells per thread: their lists are adjacent, so one
+        // network orders both (the cell as the key's top bit) and the chain of
+        // dependent LDS reads is paid once for the pair.
+#pragma unroll 1
+        for (int p0 = 64 * wave; 2 * p0 < cells; p0 += DEP_THREADS) {  // whole waves: the ballots below
+            const int c = 2 * (p0 + lane);
+            uint32_t b0 = 0, b1 = 0, b2 = 0;
+            if (c < cells) {
+                b0 = S.start[c];
+                b1 = S.start[c + 1];
+                b2 = c + 1 < cells ? S.start[c + 2] : b1;
+            }
+            const bool heavy0 = DENSE && b1 - b0 > (uint32_t)DEP_SERIAL, heavy1 = DENSE && b2 - b1 > (uint32_t)DEP_SERIAL;
+            if (heavy0) sh_heavy[atomicAdd(&sh_nheavy, 1u)] = (uint16_t)c;
+            if (heavy1) sh_heavy[atomicAdd(&sh_nheavy, 1u)] = (uint16_t)(c + 1);
+            const uint32_t first = heavy0 ? b1 : b0, n = (heavy1 ? b1 : b2) - first;
+            double sum0 = 0.0, sum1 = 0.0;
+            // entries [at0, at0 + n) of a list, at most N in every lane, the first
+            // n0 of the pair's first cell: network of N keys (cell of the pair,
+            // phase, index, entry; empty ones last), held as the bits of positive
+            // normal binary64 numbers, which order alike and compare and exchange
+            // in two instructions
+            auto network = [&](auto size, uint32_t at0, uint32_t n) {
+                constexpr int N = decltype(size)::value;
+                const uint32_t n0 = at0 < b1 ? min(n, b1 - at0) : 0u;
+                double k[N];
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    // read whether or not the entry exists (within the arrays): the
+                    // reads of all entries go out together
+                    const uint32_t at = at0 + (uint32_t)i;
+                    const uint32_t v = S.ent[min(at, 8u * DEP_CAP - 1u)];
+                    const uint32_t index = S.idx[min(v >> 3, (uint32_t)DEP_CAP - 1u)];
+                    const uint32_t top = 0x00100000u | (at >= b1 ? 1u << 18 : 0u) | ((v & 4u) << 14) | (index >> 16);
+                    const uint64_t key = ((uint64_t)((uint32_t)i < n ? top : 0x7fe00000u) << 32) | (index << 16) | v;
+                    k[i] = __longlong_as_double((long long)key);
+                }
+                // Batcher's odd-even merge sort
+#pragma unroll
+                for (int p = 1; p < N; p *= 2)  // any N: comparators past it fall away
+#pragma unroll
+                    for (int q = p; q >= 1; q /= 2)
+#pragma unroll
+                        for (int j = q % p; j + q < N; j += 2 * q)
+#pragma unroll
+                            for (int i = 0; i < q; ++i)
+                                if (i + j + q < N && (i + j) / (2 * p) == (i + j + q) / (2 * p)) {
+                                    const double x = k[i + j], y = k[i + j + q];
+                                    k[i + j] = min_f64(x, y);
+                                    k[i + j + q] = max_f64(x, y);
+                                }
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    // + 0.0 leaves a sum as it is (no sum is -0.0)
+                    const double t = term_of((uint16_t)__double_as_longlong(k[i]));
+                    sum0 += (uint32_t)i < n0 ? t : 0.0;
+                    sum1 += (uint32_t)i >= n0 && (uint32_t)i < n ? t : 0.0;
+                    // two records' fractions in registers at a time
+                    if (i & 1) __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            using I2 = std::integral_constant<int, 2>;
+            using I4 = std::integral_constant<int, 4>;
+            using I6 = std::integral_constant<int, 6>;
+            using I8 = std::integral_constant<int, 8>;
+            using I16 = std::integral_constant<int, DEP_SERIAL>;
+            if (!__ballot(n > 2)) {
+                network(I2{}, first, n);
+            } else if (!__ballot(n > 4)) {
+                network(I4{}, first, n);
+            } else if (!__ballot(n > 6)) {
+                network(I6{}, first, n);
+            } else if (!__ballot(n > 8)) {
+                network(I8{}, first, n);
+            } else {
+#pragma unroll 1
+                for (int h = 0; h < 2; ++h) {  // one cell at a time
+                    const uint32_t at = h ? b1 : first, nh = h ? first + n - b1 : b1 - first;
+                    if (!DENSE || !__ballot(nh > 8)) network(I8{}, at, nh);
+                    else if constexpr (DENSE) network(I16{}, at, nh);
+                }
+            }
+            if constexpr (!DENSE) {
+                // an even edge: the pair lies in one row and c < cells throughout
+                if (!P.raw) {
+                    sa_acc_add(win, P.sa, box_digits, sum0);
+                    sa_acc_add(win, P.sa, box_digits, sum1);
+                }
+                typedef double D2 __attribute__((ext_vector_type(2), aligned(16)));
+                const D2 out = {contrast_of(sum0, P), contrast_of(sum1, P)};
+                const int lx = c / (TT * TT), ly = (c / TT) % TT, lz = c % TT;
+                if (c < cells)
+                    *reinterpret_cast<D2*>(&mesh[(uint64_t)(uint32_t)(lx * g.N + ly) * (uint64_t)g.N + (uint32_t)lz]) = out;
+            } else {
+                if (c < cells && !heavy0) finish_cell(c, sum0);
+                if (c + 1 < cells && !heavy1) finish_cell(c + 1, sum1);
+            }
+        }
+        __syncthreads();
+        const uint32_t nheavy = DENSE ? sh_nheavy : 0u;
+        if (nheavy) {
+            // Rank of every record by particle index (the base cells are done
+            // with): each thread's records against all, sixteen indices per
+            // trip in flight, padded with the largest.
+            const uint32_t m16 = (m + 15u) & ~15u;
+            if ((uint32_t)tid < m16 - m) S.idx[m + (uint32_t)tid] = 0xffffffffu;
+            __syncthreads();
+            uint32_t mine[DEP_PER], r[DEP_PER];
+#pragma unroll
+            for (int j = 0; j < DEP_PER; ++j) {
+                const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
+                mine[j] = s < m ? S.idx[s] : 0u;
+                r[j] = 0u;
+            }
+            typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+            const U4* all = reinterpret_cast<const U4*>(S.idx);
+            for (uint32_t t = 0; t < m16 / 4u; t += 4) {
+                const U4 q[4] = {all[t], all[t + 1], all[t + 2], all[t + 3]};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int j = 0; j < DEP_PER; ++j)
+                        r[j] += (q[k].x < mine[j] ? 1u : 0u) + (q[k].y < mine[j] ? 1u : 0u) +
+                                (q[k].z < mine[j] ? 1u : 0u) + (q[k].w < mine[j] ? 1u : 0u);
+            }
+#pragma unroll
+            for (int j = 0; j < DEP_PER; ++j) {
+                const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
+                if (s < m) S.cell[s] = (uint16_t)r[j];
+            }
+            __syncthreads();
+        }
+        for (uint32_t h = (uint32_t)wave; h < nheavy; h += DEP_THREADS / 64) {
+            const int c = sh_heavy[h];
+            const uint32_t b = S.start[c], n = S.start[c + 1] - b;  // at most DEP_CAP: one corner per record
+            uint32_t* bits = sh_bits[wave];
+            auto place = [&](uint16_t e) -> uint32_t {
+                return (e & 4 ? 32u * (DEP_BITS / 2) : 0u) + S.cell[e >> 3];
+            };
+            if (lane < DEP_BITS) bits[lane] = 0u;
+            __threadfence_block();
+            __builtin_amdgcn_wave_barrier();
+            uint16_t mine[(DEP_CAP + 63) / 64];
+#pragma unroll
+            for (int q = 0; q < (DEP_CAP + 63) / 64; ++q) {
+                const uint32_t i = (uint32_t)(lane + 64 * q);
+                if (i < n) {
+                    mine[q] = S.ent[b + i];
+                    const uint32_t at = place(mine[q]);
+                    atomicOr(&bits[at >> 5], 1u << (at & 31u));
+                }
+            }
+            __threadfence_block();
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t word = lane < DEP_BITS ? bits[lane] : 0u;
+            const uint32_t below = wave_incl_scan_u32((uint32_t)__popc(word)) - (uint32_t)__popc(word);
+#pragma unroll
+            for (int q = 0; q < (DEP_CAP + 63) / 64; ++q) {
+                if (64u * q >= n) break;  // uniform
+                const bool have = (uint32_t)(lane + 64 * q) < n;
+                const uint32_t at = have ? place(mine[q]) : 0u;
+                const uint32_t w = __shfl(word, (int)(at >> 5)), w0 = __shfl(below, (int)(at >> 5));
+                if (have) S.ent[b + w0 + (uint32_t)__popc(w & ((1u << (at & 31u)) - 1u))] = mine[q];
+            }
+            __threadfence_block();
+            __builtin_amdgcn_wave_barrier();
+            double sum = 0.0;
+            for (uint32_t c0 = 0; c0 < n; c0 += 64) {
+                const double term = c0 + (uint32_t)lane < n ? term_of(S.ent[b + c0 + (uint32_t)lane]) : 0.0;
+                sum = wave_ordered_add(sum, term, (int)(n - c0 < 64u ? n - c0 : 64u));
+            }
+            if (lane == 0) finish_cell(c, sum);
+        }
+        if constexpr (!DENSE) break;
     }
-
+    if constexpr (DENSE) {
+        // the workgroup's digits summed in LDS, one atomic per digit and job
+        if (tid < 6) sh_digits[tid] = 0ull;
+        __syncthreads();
+        uint64_t v[6];
+        sa_acc_digits(win, P.sa, v);
+        if (lane == 0) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j)
+                if (v[j]) atomicAdd(&sh_digits[j], (unsigned long long)v[j]);
+        }
+        __syncthreads();
+        if (tid < 6 && P.sa.base + tid < SA_DIGITS && sh_digits[tid])
+            atomicAdd(&box_digits[P.sa.base + tid], sh_digits[tid]);
+    } else {
+        sa_acc_flush(win, P.sa, wave_out);
+        return;  // one tile per workgroup
+    }
+    }
 }
-
-template __global__ void k_deposit<double, 0>(DepParams, double*);
-template __global__ void k_deposit<double, 16>(DepParams, double*);
 
 // ---------------------------------------------------------------------------
 // Binary32 deposit: fixed-point accumulation in LDS.

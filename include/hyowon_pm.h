@@ -20,8 +20,7 @@
  *  - One context owns one HIP stream and its mesh workspace; calls on a
  *    context must be serialised (as PMSolver, include/cosmo_nbody/mesh/
  *    mass_assignment.hpp:44-45).  All device memory is allocated by
- *    hy_pm_create; the force and step entry points allocate nothing (except the
- *    deposit fallback scratch growing after an HY_ERUNTIME-free retry).
+ *    hy_pm_create; the force and step entry points allocate nothing.
  */
 #ifndef HYOWON_PM_H
 #define HYOWON_PM_H
