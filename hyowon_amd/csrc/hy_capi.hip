@@ -144,6 +144,9 @@ struct hy_pm_ctx {
     uint32_t* xcounts = nullptr;   // x-plane bins (N)
     uint32_t* xoffsets = nullptr;  // N+1
     unsigned long long* mass_digits = nullptr;  // per box: exact deposited-mass digit counters
+    uint32_t* tickets = nullptr;                // per box: arrivals of the mass reduction's workgroups
+    unsigned long long* mass_in = nullptr;      // exact sum of explicit masses (k_input_mass)
+    unsigned long long* dense_count = nullptr;  // binary64 deposit: evenly cut and planned jobs, list cursor
     uint64_t* dense_list = nullptr;             // binary64 deposit jobs of the tiles above its LDS capacity
     uint64_t even_cap = 0, plan_cap = 0;        // evenly cut and planned jobs the list holds
     unsigned long long* mass_waves = nullptr;   // per deposit wave: its exact mass (binary64: digit window,
@@ -189,6 +192,7 @@ struct hy_pm_ctx {
         uint32_t err;
         uint32_t total;
         double mass;
+        double mass_in[2];  // sum and maximum of explicit masses
     };
     Status* hstatus = nullptr;
     Status* dstatus = nullptr;
@@ -264,7 +268,6 @@ const char* const kMsgPositions = "CIC positions must be finite";
 void raise_errors(uint32_t e) {
     using namespace hy;
     if (e & ERR_POSITION_NONFINITE) fail(HY_EINVAL, kMsgPositions);
-    if (e & ERR_MASS_INVALID) fail(HY_EINVAL, "CIC masses must be finite and non-negative");
     if (e & ERR_STALE_KEYS) fail(HY_ELOGIC, "reused bucket keys do not match the input positions");
     if (e & ERR_COORDINATE) fail(HY_ELOGIC, "CIC bounded coordinate escaped the mesh domain");
     if (e & ERR_SCRATCH) fail(HY_ERUNTIME, "bucket sort scratch exhausted");
@@ -282,8 +285,9 @@ void raise_errors(uint32_t e) {
     if (e & ERR_MASS_CONSERVATION) fail(HY_ERUNTIME, "CIC deposited mass violates the forward-error bound");
 }
 
-// Input mass identity (src/gravity/pm_solver.cpp:120-130,665-684).
-double input_mass(hy_pm_ctx* c, uint64_t n, const double* masses, double uniform, bool host_ptrs) {
+// Input mass identity (src/gravity/pm_solver.cpp:120-130,665-684); masses in
+// device memory.
+double input_mass(hy_pm_ctx* c, uint64_t n, const double* masses, double uniform) {
     if (n == 0) fail(HY_ERUNTIME, "PMSolver exact input mass identity must be finite and positive");
     double M;
     c->mass_unit = uniform;
@@ -294,13 +298,17 @@ double input_mass(hy_pm_ctx* c, uint64_t n, const double* masses, double uniform
         // because n (< 2^53) is exact.
         M = uniform * static_cast<double>(n);
     } else {
-        std::vector<double> h(n);
-        if (host_ptrs) std::memcpy(h.data(), masses, n * sizeof(double));
-        else hip_check(hipMemcpyAsync(h.data(), masses, n * sizeof(double), hipMemcpyDeviceToHost, c->stream), "mass copy");
+        unsigned long long* w = c->mass_in;  // digit counters, maximum, ticket, results
+        double* out = reinterpret_cast<double*>(w + hy::SA_WORDS + 2);
+        hipLaunchKernelGGL(hy::k_input_mass, dim3((uint32_t)std::min<uint64_t>(blocks_for(n, 1024), 1024)), dim3(256),
+                           0, c->stream, n, masses, w, w + hy::SA_WORDS,
+                           reinterpret_cast<uint32_t*>(w + hy::SA_WORDS + 1), out);
+        launch_check("k_input_mass");
+        hip_check(hipMemcpyAsync(c->hstatus->mass_in, out, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream),
+                  "mass copy");
         hip_check(hipStreamSynchronize(c->stream), "sync");
-        M = hy::host::exact_sum(h.data(), n);
-        double mx = 0.0;
-        for (double v : h) mx = v > mx ? v : mx;
+        M = c->hstatus->mass_in[0];
+        const double mx = c->hstatus->mass_in[1];
         c->mass_unit = mx > 0.0 ? mx : 1.0;
         if (!std::isfinite(M)) fail(HY_EINVAL, "PMSolver explicit masses must be finite and non-negative");
     }
@@ -375,16 +383,13 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
     }
 }
 
-void reset_status(hy_pm_ctx* c) {
-    fill_u32(c, c->err, 1);
-    fill_u32(c, c->scratch_cursor, 2);
-}
+void reset_status(hy_pm_ctx* c) { fill_u32(c, c->err, 1); }
 
 // Copy err / grand total / deposited mass to the host and synchronise.
 hy_pm_ctx::Status fetch_status(hy_pm_ctx* c) {
-    hip_check(hipMemcpyAsync(&c->hstatus->err, c->err, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream), "status");
-    hip_check(hipMemcpyAsync(&c->hstatus->total, c->grand_total, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream), "status");
-    hip_check(hipMemcpyAsync(&c->hstatus->mass, c->mass_total, sizeof(double), hipMemcpyDeviceToHost, c->stream), "status");
+    // err, grand_total and the first box's mass are adjacent: one copy
+    hip_check(hipMemcpyAsync(c->hstatus, c->err, offsetof(hy_pm_ctx::Status, mass_in), hipMemcpyDeviceToHost,
+                             c->stream), "status");
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     return *c->hstatus;
 }
@@ -451,7 +456,7 @@ DepositPlan plan_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double
     }
     P.direct = (exact_mean && std::isfinite(inv_volume) && inv_volume > 0.0) ? 1 : 0;
     P.sa = sa_quanta(c->mass_unit);
-    P.dense_count = c->mass_digits + (uint64_t)hy::SA_WORDS * c->nbox;
+    P.dense_count = c->dense_count;
     P.dense_list = c->dense_list;
     P.scratch = c->scratch;
     P.scratch_cap = c->scratch_cap;
@@ -478,15 +483,14 @@ long double mass_tol_factor(const hy_pm_ctx* c, uint64_t n) {
     return f;
 }
 
-// status_check: also evaluate the routing identity and the mass bound on the
-// device (error bits reported by the synchronous check or hy_pm_check).
+// Also evaluates the routing identity and the mass bound on the device (error
+// bits reported by the synchronous check or hy_pm_check).
 // Binary32: the records lie in the layout start (dense offsets unless
 // carried in a capacity layout, whose overflow prefix is ovf).
-void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, bool status_check = true,
-                    const uint32_t* start = nullptr, const uint32_t* ovf = nullptr) {
-    // with the two job counts and the scratch cursor of the deposit behind them
-    fill_u32(c, c->mass_digits, ((uint64_t)hy::SA_WORDS * c->nbox + 3) * 2);
+void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, const uint32_t* start = nullptr,
+                    const uint32_t* ovf = nullptr) {
     if (c->prec == HY_PREC_FP64) {
+        fill_u32(c, c->dense_count, 6);  // the two job counts and the list cursor
         auto launch = [&](auto kern, uint64_t blocks) {
             hipLaunchKernelGGL(kern, dim3((uint32_t)blocks), dim3(hy::DEP_THREADS), 0, c->stream, P,
                                static_cast<double*>(c->R));
@@ -509,23 +513,19 @@ void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, bool status_check = tr
                            static_cast<float*>(c->R));
     }
     launch_check("k_deposit");
+    if (P.raw) return;  // signed values: no mass identity
     // the exact sum of every cell's deposited mass (ExactPositiveDoubleSum), per box
+    hy::DepositCheck chk{c->grand_total, P.n, P.total_mass,
+                         static_cast<double>(mass_tol_factor(c, P.n / c->nbox)), 1, c->err};
     const uint64_t waves = c->ntiles * hy::SA_WAVES_PER_TILE;
     const dim3 rgrid((uint32_t)std::min<uint64_t>(256, blocks_for(waves, 256)), c->nbox);
     if (c->prec == HY_PREC_FP64)
-        hipLaunchKernelGGL(hy::k_mass_reduce, rgrid, dim3(256), 0, c->stream, c->mass_waves, waves, c->mass_digits);
+        hipLaunchKernelGGL(hy::k_mass_finish, rgrid, dim3(256), 0, c->stream, c->mass_waves, waves, c->mass_digits,
+                           c->tickets, c->mass_total, chk);
     else
-        hipLaunchKernelGGL(hy::k_mass_reduce_fixed, rgrid, dim3(256), 0, c->stream, c->mass_waves, waves,
-                           c->mass_unit, c->mass_digits);
-    hipLaunchKernelGGL(hy::k_mass_exact, dim3((uint32_t)blocks_for(c->nbox, 64)), dim3(64), 0, c->stream,
-                       c->mass_digits, c->nbox, c->mass_total);
-    launch_check("k_mass_exact");
-    if (status_check) {
-        const double tol = static_cast<double>(mass_tol_factor(c, P.n / c->nbox));
-        hipLaunchKernelGGL(hy::k_deposit_status, dim3((uint32_t)blocks_for(c->nbox, 256)), dim3(256), 0, c->stream,
-                           c->grand_total, P.n, c->mass_total, c->nbox, P.total_mass, tol, c->err);
-        launch_check("k_deposit_status");
-    }
+        hipLaunchKernelGGL(hy::k_mass_finish_fixed, rgrid, dim3(256), 0, c->stream, c->mass_waves, waves,
+                           c->mass_unit, c->mass_digits, c->tickets, c->mass_total, chk);
+    launch_check("k_mass_finish");
 }
 
 template <typename T>
@@ -801,7 +801,7 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
     }
     mark(c, HY_STAGE_BUCKET + 1);
     auto plan = plan_deposit(c, n, x, y, z, masses, uniform, Min, shift);
-    launch_deposit(c, plan.P, true, start, ovf);
+    launch_deposit(c, plan.P, start, ovf);
     mark(c, HY_STAGE_DEPOSIT + 1);
     c->last_input_mass = Min;
     if (!sync) return;
@@ -810,7 +810,7 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
         if (carried && (st.err & hy::ERR_STALE_KEYS)) {
             // the positions changed since the keys were made: route them afresh
             // (coordinate errors of the stale routing are its artefacts)
-            raise_errors(st.err & (hy::ERR_POSITION_NONFINITE | hy::ERR_MASS_INVALID));
+            raise_errors(st.err & hy::ERR_POSITION_NONFINITE);
             carried = false;
             reset_status(c);
             bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, false, masses, nullptr, shift);
@@ -839,6 +839,14 @@ void ensure_host_staging(hy_pm_ctx* c) {
         c->hpos = (double*)c->alloc(c->cap * 4 * sizeof(double));
         c->hacc = (double*)c->alloc(c->cap * 3 * sizeof(double));
     }
+}
+
+// Device copy of a host-pointer call's masses.
+const double* stage_masses(hy_pm_ctx* c, uint64_t n, const double* masses) {
+    ensure_host_staging(c);
+    double* s = c->hpos + 3 * c->cap;
+    hip_check(hipMemcpyAsync(s, masses, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
+    return s;
 }
 
 void require_particles(hy_pm_ctx* c, uint64_t n) {
@@ -1071,10 +1079,12 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         c->counts = (uint32_t*)c->alloc(nb_max * 4);
         c->offsets = (uint32_t*)c->alloc((nb_max + 1) * 4);
         c->block_sums = (uint32_t*)c->alloc((blocks_for(nb_max, hy::SCAN_TILE) + 1) * 4);
-        c->grand_total = (uint32_t*)c->alloc(16);
         c->xcounts = (uint32_t*)c->alloc((size_t)N * 4);
         c->xoffsets = (uint32_t*)c->alloc(((size_t)N + 1) * 4);
-        c->mass_digits = (unsigned long long*)c->alloc(((uint64_t)hy::SA_WORDS * c->nbox + 3) * 8);
+        c->mass_digits = (unsigned long long*)c->alloc((uint64_t)hy::SA_WORDS * c->nbox * 8);
+        c->tickets = (uint32_t*)c->alloc((uint64_t)c->nbox * 4);
+        c->dense_count = (unsigned long long*)c->alloc(3 * 8);
+        c->mass_in = (unsigned long long*)c->alloc((hy::SA_WORDS + 4) * 8);
         if (c->prec == HY_PREC_FP64) {
             // one job per tile, or at most 64 and one per DEP_JOB_RECORDS records
             // of the tile; a record lies in at most eight tiles
@@ -1085,11 +1095,14 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         }
         const uint64_t wave_words = c->prec == HY_PREC_FP64 ? hy::SA_WAVE_WORDS : 2;  // window, or digit-sum pair
         c->mass_waves = (unsigned long long*)c->alloc(wave_words * hy::SA_WAVES_PER_TILE * c->ntiles * c->nbox * 8);
-        c->mass_total = (double*)c->alloc(std::max<uint64_t>(2, c->nbox) * 8);
+        // status words as Status mirrors them: err, grand_total, then the masses
+        const size_t status_bytes = 8 + (size_t)c->nbox * 8;
+        c->err = (uint32_t*)c->alloc(status_bytes);
+        c->grand_total = c->err + 1;
+        c->mass_total = reinterpret_cast<double*>(c->err + 2);
         c->scratch_cap = 2 * cap + (1u << 16);
         c->scratch = (uint64_t*)c->alloc(c->scratch_cap * 8);
         c->scratch_cursor = (unsigned long long*)c->alloc(16);
-        c->err = (uint32_t*)c->alloc(16);
         if (c->prec == HY_PREC_FP64) {
             c->rec64 = (hy::DepRecord64*)c->alloc(cap * sizeof(hy::DepRecord64));
             c->rec_mass64 = (double*)c->alloc(cap * sizeof(double));
@@ -1117,9 +1130,11 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         c->gz = c->alloc(cap * rb);
         hip_check(hipHostMalloc((void**)&c->hstatus, sizeof(hy_pm_ctx::Status), hipHostMallocDefault), "hipHostMalloc");
         hip_check(hipHostMalloc((void**)&c->hmass, c->nbox * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
-        hip_check(hipMemset(c->err, 0, 16), "memset");
-        hip_check(hipMemset(c->mass_total, 0, 16), "memset");
-        hip_check(hipMemset(c->grand_total, 0, 16), "memset");
+        hip_check(hipMemset(c->err, 0, status_bytes), "memset");
+        // left cleared by every kernel that uses them
+        hip_check(hipMemset(c->mass_digits, 0, (uint64_t)hy::SA_WORDS * c->nbox * 8), "memset");
+        hip_check(hipMemset(c->tickets, 0, (uint64_t)c->nbox * 4), "memset");
+        hip_check(hipMemset(c->mass_in, 0, (hy::SA_WORDS + 4) * 8), "memset");
         hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
         *out = c.release();
     });
@@ -1181,11 +1196,8 @@ int hy_pm_density(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, co
         c->keys_ready = c->rec_ready = false;
         require_particles(c, n);
         set_boxes(c, n);
-        const double M = input_mass(c, n, masses, uniform, false);
+        const double M = input_mass(c, n, masses, uniform);
         reset_status(c);
-        if (masses) {
-            hipLaunchKernelGGL(hy::k_check_mass, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, masses, c->err);
-        }
         run_deposit(c, n, x, y, z, masses, uniform, M, true);
         const size_t bytes = (size_t)c->N * c->N * c->N * c->real_bytes;
         hip_check(hipMemcpyAsync(mesh_out, c->R, bytes, hipMemcpyDeviceToDevice, c->stream), "copy mesh");
@@ -1376,8 +1388,9 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             if (c->method != HY_METHOD_PURE_PM)
                 fail(HY_EINVAL, "potential-energy collection takes a pure-PM context");
         }
-        const double M = input_mass(c, nper, masses, uniform, host);
         const double *dx_ = x, *dy_ = y, *dz_ = z, *dm = masses;
+        if (host && masses) dm = stage_masses(c, n, masses);
+        const double M = input_mass(c, nper, dm, uniform);
         if (host) {
             ensure_host_staging(c);
             double* s = c->hpos;
@@ -1385,13 +1398,8 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             hip_check(hipMemcpyAsync(s + c->cap, y, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             hip_check(hipMemcpyAsync(s + 2 * c->cap, z, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             dx_ = s; dy_ = s + c->cap; dz_ = s + 2 * c->cap;
-            if (masses) {
-                hip_check(hipMemcpyAsync(s + 3 * c->cap, masses, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
-                dm = s + 3 * c->cap;
-            }
         }
         reset_status(c);
-        if (dm) hipLaunchKernelGGL(hy::k_check_mass, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, dm, c->err);
         run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, true);
         auto fill = [&](auto& a) {
             a.g = c->geom; a.n = n;
@@ -1489,11 +1497,9 @@ int hy_pm_kdk(hy_pm_ctx* c, uint64_t n, const double* x_in, const double* y_in, 
         const bool sync = (flags & HY_ASYNC) == 0;
         const uint64_t nper = set_boxes(c, n);
         if (masses && c->nbox > 1) fail(HY_EINVAL, "explicit masses take a single-box context");
-        const double M = input_mass(c, nper, masses, uniform, false);
+        const double M = input_mass(c, nper, masses, uniform);
         if (sync) reset_status(c);
-        else fill_u32(c, c->scratch_cursor, 2);
-        if (masses) hipLaunchKernelGGL(hy::k_check_mass, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, masses, c->err);
-        // keys (or records) of the previous fused step are valid for exactly its
+            // keys (or records) of the previous fused step are valid for exactly its
         // output positions
         const bool reuse = (flags & HY_REUSE_KEYS) != 0;
         const bool carried = reuse && c->keys_ready && c->keys_n == n && c->keys_x == x_in && c->keys_y == y_in &&
@@ -1579,6 +1585,7 @@ int hy_pm_bucket_order(hy_pm_ctx* c, uint64_t n, const double* x, const double* 
         require_particles(c, n);
         set_boxes(c, n);
         reset_status(c);
+        fill_u32(c, c->scratch_cursor, 2);
         bucketize(c, n, x, y, z, 0, c->counts, offsets, c->nb, order);
         hipLaunchKernelGGL(hy::k_canonicalize, dim3(std::min<uint64_t>(c->nb, 65535)), dim3(hy::CANON_THREADS), 0,
                            c->stream, c->nb, offsets, order, c->scratch, c->scratch_cap, c->scratch_cursor, c->err);
@@ -1598,6 +1605,7 @@ int hy_pm_xplane_order(hy_pm_ctx* c, uint64_t n, const double* x, uint32_t* orde
         require_particles(c, n);
         set_boxes(c, n);
         reset_status(c);
+        fill_u32(c, c->scratch_cursor, 2);
         bucketize(c, n, x, x, x, 1, c->xcounts, offsets, (uint64_t)c->N, order);
         hipLaunchKernelGGL(hy::k_canonicalize, dim3(c->N), dim3(hy::CANON_THREADS), 0, c->stream,
                            (uint64_t)c->N, offsets, order, c->scratch, c->scratch_cap, c->scratch_cursor, c->err);
@@ -1709,7 +1717,7 @@ int hy_pm_autotune_gather(hy_pm_ctx* c, uint64_t n, const double* x, const doubl
         require_particles(c, n);
         set_boxes(c, n);
         c->keys_ready = c->rec_ready = false;
-        const double M = input_mass(c, n, nullptr, uniform, false);
+        const double M = input_mass(c, n, nullptr, uniform);
         reset_status(c);
         run_deposit(c, n, x, y, z, nullptr, uniform, M, true);  // the potential of these positions
         run_fft(c);
@@ -1817,7 +1825,7 @@ void deposit_values(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, 
         hipLaunchKernelGGL(hy::k_scatter_values<double>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, q,
                            1.0, c->keys, c->ranks, c->offsets, c->rec_mass64);
     launch_check("k_scatter_values");
-    launch_deposit(c, plan.P, false);
+    launch_deposit(c, plan.P);
 }
 
 }  // namespace
@@ -1838,7 +1846,7 @@ int hy_pm_kdk_vjp(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, co
         require_particles(c, n);
         set_boxes(c, n);
         c->keys_ready = c->rec_ready = false;
-        const double M = input_mass(c, n, nullptr, uniform, false);
+        const double M = input_mass(c, n, nullptr, uniform);
         ensure_adjoint_workspace(c);
         reset_status(c);
         // momentum adjoint entering the kick: u = lp + d_next lx
@@ -2040,9 +2048,10 @@ int hy_pm_power_spectrum(hy_pm_ctx* c, uint64_t n, const double* x, const double
             hip_check(hipStreamSynchronize(c->stream), "sync");
             msf = hy::host::mass_square_fraction(h.data(), n, nullptr);
         }
-        const double M = input_mass(c, n, masses, uniform, host);
-
         const double *px = x, *py = y, *pz = z, *pm = masses;
+        if (host && masses) pm = stage_masses(c, n, masses);
+        const double M = input_mass(c, n, pm, uniform);
+
         if (host) {
             ensure_host_staging(c);
             double* s = c->hpos;
@@ -2050,10 +2059,6 @@ int hy_pm_power_spectrum(hy_pm_ctx* c, uint64_t n, const double* x, const double
             hip_check(hipMemcpyAsync(s + c->cap, y, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             hip_check(hipMemcpyAsync(s + 2 * c->cap, z, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             px = s; py = s + c->cap; pz = s + 2 * c->cap;
-            if (masses) {
-                hip_check(hipMemcpyAsync(s + 3 * c->cap, masses, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
-                pm = s + 3 * c->cap;
-            }
         }
         const uint64_t ccount = (uint64_t)N * (uint64_t)(N / 2 + 1) * (uint64_t)N;
         if (interlaced && !c->pk_aux) c->pk_aux = c->alloc(ccount * 2 * c->real_bytes);

@@ -21,7 +21,6 @@ namespace hy {
 enum : uint32_t {
     ERR_POSITION_NONFINITE = 1u << 0,  // invalid_argument "CIC positions must be finite"
     ERR_COORDINATE = 1u << 1,          // logic_error from CICCoordinateAxis
-    ERR_MASS_INVALID = 1u << 2,        // invalid_argument (negative / non-finite mass)
     ERR_SCRATCH = 1u << 3,             // runtime_error: deposit scratch exhausted
     ERR_FIELD_NONFINITE = 1u << 4,     // invalid_argument: potential not finite
     ERR_FORCE_NONFINITE = 1u << 5,     // overflow_error: gathered force not finite

@@ -506,7 +506,7 @@ constexpr int DEP_NRANGES = 20;
 // 2^-1074 .. 2^1230 (every binary64 bit), each holding its digit's sum with
 // the carries in its upper bits, plus a word flagging an input that is not a
 // finite non-negative number.  The counters are integers, so the total is
-// exact whatever the order of the additions; k_mass_exact rounds it once to
+// exact whatever the order of the additions; sa_round rounds it once to
 // nearest (ties to even), as the host's exact_sum does.
 // ---------------------------------------------------------------------------
 constexpr int SA_DIGITS = 72;
@@ -514,8 +514,8 @@ constexpr int SA_WORDS = SA_DIGITS + 1;
 // Each wave of a binary64 deposit workgroup stores its sum as a window of
 // SA_WAVE_WIN counters from a base digit (SA_WAVE_WORDS words: base, window;
 // base -1: empty); digits outside the window go to the box's counters
-// directly.  k_mass_reduce adds the windows up per box.  (Binary32 waves store
-// the two digit sums of their fixed-point cells; k_mass_reduce_fixed.)
+// directly.  k_mass_finish adds the windows up per box.  (Binary32 waves store
+// the two digit sums of their fixed-point cells; k_mass_finish_fixed.)
 constexpr int SA_WAVE_WIN = 8;
 constexpr int SA_WAVE_WORDS = SA_WAVE_WIN + 1;
 constexpr int SA_WAVES_PER_TILE = 8;  // deposit workgroups of 512 threads
@@ -1889,7 +1889,7 @@ __global__ void __launch_bounds__(DEPFX_THREADS) k_deposit_fixed(DepFxParams Q, 
             mesh[(gx * g.N + gy) * g.N + gz] = contrast_fp32(mcell, P);
         }
     }
-    // each wave's two digit sums (below 2^41), for k_mass_reduce_fixed
+    // each wave's two digit sums (below 2^41), for k_mass_finish_fixed
     static_assert(DEPFX_THREADS / 64 == SA_WAVES_PER_TILE, "one mass pair per wave");
     if (P.raw) dig0 = dig1 = 0;  // signed cells: no mass identity
     const uint64_t s0 = wave_sum_u64(dig0), s1 = wave_sum_u64(dig1);
@@ -1916,14 +1916,120 @@ __global__ void k_set_factors(double* __restrict__ f, double k_prev, double k_ne
     }
 }
 
-// Per box (grid row): the waves' digit windows added up, windows of nearby
-// bases in a thread's registers first, then LDS counters, then one atomic per
-// non-zero counter and workgroup into the box's counters.  Integer sums: the
-// total is exact whatever the order.
-__global__ void __launch_bounds__(256) k_mass_reduce(const unsigned long long* __restrict__ waves,
-                                                     uint64_t waves_per_box,
-                                                     unsigned long long* __restrict__ digits) {
-    __shared__ unsigned long long cnt[SA_DIGITS];
+// The exact sum held by the digit counters d (LDS, SA_DIGITS + 2 words, each
+// below 2^62), rounded once to nearest with ties to even; the first wave calls
+// it, d is normalised in place and lane 0 holds the result.  The carry chain
+// runs over the digits in use only (a handful: the masses of a box lie within
+// a few binary orders of each other).
+__device__ __forceinline__ double sa_round(unsigned long long* d) {
+    constexpr int ND = SA_DIGITS + 2;
+    const int lane = (int)lane_id();
+    const uint64_t m0 = __ballot(d[lane] != 0ull);
+    const uint64_t m1 = __ballot(lane < SA_DIGITS - 64 && d[64 + lane] != 0ull);
+    if (!(m0 | m1)) return 0.0;
+    double out = 0.0;
+    if (lane == 0) {
+        const int first = m0 ? __ffsll((unsigned long long)m0) - 1 : 64 + __ffsll((unsigned long long)m1) - 1;
+        const int last = m1 ? 127 - __clzll(m1) : 63 - __clzll(m0);
+        d[SA_DIGITS] = d[SA_DIGITS + 1] = 0ull;
+        uint64_t carry = 0;
+        int end = first;  // one past the highest digit written
+        for (int i = first; i < ND && (i <= last || carry); ++i) {
+            const uint64_t sum = d[i] + carry;
+            d[i] = sum & 0xffffffffull;
+            carry = sum >> 32;
+            end = i + 1;
+        }
+        int top = -1;
+        for (int i = end - 1; i >= first && top < 0; --i)
+            if (d[i]) top = i * 32 + (31 - __clz((uint32_t)d[i]));
+        auto digit = [&](int i) -> uint64_t { return i >= first && i < end ? d[i] : 0ull; };
+        // bits [lo, lo + 64) of the sum
+        auto bits64 = [&](int lo) -> uint64_t {
+            const int i = lo >> 5, o = lo & 31;
+            const uint64_t v = digit(i) >> o | digit(i + 1) << (32 - o);
+            return o ? v | digit(i + 2) << (64 - o) : v;
+        };
+        if (top < 53) {
+            out = ldexp((double)(bits64(0) & ((1ull << 53) - 1ull)), -1074);
+        } else {
+            const int lo = top - 52, r = lo - 1;  // r: the rounding bit
+            uint64_t m = bits64(lo) & ((1ull << 53) - 1ull);
+            const uint32_t rd = (uint32_t)digit(r >> 5);
+            bool sticky = (rd & ((1u << (r & 31)) - 1u)) != 0u;
+            for (int i = first; i < (r >> 5) && !sticky; ++i) sticky = d[i] != 0ull;
+            if (((rd >> (r & 31)) & 1u) && (sticky || (m & 1ull))) ++m;
+            out = ldexp((double)m, lo - 1074);
+        }
+    }
+    return out;
+}
+
+// Last workgroup of a grid row to arrive at ticket (reset for the next launch);
+// its later reads see what the others wrote before arriving.
+__device__ __forceinline__ bool last_block(uint32_t* ticket) {
+    __shared__ uint32_t arrived;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        arrived = atomicAdd(ticket, 1u);
+        if (arrived == gridDim.x - 1) atomicExch(ticket, 0u);
+    }
+    __syncthreads();
+    const bool last = arrived == gridDim.x - 1;
+    if (last) __threadfence();
+    return last;
+}
+
+// Takes a box's digit counters (SA_WORDS words) into LDS and clears them for the
+// next deposit; the flag word's value to flag.  The whole workgroup.
+__device__ __forceinline__ void sa_take(unsigned long long* d, unsigned long long* cnt, unsigned long long* flag) {
+    for (int w = threadIdx.x; w < SA_WORDS; w += blockDim.x) {
+        const unsigned long long v = atomicExch(&d[w], 0ull);
+        if (w < SA_DIGITS) cnt[w] = v;
+        else *flag = v;
+    }
+    __syncthreads();
+}
+
+// Deposit status on the device, so that calls which do not synchronise stay
+// fail-closed: the routing-count identity of the x-plane bins
+// (src/mesh/mass_assignment_deposit.inc:269-284: every particle routed exactly
+// once) and the mass-conservation bound of src/math/cic_mass_conservation.cpp:
+// 25-63 per box, |deposited - input| <= tol_factor * max(input, deposited)
+// with a finite positive deposited mass.
+struct DepositCheck {
+    const uint32_t* grand_total;  // routed particles
+    uint64_t n;
+    double input_per_box, tol_factor;
+    int check;                    // 0: sums only
+    uint32_t* err;
+};
+
+__device__ __forceinline__ void deposit_check(const DepositCheck& c, uint32_t box, double dep) {
+    if (!c.check) return;
+    uint32_t bits = 0;
+    if (box == 0 && (uint64_t)*c.grand_total != c.n) bits |= ERR_ROUTING;
+    const double scale = dep > c.input_per_box ? dep : c.input_per_box;
+    if (!isfinite(dep) || !(dep > 0.0) || fabs(dep - c.input_per_box) > c.tol_factor * scale)
+        bits |= ERR_MASS_CONSERVATION;
+    if (bits) atomicOr(c.err, bits);
+}
+
+// Per box (grid row): the deposit's mass records added up, the box's exact mass
+// rounded (NaN when a cell was not a finite non-negative number) and checked
+// by the row's last workgroup.  One launch in place of the former reduction,
+// one-thread rounding (15 to 40 us over a private digit array) and status
+// kernels.  Integer sums: exact whatever the order.
+// Binary64: the waves' digit windows, those of nearby bases in a thread's
+// registers first, then LDS counters, then one atomic per non-zero counter
+// and workgroup.
+__global__ void __launch_bounds__(256) k_mass_finish(const unsigned long long* __restrict__ waves,
+                                                     uint64_t waves_per_box, unsigned long long* digits,
+                                                     uint32_t* tickets, double* __restrict__ mass_total,
+                                                     DepositCheck chk) {
+    __shared__ unsigned long long cnt[SA_DIGITS + 2];
+    __shared__ unsigned long long flag;
     const uint64_t box = blockIdx.y;
     for (int w = threadIdx.x; w < SA_DIGITS; w += blockDim.x) cnt[w] = 0ull;
     __syncthreads();
@@ -1960,19 +2066,31 @@ __global__ void __launch_bounds__(256) k_mass_reduce(const unsigned long long* _
             if (acc[j] && tb + j < SA_DIGITS) atomicAdd(&cnt[tb + j], (unsigned long long)acc[j]);
     }
     __syncthreads();
+    unsigned long long* d = digits + box * SA_WORDS;
     for (int w = threadIdx.x; w < SA_DIGITS; w += blockDim.x)
-        if (cnt[w]) atomicAdd(&digits[box * SA_WORDS + w], cnt[w]);
+        if (cnt[w]) atomicAdd(&d[w], cnt[w]);
+    if (!last_block(&tickets[box])) return;
+    sa_take(d, cnt, &flag);
+    if (threadIdx.x >= 64) return;
+    const double total = sa_round(cnt);
+    if (threadIdx.x == 0) {
+        const double dep = flag ? __builtin_nan("") : total;
+        mass_total[box] = dep;
+        deposit_check(chk, (uint32_t)box, dep);
+    }
 }
 
-// Binary32 deposit: per box (grid row), the waves' digit-sum pairs (s0, s1)
-// added up per workgroup (below 2^54 each: at most 2^13 waves of under 2^41
-// per thread at the grid's 2^16 threads per box and a mesh of 4096^3), and
-// the workgroup's exact total (s0 + s1 2^32) * unit * 2^-32 added to the box's
-// counters as digits.
-__global__ void __launch_bounds__(256) k_mass_reduce_fixed(const unsigned long long* __restrict__ waves,
+// Binary32: the waves' digit-sum pairs (s0, s1) added up per workgroup (below
+// 2^54 each: at most 2^13 waves of under 2^41 per thread at the grid's 2^16
+// threads per box and a mesh of 4096^3), and the workgroup's exact total
+// (s0 + s1 2^32) * unit * 2^-32 added to the box's counters as digits.
+__global__ void __launch_bounds__(256) k_mass_finish_fixed(const unsigned long long* __restrict__ waves,
                                                            uint64_t waves_per_box, double unit,
-                                                           unsigned long long* __restrict__ digits) {
+                                                           unsigned long long* digits, uint32_t* tickets,
+                                                           double* __restrict__ mass_total, DepositCheck chk) {
     __shared__ uint64_t part[2][4];
+    __shared__ unsigned long long cnt[SA_DIGITS + 2];
+    __shared__ unsigned long long flag;
     const uint64_t box = blockIdx.y;
     typedef unsigned long long U2 __attribute__((ext_vector_type(2)));
     uint64_t s0 = 0, s1 = 0;
@@ -1989,98 +2107,111 @@ __global__ void __launch_bounds__(256) k_mass_reduce_fixed(const unsigned long l
         part[1][threadIdx.x / 64] = s1;
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    uint64_t a0 = 0, a1 = 0;
-    for (int w = 0; w < (int)blockDim.x / 64; ++w) {
-        a0 += part[0][w];
-        a1 += part[1][w];
-    }
-    const uint64_t q0 = a0 + (a1 << 32);
-    const uint64_t q1 = (a1 >> 32) + (q0 < a0 ? 1ull : 0ull);
     unsigned long long* d = digits + box * SA_WORDS;
-    int limb = 0;
-    uint32_t dig[SA_WAVE_WIN];
-    if (!sa_fixed_digits(q0, q1, unit, limb, dig)) {
-        atomicOr(&d[SA_DIGITS], 1ull);
-        return;
-    }
-    for (int k = 0; k < SA_WAVE_WIN; ++k)
-        if (dig[k] && limb + k < SA_DIGITS) atomicAdd(&d[limb + k], (unsigned long long)dig[k]);
-}
-
-// Per box: the exact deposited mass from its counters, rounded once to nearest
-// with ties to even (NaN when a cell was not a finite non-negative number).
-// One thread per box.
-__global__ void k_mass_exact(const unsigned long long* __restrict__ digits, uint32_t nbox,
-                             double* __restrict__ out) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbox) return;
-    const unsigned long long* d = digits + (uint64_t)b * SA_WORDS;
-    if (d[SA_DIGITS]) {
-        out[b] = __builtin_nan("");
-        return;
-    }
-    constexpr int ND = SA_DIGITS + 2;
-    uint32_t v[ND];
-    uint64_t carry = 0;
-    for (int i = 0; i < SA_DIGITS; ++i) {
-        const uint64_t sum = d[i] + carry;  // d[i] < 2^62, carry < 2^32
-        v[i] = (uint32_t)sum;
-        carry = sum >> 32;
-    }
-    v[SA_DIGITS] = (uint32_t)carry;
-    v[SA_DIGITS + 1] = (uint32_t)(carry >> 32);
-    int top = -1;
-    for (int i = ND - 1; i >= 0 && top < 0; --i)
-        if (v[i]) top = i * 32 + (31 - __clz(v[i]));
-    if (top < 0) {
-        out[b] = 0.0;
-        return;
-    }
-    // bits [lo, lo + 64) of the sum
-    auto bits64 = [&](int lo) -> uint64_t {
-        uint64_t r = 0;
-        for (int k = 0; k < 3; ++k) {
-            const int i = (lo >> 5) + k;
-            if (i < 0 || i >= ND) continue;
-            const int sh = k * 32 - (lo & 31);
-            const uint64_t w = v[i];
-            r |= sh >= 0 ? (sh < 64 ? w << sh : 0ull) : w >> (-sh);
+    if (threadIdx.x == 0) {
+        uint64_t a0 = 0, a1 = 0;
+        for (int w = 0; w < (int)blockDim.x / 64; ++w) {
+            a0 += part[0][w];
+            a1 += part[1][w];
         }
-        return r;
-    };
-    if (top < 53) {
-        out[b] = ldexp((double)(bits64(0) & ((1ull << 53) - 1ull)), -1074);
-        return;
+        const uint64_t q0 = a0 + (a1 << 32);
+        const uint64_t q1 = (a1 >> 32) + (q0 < a0 ? 1ull : 0ull);
+        int limb = 0;
+        uint32_t dig[SA_WAVE_WIN];
+        if (!sa_fixed_digits(q0, q1, unit, limb, dig)) {
+            atomicOr(&d[SA_DIGITS], 1ull);
+        } else {
+            for (int k = 0; k < SA_WAVE_WIN; ++k)
+                if (dig[k] && limb + k < SA_DIGITS) atomicAdd(&d[limb + k], (unsigned long long)dig[k]);
+        }
     }
-    const int lo = top - 52;
-    uint64_t m = bits64(lo) & ((1ull << 53) - 1ull);
-    const int r = lo - 1;  // the rounding bit
-    const bool round = (v[r >> 5] >> (r & 31)) & 1u;
-    bool sticky = (v[r >> 5] & ((1u << (r & 31)) - 1u)) != 0u;
-    for (int i = 0; i < (r >> 5) && !sticky; ++i) sticky = v[i] != 0u;
-    if (round && (sticky || (m & 1ull))) ++m;
-    out[b] = ldexp((double)m, lo - 1074);
+    if (!last_block(&tickets[box])) return;
+    sa_take(d, cnt, &flag);
+    if (threadIdx.x >= 64) return;
+    const double total = sa_round(cnt);
+    if (threadIdx.x == 0) {
+        const double dep = flag ? __builtin_nan("") : total;
+        mass_total[box] = dep;
+        deposit_check(chk, (uint32_t)box, dep);
+    }
 }
 
-// Deposit status on the device, so that calls which do not synchronise stay
-// fail-closed: the routing-count identity of the x-plane bins
-// (src/mesh/mass_assignment_deposit.inc:269-284: every particle routed exactly
-// once) and the mass-conservation bound of src/math/cic_mass_conservation.cpp:
-// 25-63 per box, |deposited - input| <= tol_factor * max(input, deposited)
-// with a finite positive deposited mass.  One thread per box.
-__global__ void k_deposit_status(const uint32_t* __restrict__ grand_total, uint64_t n,
-                                 const double* __restrict__ mass_total, uint32_t nbox, double input_per_box,
-                                 double tol_factor, uint32_t* __restrict__ err) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbox) return;
-    uint32_t bits = 0;
-    if (b == 0 && (uint64_t)*grand_total != n) bits |= ERR_ROUTING;
-    const double dep = mass_total[b];
-    const double scale = dep > input_per_box ? dep : input_per_box;
-    if (!isfinite(dep) || !(dep > 0.0) || fabs(dep - input_per_box) > tol_factor * scale)
-        bits |= ERR_MASS_CONSERVATION;
-    if (bits) atomicOr(err, bits);
+// Exact sum and maximum of explicit particle masses (out[0], out[1]; the sum
+// is NaN when a mass is not a finite non-negative number): the input-mass
+// identity of src/gravity/pm_solver.cpp:120-130, rounded once.  Each mass is
+// three 32-bit digits from its limb; a thread keeps six digit sums from one
+// limb below its first mass, which takes masses within a factor 2^64 of each
+// other, and other masses go to LDS counters.  Bound by the read of the
+// masses (8 B each); the host pass that it replaces copied them and took
+// about 3 ns per mass (3M masses: 9.4 ms -> 0.03 ms).
+__global__ void __launch_bounds__(256) k_input_mass(uint64_t n, const double* __restrict__ m,
+                                                    unsigned long long* digits, unsigned long long* max_bits,
+                                                    uint32_t* ticket, double* __restrict__ out) {
+    __shared__ unsigned long long cnt[SA_DIGITS + 2];
+    __shared__ unsigned long long flag;
+    for (int w = threadIdx.x; w < SA_DIGITS + 2; w += blockDim.x) cnt[w] = 0ull;
+    __syncthreads();
+    constexpr int AW = 6;
+    uint64_t acc[AW];
+#pragma unroll
+    for (int j = 0; j < AW; ++j) acc[j] = 0ull;
+    int tb = -1;
+    double mx = 0.0;
+    bool bad = false;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        const double x = m[i];
+        if (!isfinite(x) || x < 0.0) {
+            bad = true;
+            continue;
+        }
+        if (x == 0.0) continue;
+        mx = x > mx ? x : mx;
+        const uint64_t bits = (uint64_t)__double_as_longlong(x);
+        const int e = (int)((bits >> 52) & 0x7ff);
+        const uint64_t frac = bits & ((1ull << 52) - 1ull);
+        const uint64_t mant = e ? (frac | (1ull << 52)) : frac;
+        const int shift = e ? e - 1 : 0, limb = shift >> 5, off = shift & 31;
+        const uint64_t lo = mant << off, hi = off ? mant >> (64 - off) : 0ull;
+        if (tb < 0) tb = limb > 0 ? limb - 1 : 0;
+        const int k = limb - tb;
+        if (k >= 0 && k <= 3) {
+#pragma unroll
+            for (int o = 0; o <= 3; ++o) {
+                if (k == o) {
+                    acc[o] += (uint32_t)lo;
+                    acc[o + 1] += lo >> 32;
+                    acc[o + 2] += hi;
+                }
+            }
+        } else {
+            atomicAdd(&cnt[limb], (unsigned long long)(uint32_t)lo);
+            if (limb + 1 < SA_DIGITS) atomicAdd(&cnt[limb + 1], (unsigned long long)(lo >> 32));
+            if (limb + 2 < SA_DIGITS) atomicAdd(&cnt[limb + 2], (unsigned long long)hi);
+        }
+    }
+    if (tb >= 0) {
+#pragma unroll
+        for (int j = 0; j < AW; ++j)
+            if (acc[j] && tb + j < SA_DIGITS) atomicAdd(&cnt[tb + j], (unsigned long long)acc[j]);
+    }
+    // non-negative binary64 numbers order as their bits do
+    if (mx > 0.0) atomicMax(&cnt[SA_DIGITS], (unsigned long long)__double_as_longlong(mx));
+    if (bad) atomicOr(&cnt[SA_DIGITS + 1], 1ull);
+    __syncthreads();
+    for (int w = threadIdx.x; w < SA_DIGITS; w += blockDim.x)
+        if (cnt[w]) atomicAdd(&digits[w], cnt[w]);
+    if (threadIdx.x == 0) {
+        if (cnt[SA_DIGITS + 1]) atomicOr(&digits[SA_DIGITS], 1ull);
+        atomicMax(max_bits, cnt[SA_DIGITS]);
+    }
+    if (!last_block(ticket)) return;
+    sa_take(digits, cnt, &flag);
+    if (threadIdx.x >= 64) return;
+    const double total = sa_round(cnt);
+    if (threadIdx.x == 0) {
+        out[0] = flag ? __builtin_nan("") : total;
+        out[1] = __longlong_as_double((long long)atomicExch(max_bits, 0ull));
+    }
 }
 
 // ===========================================================================
@@ -2670,22 +2801,6 @@ __global__ void k_commit_force(uint64_t n, const T* __restrict__ gx, const T* __
     ax[p] += (double)gx[p];
     ay[p] += (double)gy[p];
     az[p] += (double)gz[p];
-}
-
-// Finite checks used by the force entry before anything is published.
-__global__ void k_check_finite(uint64_t n, const double* __restrict__ a, const double* __restrict__ b,
-                               const double* __restrict__ c, uint32_t bit, uint32_t* __restrict__ err) {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool bad = false;
-    if (p < n) bad = !isfinite(a[p]) || !isfinite(b[p]) || !isfinite(c[p]);
-    if (__ballot(bad) && lane_id() == 0) atomicOr(err, bit);
-}
-
-__global__ void k_check_mass(uint64_t n, const double* __restrict__ m, uint32_t* __restrict__ err) {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool bad = false;
-    if (p < n) bad = !isfinite(m[p]) || m[p] < 0.0;
-    if (__ballot(bad) && lane_id() == 0) atomicOr(err, ERR_MASS_INVALID);
 }
 
 // ===========================================================================
