@@ -955,6 +955,7 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         c->real_bytes = c->prec == HY_PREC_FP64 ? sizeof(double) : sizeof(float);
         c->fft32 = k32;
         c->fft64 = k64;
+        std::copy_n(c->prec == HY_PREC_FP64 ? k64.plan : k32.plan, hy::FFT_PASSES, c->fft_var);
         const double dx = L / (double)N;
         if (!std::isfinite(dx) || dx <= 0.0) fail(HY_EOVERFLOW, "MeshGeometry cell size is not representable");
         c->geom.L = L;
@@ -990,7 +991,8 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         hip_check(hipDeviceGetAttribute(&c->max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, desc->device),
                   "hipDeviceGetAttribute");
         for (int p = 0; p < hy::FFT_PASSES; ++p)
-            if (std::max(k32.pass[p][0].lds, k64.pass[p][0].lds) > c->max_lds)
+            if (std::max({k32.pass[p][0].lds, k64.pass[p][0].lds, k32.pass[p][k32.plan[p]].lds,
+                          k64.pass[p][k64.plan[p]].lds}) > c->max_lds)
                 fail(HY_EDEVICE, "device LDS per workgroup is below the FFT passes' requirement");
         if (desc->stream) {
             c->stream = static_cast<hipStream_t>(desc->stream);

@@ -1,10 +1,8 @@
-// LDS-staged pencil FFT building blocks for the PM Poisson solve (gfx950).
+// Pencil FFT building blocks for the PM Poisson solve (gfx950).
 //
-// A workgroup holds ROWS rows of LEN complex values in LDS (row stride
-// LEN+1) and runs an in-place Stockham autosort transform over all rows at
-// once: every stage each thread loads E/R radix-R butterflies into registers,
-// twiddles and transforms them, then (after a barrier) stores them at their
-// autosorted positions.  LEN = 2^a or 3*2^a; radices 3, 8, 4, 2.
+// A row of LEN complex values is transformed in two levels of register DFTs
+// (lengths A and B, LEN = A * B) with one exchange through LDS between them;
+// a workgroup holds ROWS rows.  LEN = 2^a or 3*2^a.
 //
 // Twiddles come from one table tw[m] = exp(-2*pi*i*m/NT) (NT = mesh size),
 // evaluated in binary64 on the host, read with a stride NT/LEN.
@@ -18,39 +16,6 @@
 #include "hy_device.hpp"
 
 namespace hy {
-
-// ---------------------------------------------------------------------------
-// Compile-time plan
-// ---------------------------------------------------------------------------
-template <int LEN>
-struct FftPlan {
-    static constexpr bool has3 = (LEN % 3) == 0;
-    static constexpr int E = has3 ? (LEN < 24 ? LEN : 24) : (LEN < 16 ? LEN : 16);
-    static constexpr int TPR = LEN / E;  // threads per row
-    static constexpr int radix(int s) {
-        int rem = LEN;
-        int r = 1;
-        for (int i = 0; i <= s; ++i) {
-            if (rem == 1) return 1;
-            if (i == 0 && rem % 3 == 0) r = 3;
-            else if (rem % 8 == 0) r = 8;
-            else if (rem % 4 == 0) r = 4;
-            else r = 2;
-            rem /= r;
-        }
-        return r;
-    }
-    static constexpr int stages() {
-        int s = 0;
-        while (radix(s) != 1) ++s;
-        return s;
-    }
-    static constexpr int prod_before(int s) {
-        int p = 1;
-        for (int i = 0; i < s; ++i) p *= radix(i);
-        return p;
-    }
-};
 
 // ---------------------------------------------------------------------------
 // Complex helpers
@@ -176,30 +141,64 @@ constexpr double kW32[32][2] = {
     {      0.9807852804032303,     -0.19509032201612872},
 };
 
-// exp(S 2 pi i m / R) for R | 32, as a complex constant of type C.
+// exp(2 pi i m / 24), m = 0..23, likewise.
+constexpr double kW24[24][2] = {
+    {                       1.0,                        0.0},
+    {        0.9659258262890683,        0.25881904510252074},
+    {        0.8660254037844387,        0.49999999999999994},
+    {        0.7071067811865476,         0.7071067811865475},
+    {        0.5000000000000001,         0.8660254037844386},
+    {       0.25881904510252074,         0.9659258262890683},
+    {     6.123233995736766e-17,                        1.0},
+    {      -0.25881904510252063,         0.9659258262890683},
+    {       -0.4999999999999998,         0.8660254037844387},
+    {       -0.7071067811865475,         0.7071067811865476},
+    {       -0.8660254037844387,        0.49999999999999994},
+    {       -0.9659258262890682,          0.258819045102521},
+    {                      -1.0,     1.2246467991473532e-16},
+    {       -0.9659258262890683,        -0.2588190451025208},
+    {       -0.8660254037844388,        -0.4999999999999997},
+    {       -0.7071067811865479,        -0.7071067811865471},
+    {       -0.5000000000000004,        -0.8660254037844384},
+    {      -0.25881904510252063,        -0.9659258262890683},
+    {   -1.8369701987210297e-16,                       -1.0},
+    {        0.2588190451025203,        -0.9659258262890684},
+    {        0.5000000000000001,        -0.8660254037844386},
+    {        0.7071067811865474,        -0.7071067811865477},
+    {        0.8660254037844384,        -0.5000000000000004},
+    {        0.9659258262890681,       -0.25881904510252157},
+};
+
+// exp(S 2 pi i m / R) for R | 32 or R | 24, as a complex constant of type C.
 template <int R, int S, typename C>
 HY_HD C wconst(int m) {
     using T = decltype(C{}.x);
-    const int q = ((m % R) + R) % R * (32 / R);
-    return C{(T)kW32[q][0], (T)(S * kW32[q][1])};
+    if constexpr (R % 3 == 0) {
+        static_assert(24 % R == 0, "twiddle table");
+        const int q = ((m % R) + R) % R * (24 / R);
+        return C{(T)kW24[q][0], (T)(S * kW24[q][1])};
+    } else {
+        const int q = ((m % R) + R) % R * (32 / R);
+        return C{(T)kW32[q][0], (T)(S * kW32[q][1])};
+    }
 }
 
-// In-register DFT of length R (power of two <= 32), natural order in place:
-// R = A * B with a length-A DFT over each stride-B column, the twiddle
+// In-register DFT of length R (2^a <= 32, or 3 * 2^a <= 24), natural order in
+// place: R = A * B with a length-A DFT over each stride-B column, the twiddle
 // exp(S 2 pi i n2 k1 / R), then a length-B DFT over each row.
 template <int R, int S, typename C>
 HY_HD void dft_reg(C* u) {
-    if constexpr (R <= 8) {
+    if constexpr (R == 2 || R == 3 || R == 4 || R == 8) {
         dftR<R, S>(u);
     } else {
-        constexpr int A = 4, B = R / 4;
+        constexpr int A = R % 3 == 0 ? 3 : 4, B = R / A;
         C y[R];
 #pragma unroll
         for (int n2 = 0; n2 < B; ++n2) {
             C col[A];
 #pragma unroll
             for (int n1 = 0; n1 < A; ++n1) col[n1] = u[B * n1 + n2];
-            dft4<S>(col);
+            dftR<A, S>(col);
 #pragma unroll
             for (int k1 = 0; k1 < A; ++k1)
                 y[k1 * B + n2] = (k1 * n2 == 0) ? col[k1] : cmul(col[k1], wconst<R, S, C>(k1 * n2));
@@ -216,7 +215,8 @@ HY_HD void dft_reg(C* u) {
     }
 }
 
-// Two-level row FFT of a power-of-two length LEN = A * B (A, B <= 32):
+// Two-level row FFT of length LEN = A * B (A <= B <= 32; 2^a from 4 to 1024 or
+// 3 * 2^a from 6 to 384; A and B as near each other as the length allows):
 //   level 1: thread n2 < B holds the stride-B column x[n2 + B n1] (n1 < A),
 //            transforms it (length A) and multiplies by W_LEN^(n2 k1);
 //   exchange: Y[k1][n2] through LDS (row stride B + 1);
@@ -227,7 +227,9 @@ HY_HD void dft_reg(C* u) {
 template <int LEN>
 struct TwoLevel {
     static constexpr int lg(int v) { return v <= 1 ? 0 : 1 + lg(v / 2); }
-    static constexpr int A = 1 << (lg(LEN) / 2);
+    static constexpr bool has3 = LEN % 3 == 0;
+    static constexpr int K = lg(has3 ? LEN / 3 : LEN);
+    static constexpr int A = !has3 ? 1 << (K / 2) : (K % 2 ? 1 << ((K + 1) / 2) : 3 << (K / 2 - 1));
     static constexpr int B = LEN / A;
     static constexpr int TPR = A > B ? A : B;
     static constexpr int EMAX = A > B ? A : B;
@@ -317,76 +319,6 @@ HY_HD void tl_twiddle(C* v, int col, const C* tw, int stride) {
     }
 }
 
-// LDS slot of logical element j of a row: one padding slot every 32 entries,
-// so the stride-R stores of the first Stockham stage and the row-strided
-// transposes spread over all banks.
-__device__ __forceinline__ constexpr int lds_slot(int j) { return j + (j >> 5); }
-
-template <int LEN>
-struct LdsRow {
-    static constexpr int SPAN = LEN + (LEN >> 5) + 1;          // LEN+1 logical entries
-    static constexpr int RS = (SPAN % 2 == 0) ? SPAN + 1 : SPAN;  // odd stride in complex units
-};
-
-// One Stockham stage over all rows held in LDS.
-template <typename C, int LEN, int ROWS, int RS, int STAGE, int S>
-__device__ __forceinline__ void fft_stage(C* lds, const C* __restrict__ tw, int tw_stride,
-                                          int tid) {
-    using P = FftPlan<LEN>;
-    constexpr int R = P::radix(STAGE);
-    constexpr int p = P::prod_before(STAGE);
-    constexpr int M = LEN / R;
-    constexpr int NB = P::E / R;  // butterflies per thread
-    constexpr int TPR = P::TPR;
-    const int row = tid / TPR;
-    const int t = tid % TPR;
-    C* x = lds + row * RS;
-    C v[P::E];
-    if (row < ROWS) {
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int i = t + j * TPR;
-            const int k = i % p;
-            C u[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) u[r] = x[lds_slot(i + r * M)];
-            if (k != 0) {
-#pragma unroll
-                for (int r = 1; r < R; ++r) {
-                    const int m = (r * k * (LEN / (p * R))) % LEN;
-                    C w = tw[m * tw_stride];
-                    if constexpr (S > 0) w.y = -w.y;
-                    u[r] = cmul(u[r], w);
-                }
-            }
-            dftR<R, S>(u);
-#pragma unroll
-            for (int r = 0; r < R; ++r) v[j * R + r] = u[r];
-        }
-    }
-    __syncthreads();
-    if (row < ROWS) {
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int i = t + j * TPR;
-            const int k = i % p;
-            const int base = (i - k) * R + k;
-#pragma unroll
-            for (int r = 0; r < R; ++r) x[lds_slot(base + r * p)] = v[j * R + r];
-        }
-    }
-    __syncthreads();
-}
-
-template <typename C, int LEN, int ROWS, int RS, int S, int STAGE = 0>
-__device__ __forceinline__ void fft_rows(C* lds, const C* __restrict__ tw, int tw_stride,
-                                         int tid) {
-    if constexpr (STAGE < FftPlan<LEN>::stages()) {
-        fft_stage<C, LEN, ROWS, RS, STAGE, S>(lds, tw, tw_stride, tid);
-        fft_rows<C, LEN, ROWS, RS, S, STAGE + 1>(lds, tw, tw_stride, tid);
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Per-pass launch geometry
 // ---------------------------------------------------------------------------
@@ -398,30 +330,20 @@ constexpr int kFftVariants = 4;
 constexpr int fft_lds_budget(int v) {
     return v == 0 ? 80 * 1024 : v == 1 ? 40 * 1024 : v == 2 ? 136 * 1024 : 20 * 1024;
 }
-constexpr int fft_thread_cap(int v) { return v == 2 ? 1024 : 512; }
+// Rows shorter than 64, and the y and x rows of a 64^3 mesh: 128 threads, so
+// that a small mesh still makes a workgroup or two per CU (a 64^3 mesh: 132 per
+// y pass, 16 rows each; 4.8 -> 3.2 us against one workgroup of 64 rows).  The
+// z rows of a 128^3 mesh (LEN 64) keep 64 rows: 16 of them read 128-byte runs,
+// 0.29 against 0.20 ms for 64 boxes.
+constexpr int fft_thread_cap(int v, int len, int dim) {
+    return len < 64 || (len == 64 && dim != 128) ? 128 : v == 2 ? 1024 : 512;
+}
 
 constexpr int pow2_floor(int v) {
     int p = 1;
     while (p * 2 <= v) p *= 2;
     return p;
 }
-
-// Rows per workgroup for a transform of length LEN whose rows are blocked from
-// a dimension of extent DIM (ROWS must divide DIM), launch variant V.
-template <typename T, int LEN, int DIM, int V = 0>
-struct RowsCfg {
-    using C = cplx<T>;
-    static constexpr int RS = LdsRow<LEN>::RS;
-    static constexpr int by_threads = fft_thread_cap(V) / FftPlan<LEN>::TPR;
-    static constexpr int by_lds = fft_lds_budget(V) / (RS * (int)sizeof(C));
-    static constexpr int cap = by_threads < by_lds ? by_threads : by_lds;
-    static constexpr int dim_pow2 = (DIM & (-DIM));  // largest power of two dividing DIM
-    static constexpr int ROWS0 = pow2_floor(cap < 1 ? 1 : cap);
-    static constexpr int ROWS = ROWS0 < dim_pow2 ? ROWS0 : dim_pow2;
-    static constexpr int THREADS = ROWS * FftPlan<LEN>::TPR;
-    static constexpr int LDS_BYTES = ROWS * RS * (int)sizeof(C);
-    static_assert(LDS_BYTES <= 160 * 1024, "LDS per workgroup");
-};
 
 // Launch geometry of the two-level passes: ROWS rows per workgroup, TPR
 // threads per row; the LDS holds either the per-row exchange (XS complex per
@@ -433,7 +355,7 @@ struct TLCfg {
     using TL = TwoLevel<LEN>;
     static constexpr int TPR = TL::TPR;
     static constexpr int PER_ROW = (TL::XS > LEN + 1 ? TL::XS : LEN + 1) + LEN / 8 + 1;
-    static constexpr int by_threads = fft_thread_cap(V) / TPR;
+    static constexpr int by_threads = fft_thread_cap(V, LEN, DIM) / TPR;
     static constexpr int by_lds = fft_lds_budget(V) / (PER_ROW * (int)sizeof(C));
     static constexpr int cap = by_threads < by_lds ? by_threads : by_lds;
     static constexpr int dim_pow2 = (DIM & (-DIM));

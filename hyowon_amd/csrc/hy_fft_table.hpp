@@ -27,66 +27,68 @@ struct FftKernels {
     FftPass<T> sg[3];  // spectral-gradient x, y^-1 and z^-1 passes (TreePM long range; variant 0)
     bool sg_x_dual = false;  // sg[0] writes the -i k_x and the plain inverse from one read of B
     FftPass<T> sg_y_dual;    // y^-1 pass writing the -i k_y and the plain inverse from one read of B (or none)
-    int variants = 0;  // launch variants compiled for this size (variant 0 is the default)
+    int variants = 0;  // launch variants compiled for this size
+    int plan[FFT_PASSES] = {0, 0, 0, 0, 0};  // variants a context starts with (hy_pm_autotune refines them)
 };
 
 // Sizes below this have one launch variant (their passes are latency-bound and
 // the variants collapse onto the same row counts).
 constexpr int kFftTunedFrom = 192;
+// Variant of the x passes that come in one (spectral gradient, forward or
+// inverse only) from that size up.
+constexpr int kFftXVariant = 3;
 
 // Defined in hy_fft_f32.hip / hy_fft_f64.hip; false for an unsupported size.
 bool lookup_fft(int N, FftKernels<float>& out);
 bool lookup_fft(int N, FftKernels<double>& out);
 
-// Power-of-two meshes from 128 up use the two-level register passes; the
-// others (3*2^a, small meshes) use the LDS Stockham passes.
-constexpr bool fft_two_level(int N) { return N >= 128 && (N & (N - 1)) == 0; }
-
 #ifdef HY_FFT_INSTANTIATE
 template <typename T, int N, int V>
 void fill_variant(FftKernels<T>& k) {
-    if constexpr (fft_two_level(N)) {
-        using RZ = TLCfg<T, N / 2, N, V>;
-        using RY = TLCfg<T, N, N, V>;
-        using RX = TLCfg<T, N, (N / 2 + 1) * N, V>;
-        k.pass[FFT_Z_R2C][V] = {k_tl_z_r2c<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-        k.pass[FFT_Y_FWD][V] = {k_tl_y_fwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-        k.pass[FFT_X_GREEN][V] = {k_tl_x_green<T, N, V>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
-        k.pass[FFT_Y_BWD][V] = {k_tl_y_bwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-        k.pass[FFT_Z_C2R][V] = {k_tl_z_c2r<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-        if constexpr (V == 0) {
-            k.x_fwd = {k_tl_x_dft<T, N, V, -1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
-            k.z_fwd = {k_tl_z_r2c<T, N, V, true>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-            k.x_inv = {k_tl_x_dft<T, N, V, +1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
-            if constexpr (sizeof(T) == 4) {
-                // binary32: the second held column fits the register file
-                k.sg[0] = {k_tl_x_green_dual<T, N, V>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
-                k.sg_x_dual = true;
-                k.sg_y_dual = {k_tl_y_bwd<T, N, V, 2>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-            } else {
-                k.sg[0] = {k_tl_x_green<T, N, V, 1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
-            }
-            k.sg[1] = {k_tl_y_bwd<T, N, V, 1>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-            k.sg[2] = {k_tl_z_c2r<T, N, V, 1>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-        }
-    } else {
-        using RZ = RowsCfg<T, N / 2, N, V>;
-        using RY = RowsCfg<T, N, N, V>;
-        using RX = RowsCfg<T, N, (N / 2 + 1) * N, V>;
-        k.pass[FFT_Z_R2C][V] = {k_fft_z_r2c<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-        k.pass[FFT_Y_FWD][V] = {k_fft_y_fwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-        k.pass[FFT_X_GREEN][V] = {k_fft_x_green<T, N, V>, RX::ROWS, RX::THREADS, RX::LDS_BYTES};
-        k.pass[FFT_Y_BWD][V] = {k_fft_y_bwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-        k.pass[FFT_Z_C2R][V] = {k_fft_z_c2r<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-        if constexpr (V == 0) {
-            k.x_fwd = {k_fft_x_dft<T, N, V, -1>, RX::ROWS, RX::THREADS, RX::LDS_BYTES};
-            k.z_fwd = k.pass[FFT_Z_R2C][V];  // stores every plane
-            k.x_inv = {k_fft_x_dft<T, N, V, +1>, RX::ROWS, RX::THREADS, RX::LDS_BYTES};
-            k.sg[0] = {k_fft_x_green<T, N, V, 1>, RX::ROWS, RX::THREADS, RX::LDS_BYTES};
-            k.sg[1] = {k_fft_y_bwd<T, N, V, 1>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
-            k.sg[2] = {k_fft_z_c2r<T, N, V, 1>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
+    using RZ = TLCfg<T, N / 2, N, V>;
+    using RY = TLCfg<T, N, N, V>;
+    using RX = TLCfg<T, N, (N / 2 + 1) * N, V>;
+    k.pass[FFT_Z_R2C][V] = {k_tl_z_r2c<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
+    k.pass[FFT_Y_FWD][V] = {k_tl_y_fwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
+    k.pass[FFT_X_GREEN][V] = {k_tl_x_green<T, N, V>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
+    k.pass[FFT_Y_BWD][V] = {k_tl_y_bwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
+    k.pass[FFT_Z_C2R][V] = {k_tl_z_c2r<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
+    if constexpr (V == (N >= kFftTunedFrom ? kFftXVariant : 0)) {
+        k.x_fwd = {k_tl_x_dft<T, N, V, -1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
+        k.x_inv = {k_tl_x_dft<T, N, V, +1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
+        if constexpr (sizeof(T) == 4) {
+            // binary32: the second held column fits the register file
+            k.sg[0] = {k_tl_x_green_dual<T, N, V>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
+            k.sg_x_dual = true;
+        } else {
+            k.sg[0] = {k_tl_x_green<T, N, V, 1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
         }
     }
+    if constexpr (V == 0) {
+        k.z_fwd = {k_tl_z_r2c<T, N, V, true>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
+        if constexpr (sizeof(T) == 4)
+            k.sg_y_dual = {k_tl_y_bwd<T, N, V, 2>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
+        k.sg[1] = {k_tl_y_bwd<T, N, V, 1>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
+        k.sg[2] = {k_tl_z_c2r<T, N, V, 1>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
+    }
+}
+
+// Variants a context starts with, from the measured times of all four:
+//   x + Green: the pass needs LDS for its exchange only, so small workgroups
+//     keep more of them resident: 20 KB on 2^a meshes (512^3 binary32 0.39 ->
+//     0.28 ms, binary64 0.71 -> 0.60), 40 KB on 3*2^a (384^3 0.126 -> 0.107);
+//   256^3 y and y^-1: 40 KB (0.025 -> 0.021 ms);
+//   192^3 z c2r: 64 rows in binary32 (64 boxes 1.06 -> 0.70 ms), and 16 in
+//     binary64 with z r2c (0.023 -> 0.019, 0.022 -> 0.017 ms).
+template <typename T, int N>
+constexpr int fft_plan(int pass) {
+    constexpr bool pow2 = (N & (N - 1)) == 0;
+    if (N < kFftTunedFrom) return 0;
+    if (pass == FFT_X_GREEN) return pow2 ? 3 : 1;
+    if (N == 256 && (pass == FFT_Y_FWD || pass == FFT_Y_BWD)) return 1;
+    if (N == 192 && sizeof(T) == 4 && pass == FFT_Z_C2R) return 2;
+    if (N == 192 && sizeof(T) == 8 && (pass == FFT_Z_R2C || pass == FFT_Z_C2R)) return 1;
+    return 0;
 }
 
 template <typename T, int N>
@@ -100,6 +102,7 @@ FftKernels<T> make_fft() {
         fill_variant<T, N, 3>(k);
         k.variants = kFftVariants;
     }
+    for (int p = 0; p < FFT_PASSES; ++p) k.plan[p] = fft_plan<T, N>(p);
     return k;
 }
 

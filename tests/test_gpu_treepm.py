@@ -71,8 +71,8 @@ def test_treepm_force_matches_oracle(gpu, oracle_mod, prec, tol, N, L, rs_cells,
             assert abs(a.sum()) < 1e-9 * np.abs(a).sum()
 
 
-# fp64 at N = 32 runs the LDS Stockham passes; fp32 at N = 128 runs the
-# two-level dual passes (both x outputs, and the -i k_y and plain y^-1 outputs,
+# fp64 at N = 32 runs the single-output passes; fp32 at N = 128 runs the
+# dual passes (both x outputs, and the -i k_y and plain y^-1 outputs,
 # from one read each), so each of F_x, F_y, F_z is checked on its own.
 @pytest.mark.parametrize("prec,N,L,tol", [("fp64", 32, 40.0, 1e-10), ("fp32", 128, 160.0, 1e-4),
                                           ("fp32", 256, 256.0, 1e-4)])
