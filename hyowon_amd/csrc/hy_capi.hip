@@ -343,7 +343,8 @@ void cap_scan(hy_pm_ctx* c, const uint32_t* cur, uint32_t* dense, uint32_t* capn
 // step's carried records from these counts.
 void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const double* z, int mode,
                uint32_t* counts, uint32_t* offsets, uint64_t nb, uint32_t* order, bool carried = false,
-               const double* masses = nullptr, uint32_t* capn = nullptr, double shift = 0.0) {
+               const double* masses = nullptr, uint32_t* capn = nullptr, double shift = 0.0,
+               hy::ForceRecord* force = nullptr) {
     if (!carried) {
         fill_u32(c, counts, nb);
         hipLaunchKernelGGL(hy::k_bucket_key, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y, z,
@@ -365,12 +366,12 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
     if (mode == 0 && c->prec == HY_PREC_FP32_MIXED) {
         hipLaunchKernelGGL((hy::k_scatter_records<hy::DepRecord, float>), dim3(blocks_for(n, 256)), dim3(256), 0,
                            c->stream, n, x, y, z, masses, 1.0 / c->mass_unit, c->geom, c->keys, c->ranks, offsets,
-                           order, c->rec, c->rec_mass, c->err, shift);
+                           order, c->rec, c->rec_mass, c->err, shift, force);
         launch_check("k_scatter_records");
     } else if (mode == 0) {
         hipLaunchKernelGGL((hy::k_scatter_records<hy::DepRecord64, double>), dim3(blocks_for(n, 256)), dim3(256), 0,
                            c->stream, n, x, y, z, masses, 1.0, c->geom, c->keys, c->ranks, offsets, order,
-                           c->rec64, c->rec_mass64, c->err, shift);
+                           c->rec64, c->rec_mass64, c->err, shift, (hy::ForceRecord*)nullptr);
         launch_check("k_scatter_records");
     } else if (carried) {
         hipLaunchKernelGGL(hy::k_scatter_checked, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y,
@@ -674,6 +675,27 @@ void launch_interp(hy_pm_ctx* c, hy::InterpArgs<T> a) {
     launch_check("k_interp");
 }
 
+// Force of the n particles just deposited, in record order, over their force
+// records (binary32): the gradient of the potentials in R, or the force meshes
+// R, R2, R3 of the TreePM long range.
+void launch_slot_force(hy_pm_ctx* c, uint64_t n, hy::ForceRecord* force) {
+    hy::SlotForceArgs a{};
+    a.g = c->geom;
+    a.n = n;
+    a.rec = c->rec;
+    a.force = force;
+    a.f[0] = static_cast<const float*>(c->R);
+    a.f[1] = static_cast<const float*>(c->R2);
+    a.f[2] = static_cast<const float*>(c->R3);
+    a.err = c->err;
+    const bool o32 = c->nbox == 1 && (uint64_t)c->N * c->N * c->N * sizeof(float) <= (1ull << 32);
+    const bool sg = c->method == HY_METHOD_TREEPM_LONG_RANGE;
+    auto kern = sg ? (o32 ? hy::k_slot_force<true, true> : hy::k_slot_force<true, false>)
+                   : (o32 ? hy::k_slot_force<false, true> : hy::k_slot_force<false, false>);
+    hipLaunchKernelGGL(kern, dim3((uint32_t)blocks_for(n, 256)), dim3(256), 0, c->stream, a);
+    launch_check("k_slot_force");
+}
+
 void require_pure_pm(const hy_pm_ctx* c, const char* what) {
     if (c->method != HY_METHOD_PURE_PM)
         fail(HY_EINVAL, std::string(what) + " takes a pure-PM context (the TreePM long-range force needs the "
@@ -776,7 +798,8 @@ void check_mass(hy_pm_ctx* c, double input, double deposited, uint64_t n) {
 // partner), routed and wrapped as the reference's shifted copy would be.
 void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const double* z,
                  const double* masses, double uniform, double Min, bool sync, bool carried = false,
-                 bool carried_rec = false, bool rec_out = false, double shift = 0.0) {
+                 bool carried_rec = false, bool rec_out = false, double shift = 0.0,
+                 hy::ForceRecord* force = nullptr) {
     mark(c, 0);
     // the binary32 deposit reads records only: no particle order is written
     uint32_t* order = nullptr;
@@ -797,7 +820,7 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
         start = c->cap_cur;
         ovf = c->ovf_start;
     } else {
-        bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, carried, masses, capn, shift);
+        bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, carried, masses, capn, shift, force);
     }
     mark(c, HY_STAGE_BUCKET + 1);
     auto plan = plan_deposit(c, n, x, y, z, masses, uniform, Min, shift);
@@ -1402,16 +1425,21 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             dx_ = s; dy_ = s + c->cap; dz_ = s + 2 * c->cap;
         }
         reset_status(c);
-        run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, true);
-        auto fill = [&](auto& a) {
-            a.g = c->geom; a.n = n;
-            a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
-            a.err = c->err;
-        };
-        if (c->method == HY_METHOD_TREEPM_LONG_RANGE) {
-            run_fft_sg(c);
-            auto interp = [&](auto tag) {
-                using T = decltype(tag);
+        // Binary32: the forces are gathered in record order, the force records
+        // behind the n records of the call (room for two per particle exists
+        // where the carried layout does).  Binary64 records hold the fractions
+        // of the deposit only, and gather in particle order.
+        hy::ForceRecord* slots = nullptr;
+        static_assert(sizeof(hy::ForceRecord) == sizeof(hy::DepRecord), "force records behind the deposit records");
+        if (c->rec_layout) slots = reinterpret_cast<hy::ForceRecord*>(c->rec + c->cap);
+        run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, true, false, false, false, 0.0, slots);
+        const bool sg = c->method == HY_METHOD_TREEPM_LONG_RANGE;
+        if (sg) run_fft_sg(c);
+        else run_fft(c);
+        if (collect) launch_potential_energy(c, n, dx_, dy_, dz_, dm, uniform);
+        auto gather = [&](auto tag) {
+            using T = decltype(tag);
+            if (sg) {
                 hy::InterpArgs<T> a{};
                 a.n = n;
                 a.x = dx_; a.y = dy_; a.z = dz_;
@@ -1423,26 +1451,19 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
                 a.out[2] = static_cast<T*>(c->gz);
                 a.meshes = 3;
                 launch_interp(c, a);
-            };
-            if (c->prec == HY_PREC_FP64) interp(double{});
-            else interp(float{});
-        } else {
-            run_fft(c);
-            if (collect) launch_potential_energy(c, n, dx_, dy_, dz_, dm, uniform);
-            if (c->prec == HY_PREC_FP64) {
-                hy::GatherArgs<double, double> a{};
-                fill(a);
-                a.phi = static_cast<const double*>(c->R);
-                a.g_x = (double*)c->gx; a.g_y = (double*)c->gy; a.g_z = (double*)c->gz;
-                launch_gather(c, a);
             } else {
-                hy::GatherArgs<float, float> a{};
-                fill(a);
-                a.phi = static_cast<const float*>(c->R);
-                a.g_x = (float*)c->gx; a.g_y = (float*)c->gy; a.g_z = (float*)c->gz;
+                hy::GatherArgs<T, T> a{};
+                a.g = c->geom; a.n = n;
+                a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
+                a.err = c->err;
+                a.phi = static_cast<const T*>(c->R);
+                a.g_x = (T*)c->gx; a.g_y = (T*)c->gy; a.g_z = (T*)c->gz;
                 launch_gather(c, a);
             }
-        }
+        };
+        if (slots) launch_slot_force(c, n, slots);
+        else if (c->prec == HY_PREC_FP64) gather(double{});
+        else gather(float{});
         mark(c, HY_STAGE_GATHER_KDK + 1);
         end_call(c);
         const auto st = fetch_status(c);
@@ -1461,7 +1482,10 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             hip_check(hipMemcpyAsync(cy, ay, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             hip_check(hipMemcpyAsync(cz, az, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
         }
-        if (c->prec == HY_PREC_FP64)
+        if (slots)
+            hipLaunchKernelGGL(hy::k_commit_slots, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, c->keys,
+                               c->ranks, c->offsets, slots, cx, cy, cz);
+        else if (c->prec == HY_PREC_FP64)
             hipLaunchKernelGGL(hy::k_commit_force<double>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n,
                                (const double*)c->gx, (const double*)c->gy, (const double*)c->gz, cx, cy, cz);
         else
