@@ -2756,17 +2756,62 @@ __global__ void __launch_bounds__(256) k_commit_slots(uint64_t n, const uint32_t
 // (x outer, z inner) of phi_c * ((wx wy) wz), then m * value, with the
 // reference's lost-product checks (ERR_INTERP_UNDERFLOW).  The summation is the
 // reference's deterministic blocked sum (include/cosmo_nbody/math/
-// deterministic_sum.hpp:48-104): workgroup b forms the terms of particles
-// [b*4096, (b+1)*4096) in LDS, then one lane adds them in index order with
-// Neumaier compensation; k_potential_total adds the block sums in order.
+// deterministic_sum.hpp:48-104): workgroup b adds the terms of particles
+// [b*4096, (b+1)*4096) in index order with Neumaier compensation;
+// k_potential_total adds the block sums in order.
 constexpr int ENERGY_THREADS = 256;
 constexpr int ENERGY_BLOCK = 4096;
+constexpr int ENERGY_CHUNK = 2048;  // terms in LDS at a time
 
-__device__ __forceinline__ void neumaier_add(double v, double& sum, double& comp) {
-    const double t = sum + v;
-    if (fabs(sum) >= fabs(v)) comp += (sum - t) + v;
-    else comp += (v - t) + sum;
-    sum = t;
+// Neumaier's sum over count <= ENERGY_CHUNK terms in LDS, continued from (sum,
+// comp) of thread 0, by the whole workgroup.  Only two chains are serial, one
+// addition per term each: the running sums, which thread 0 leaves in sums, and
+// the compensation; the rounding error of each step needs the two sums around
+// it and is formed by all threads (one lane doing it all: 229 cycles per term,
+// 0.45 ms for 3M particles).
+__device__ __forceinline__ void neumaier_terms(double* terms, double* sums, uint32_t count, double& sum,
+                                               double& comp) {
+    constexpr uint32_t U = 16;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = sum;
+        uint32_t i = 0;
+        for (; i + U <= count; i += U) {
+            double v[U];
+#pragma unroll
+            for (uint32_t j = 0; j < U; ++j) v[j] = terms[i + j];
+#pragma unroll
+            for (uint32_t j = 0; j < U; ++j) {
+                sums[i + j] = s;
+                s += v[j];
+            }
+        }
+        for (; i < count; ++i) {
+            sums[i] = s;
+            s += terms[i];
+        }
+        sums[count] = s;
+        sum = s;
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < count; i += ENERGY_THREADS) {
+        const double s = sums[i], v = terms[i], t = sums[i + 1];
+        terms[i] = fabs(s) >= fabs(v) ? (s - t) + v : (v - t) + s;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double c = comp;
+        uint32_t i = 0;
+        for (; i + U <= count; i += U) {
+            double v[U];
+#pragma unroll
+            for (uint32_t j = 0; j < U; ++j) v[j] = terms[i + j];
+#pragma unroll
+            for (uint32_t j = 0; j < U; ++j) c += v[j];
+        }
+        for (; i < count; ++i) c += terms[i];
+        comp = c;
+    }
 }
 
 template <typename T>
@@ -2777,62 +2822,69 @@ __global__ void __launch_bounds__(ENERGY_THREADS) k_potential_partials(Geom g, u
                                                                       double uniform_mass, const T* __restrict__ phi,
                                                                       double* __restrict__ partials,
                                                                       uint32_t* __restrict__ err) {
-    __shared__ double terms[ENERGY_BLOCK];
+    __shared__ double terms[ENERGY_CHUNK], sums[ENERGY_CHUNK + 1];
     const uint64_t b0 = (uint64_t)blockIdx.x * ENERGY_BLOCK;
     const uint64_t b1 = n < b0 + ENERGY_BLOCK ? n : b0 + ENERGY_BLOCK;
     const int N = g.N;
     const uint64_t NN = (uint64_t)N * (uint64_t)N;
     bool lost = false, bad = false;
-    for (uint64_t p = b0 + threadIdx.x; p < b1; p += ENERGY_THREADS) {
-        int ix, iy, iz;
-        double fx, fy, fz;
-        double weighted = 0.0;
-        if (!cic_axes(x[p], y[p], z[p], g, ix, iy, iz, fx, fy, fz)) {
-            bad = true;
-        } else {
-            const double m = masses ? masses[p] : uniform_mass;
-            const double wx[2] = {1.0 - fx, fx}, wy[2] = {1.0 - fy, fy}, wz[2] = {1.0 - fz, fz};
-            const uint64_t xs[2] = {(uint64_t)ix, (uint64_t)wrap_cell(ix + 1, N)};
-            const uint64_t ys[2] = {(uint64_t)iy, (uint64_t)wrap_cell(iy + 1, N)};
-            const uint64_t zs[2] = {(uint64_t)iz, (uint64_t)wrap_cell(iz + 1, N)};
-            double value = 0.0;
+    double sum = 0.0, comp = 0.0;
+    for (uint64_t c0 = b0; c0 < b1; c0 += ENERGY_CHUNK) {
+        const uint64_t c1 = b1 < c0 + ENERGY_CHUNK ? b1 : c0 + ENERGY_CHUNK;
+        __syncthreads();
+        for (uint64_t p = c0 + threadIdx.x; p < c1; p += ENERGY_THREADS) {
+            int ix, iy, iz;
+            double fx, fy, fz;
+            double weighted = 0.0;
+            if (!cic_axes(x[p], y[p], z[p], g, ix, iy, iz, fx, fy, fz)) {
+                bad = true;
+            } else {
+                const double m = masses ? masses[p] : uniform_mass;
+                const double wx[2] = {1.0 - fx, fx}, wy[2] = {1.0 - fy, fy}, wz[2] = {1.0 - fz, fz};
+                const uint64_t xs[2] = {(uint64_t)ix, (uint64_t)wrap_cell(ix + 1, N)};
+                const uint64_t ys[2] = {(uint64_t)iy, (uint64_t)wrap_cell(iy + 1, N)};
+                const uint64_t zs[2] = {(uint64_t)iz, (uint64_t)wrap_cell(iz + 1, N)};
+                double value = 0.0;
 #pragma unroll
-            for (int ox = 0; ox < 2; ++ox)
+                for (int ox = 0; ox < 2; ++ox)
 #pragma unroll
-                for (int oy = 0; oy < 2; ++oy)
+                    for (int oy = 0; oy < 2; ++oy)
 #pragma unroll
-                    for (int oz = 0; oz < 2; ++oz) {
-                        const double fv = (double)phi[xs[ox] * NN + ys[oy] * (uint64_t)N + zs[oz]];
-                        const double xy = wx[ox] * wy[oy];
-                        const double w = xy * wz[oz];
-                        if (wx[ox] != 0.0 && wy[oy] != 0.0 && wz[oz] != 0.0 && w == 0.0 && fv != 0.0 && m != 0.0)
-                            lost = true;
-                        const double c = fv * w;
-                        if (fv != 0.0 && w != 0.0 && c == 0.0 && m != 0.0) lost = true;
-                        value += c;
-                    }
-            weighted = m * value;
-            if (m != 0.0 && value != 0.0 && weighted == 0.0) lost = true;
+                        for (int oz = 0; oz < 2; ++oz) {
+                            const double fv = (double)phi[xs[ox] * NN + ys[oy] * (uint64_t)N + zs[oz]];
+                            const double xy = wx[ox] * wy[oy];
+                            const double w = xy * wz[oz];
+                            if (wx[ox] != 0.0 && wy[oy] != 0.0 && wz[oz] != 0.0 && w == 0.0 && fv != 0.0 && m != 0.0)
+                                lost = true;
+                            const double c = fv * w;
+                            if (fv != 0.0 && w != 0.0 && c == 0.0 && m != 0.0) lost = true;
+                            value += c;
+                        }
+                weighted = m * value;
+                if (m != 0.0 && value != 0.0 && weighted == 0.0) lost = true;
+            }
+            terms[p - c0] = weighted;
         }
-        terms[p - b0] = weighted;
+        neumaier_terms(terms, sums, (uint32_t)(c1 - c0), sum, comp);
     }
     if (bad) atomicOr(err, ERR_POSITION_NONFINITE);
     if (lost) atomicOr(err, ERR_INTERP_UNDERFLOW);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0, c = 0.0;
-        const uint32_t count = (uint32_t)(b1 - b0);
-        for (uint32_t i = 0; i < count; ++i) neumaier_add(terms[i], s, c);
-        partials[blockIdx.x] = s + c;
-    }
+    if (threadIdx.x == 0) partials[blockIdx.x] = sum + comp;
 }
 
-// 0.5 * (Neumaier sum of the workgroup partials, in order) -> out[0]
-__global__ void k_potential_total(const double* __restrict__ partials, uint64_t count, double* __restrict__ out,
-                                  uint32_t* __restrict__ err) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// 0.5 * (Neumaier sum of the workgroup partials, in order) -> out[0]; one workgroup
+__global__ void __launch_bounds__(ENERGY_THREADS) k_potential_total(const double* __restrict__ partials, uint64_t count,
+                                                                    double* __restrict__ out,
+                                                                    uint32_t* __restrict__ err) {
+    __shared__ double terms[ENERGY_CHUNK], sums[ENERGY_CHUNK + 1];
     double s = 0.0, c = 0.0;
-    for (uint64_t i = 0; i < count; ++i) neumaier_add(partials[i], s, c);
+    for (uint64_t c0 = 0; c0 < count; c0 += ENERGY_CHUNK) {
+        const uint32_t m = (uint32_t)(count - c0 < ENERGY_CHUNK ? count - c0 : ENERGY_CHUNK);
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < m; i += ENERGY_THREADS) terms[i] = partials[c0 + i];
+        neumaier_terms(terms, sums, m, s, c);
+    }
+    if (threadIdx.x != 0) return;
     const double total = s + c;
     const double half = 0.5 * total;
     if (!isfinite(total) || (total != 0.0 && half == 0.0)) atomicOr(err, ERR_INTERP_UNDERFLOW);
