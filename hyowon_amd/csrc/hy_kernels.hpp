@@ -2230,14 +2230,36 @@ __global__ void __launch_bounds__(256) k_input_mass(uint64_t n, const double* __
 // ===========================================================================
 // Block schedule for particle arrays stored in Lagrangian lattice order
 // p = (ix*S + iy)*S + iz (the order of lattice initial conditions, which
-// particles keep for the whole run).  Logical block L covers 256-particle
-// chunks of z-rows; consecutive L walk a TX x TY column of lattice rows
-// (all z) before the next column, so the blocks resident on one XCD touch a
-// compact region of the potential that stays in its L2.  S == 0: identity.
+// particles keep for the whole run).  Consecutive logical blocks walk a
+// TX x TY column of lattice rows (all z) before the next column, so the blocks
+// resident on one XCD touch a compact region of the potential that stays in
+// its L2.  S == 0: identity.  S a multiple of 256: a block is one 256-particle
+// chunk of a z-row (ZC of them per row, TX and TY divide S).  Otherwise (WC > 0) a
+// wave is one 64-particle chunk (WC per row, the last one short) and the
+// columns at the upper edges are narrower.
 struct LatticeTiling {
     uint32_t S, TX, TY, ZC;  // lattice side, column tile, 256-chunks per z-row
     int lS, lTX, lTY, lZC;   // log2 of each when all four are powers of two, else lS < 0
+    uint32_t WC;             // 64-chunks per z-row, or 0
 };
+
+// Particle of this thread (256-thread blocks) under the wave-chunk schedule;
+// past the row or the lattice: n.
+__device__ __forceinline__ uint64_t lattice_wave_particle(uint32_t block, const LatticeTiling& t, uint64_t n) {
+    const uint32_t unit = block * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (unit >= t.S * t.S * t.WC) return n;
+    const uint32_t strip = t.TX * t.S * t.WC;
+    const uint32_t tx = unit / strip, u = unit % strip;
+    const uint32_t wx = t.S - tx * t.TX < t.TX ? t.S - tx * t.TX : t.TX;
+    const uint32_t tile = wx * t.TY * t.WC;
+    const uint32_t ty = u / tile, w = u % tile;
+    const uint32_t wy = t.S - ty * t.TY < t.TY ? t.S - ty * t.TY : t.TY;
+    const uint32_t row = w / t.WC;
+    const uint32_t iz = (w - row * t.WC) * 64u + lane_id();
+    if (iz >= t.S) return n;
+    const uint32_t ix = tx * t.TX + row / wy, iy = ty * t.TY + row % wy;
+    return ((uint64_t)ix * t.S + iy) * t.S + iz;
+}
 
 __device__ __forceinline__ uint32_t lattice_block(uint32_t L, const LatticeTiling& t) {
     if (t.S == 0) return L;
@@ -2433,7 +2455,9 @@ template <typename T, typename PT, bool O32 = false, bool REC = false, bool OUT 
 __global__ void __launch_bounds__(256) k_gather_kdk(GatherArgs<T, PT> a) {
     // each XCD walks a contiguous particle range (spatially compact for
     // lattice-ordered particles), so potential lines are reused in its L2
-    const uint64_t p = (uint64_t)lattice_block(xcd_block(blockIdx.x, gridDim.x), a.lat) * blockDim.x + threadIdx.x;
+    const uint32_t bid = xcd_block(blockIdx.x, gridDim.x);
+    const uint64_t p = a.lat.WC ? lattice_wave_particle(bid, a.lat, a.n)
+                                : (uint64_t)lattice_block(bid, a.lat) * blockDim.x + threadIdx.x;
     const Geom& g = a.g;
     const int N = g.N;
     uint32_t fail = 0;

@@ -254,14 +254,14 @@ int hy_pm_set_tuning(hy_pm_ctx* ctx, const hy_fft_tuning* in);
 int hy_pm_autotune(hy_pm_ctx* ctx, uint32_t reps, hy_fft_tuning* out);
 
 /* Gather schedule.  The fused gather walks particle arrays held in Lagrangian
- * lattice order (n = S^3, S a multiple of 256) in column tiles of TX x TY
- * lattice rows, so the blocks resident on one XCD share that XCD's L2.
+ * lattice order (n = S^3, S a multiple of 256 or rows that fill at least 7/8 of
+ * their 64-particle chunks) in column tiles of TX x TY lattice rows, so the blocks resident on one XCD share that XCD's L2.
  * hy_pm_autotune_gather deposits and solves for the given positions (single
  * box, pure PM, uniform mass), times the gather under each candidate number
  * of rows per tile (0 = particle order, 16, 64, 256, 1024; ms_out[5] receives
  * the times, 0 where the lattice does not admit one) and keeps the fastest in
  * the context; hy_pm_set_gather_rows sets it (0, a power of two, or
- * HY_GATHER_ROWS_DEFAULT = 256 / (S / 256)).  Every schedule gives identical
+ * HY_GATHER_ROWS_DEFAULT = about 65536 / S).  Every schedule gives identical
  * results.  No reference counterpart (the reference gathers on CPU threads);
  * the FFT launch shapes are tuned by hy_pm_autotune, as FFTW_MEASURE plans do
  * for the reference (src/mesh/fft_backend.cpp:967-1003). */
