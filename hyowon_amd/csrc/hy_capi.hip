@@ -193,6 +193,7 @@ struct hy_pm_ctx {
         uint32_t total;
         double mass;
         double mass_in[2];  // sum and maximum of explicit masses
+        double energy;      // potential energy of the call
     };
     Status* hstatus = nullptr;
     Status* dstatus = nullptr;
@@ -330,6 +331,11 @@ void cap_scan(hy_pm_ctx* c, const uint32_t* cur, uint32_t* dense, uint32_t* capn
     s.capn = capn;
     s.block_sums = c->cap_block_sums;
     s.grand_total = c->grand_total;
+    if (c->nball <= hy::SMALL_SCAN_MAX) {
+        hipLaunchKernelGGL(hy::k_cap_small, dim3(1), dim3(hy::SMALL_SCAN_THREADS), 0, c->stream, s);
+        launch_check("k_cap_small");
+        return;
+    }
     const uint64_t nblk = blocks_for(c->nball, hy::SCAN_TILE);
     hipLaunchKernelGGL(hy::k_cap_reduce, dim3(nblk), dim3(hy::SCAN_THREADS), 0, c->stream, s);
     hipLaunchKernelGGL(hy::k_cap_blocks, dim3(1), dim3(hy::SCAN_THREADS), 0, c->stream, s, (uint32_t)nblk);
@@ -353,6 +359,14 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
     }
     if (mode == 0 && c->prec == HY_PREC_FP32_MIXED && c->rec_layout) {
         cap_scan(c, nullptr, offsets, capn);
+    } else if (nb <= hy::SMALL_SCAN_MAX) {
+        hy::CapScan s{};
+        s.counts = counts;
+        s.nb = nb;
+        s.dense = offsets;
+        s.grand_total = c->grand_total;
+        hipLaunchKernelGGL(hy::k_cap_small, dim3(1), dim3(hy::SMALL_SCAN_THREADS), 0, c->stream, s);
+        launch_check("k_cap_small");
     } else {
         const uint64_t nblk = blocks_for(nb, hy::SCAN_TILE);
         hipLaunchKernelGGL(hy::k_scan_reduce, dim3(nblk), dim3(hy::SCAN_THREADS), 0, c->stream, counts, nb,
@@ -808,6 +822,23 @@ void check_mass(hy_pm_ctx* c, double input, double deposited, uint64_t n) {
         fail(HY_ERUNTIME, "CIC deposited mass violates the forward-error bound");
 }
 
+// Deposit part of a call's status: its error bits, the routing identity, and the
+// mass identity of each box.  Raised before the bits of the later stages.
+void check_deposit(hy_pm_ctx* c, uint64_t n, const hy_pm_ctx::Status& st) {
+    raise_errors(st.err & (hy::ERR_POSITION_NONFINITE | hy::ERR_STALE_KEYS | hy::ERR_COORDINATE | hy::ERR_SCRATCH |
+                           hy::ERR_ROUTING | hy::ERR_MASS_CONSERVATION));
+    if (st.total != n) fail(HY_ELOGIC, "CIC bucket routing does not cover each particle exactly once");
+    c->last_deposited_mass = st.mass;
+    if (c->nbox == 1) {
+        check_mass(c, c->last_input_mass, st.mass, n);
+    } else {
+        hip_check(hipMemcpyAsync(c->hmass, c->mass_total, c->nbox * sizeof(double), hipMemcpyDeviceToHost, c->stream),
+                  "mass copy");
+        hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        for (uint32_t b = 0; b < c->nbox; ++b) check_mass(c, c->last_input_mass, c->hmass[b], n / c->nbox);
+    }
+}
+
 // Deposit stage: bucketize, deposit.
 // carried_rec (binary32, asynchronous): deposit the records the previous
 // fused step wrote into its capacity layout for these positions.  rec_out:
@@ -845,33 +876,7 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
     launch_deposit(c, plan.P, start, ovf);
     mark(c, HY_STAGE_DEPOSIT + 1);
     c->last_input_mass = Min;
-    if (!sync) return;
-    for (;;) {
-        const auto st = fetch_status(c);
-        if (carried && (st.err & hy::ERR_STALE_KEYS)) {
-            // the positions changed since the keys were made: route them afresh
-            // (coordinate errors of the stale routing are its artefacts)
-            raise_errors(st.err & hy::ERR_POSITION_NONFINITE);
-            carried = false;
-            reset_status(c);
-            bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, false, masses, nullptr, shift);
-            plan = plan_deposit(c, n, x, y, z, masses, uniform, Min, shift);
-            launch_deposit(c, plan.P);
-            continue;
-        }
-        raise_errors(st.err);
-        if (st.total != n) fail(HY_ELOGIC, "CIC bucket routing does not cover each particle exactly once");
-        c->last_deposited_mass = st.mass;
-        if (c->nbox == 1) {
-            check_mass(c, Min, st.mass, n);
-        } else {
-            hip_check(hipMemcpyAsync(c->hmass, c->mass_total, c->nbox * sizeof(double), hipMemcpyDeviceToHost,
-                                     c->stream), "mass copy");
-            hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-            for (uint32_t b = 0; b < c->nbox; ++b) check_mass(c, Min, c->hmass[b], n / c->nbox);
-        }
-        return;
-    }
+    if (sync) check_deposit(c, n, fetch_status(c));
 }
 
 // Device staging of host-pointer calls: positions and masses (4 * cap), accelerations (3 * cap).
@@ -1450,7 +1455,7 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
         hy::ForceRecord* slots = nullptr;
         static_assert(sizeof(hy::ForceRecord) == sizeof(hy::DepRecord), "force records behind the deposit records");
         if (c->rec_layout) slots = reinterpret_cast<hy::ForceRecord*>(c->rec + c->cap);
-        run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, true, false, false, false, 0.0, slots);
+        run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, false, false, false, false, 0.0, slots);
         const bool sg = c->method == HY_METHOD_TREEPM_LONG_RANGE;
         if (sg) run_fft_sg(c);
         else run_fft(c);
@@ -1484,15 +1489,10 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
         else gather(float{});
         mark(c, HY_STAGE_GATHER_KDK + 1);
         end_call(c);
-        const auto st = fetch_status(c);
-        raise_errors(st.err);
-        if (collect) {
-            hip_check(hipMemcpyAsync(&c->last_potential_energy, c->energy_partials + c->energy_cap, sizeof(double),
+        if (collect)
+            hip_check(hipMemcpyAsync(&c->hstatus->energy, c->energy_partials + c->energy_cap, sizeof(double),
                                      hipMemcpyDeviceToHost, c->stream), "energy copy");
-            hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-            c->energy_valid = true;
-        }
-        // commit: acc += g (only after every check passed)
+        // commit: acc += g, on the device only where every check passed
         double *cx = ax, *cy = ay, *cz = az;
         if (host) {
             cx = c->hacc; cy = c->hacc + c->cap; cz = c->hacc + 2 * c->cap;
@@ -1502,20 +1502,27 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
         }
         if (slots)
             hipLaunchKernelGGL(hy::k_commit_slots, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, c->keys,
-                               c->ranks, c->offsets, slots, cx, cy, cz);
+                               c->ranks, c->offsets, slots, cx, cy, cz, c->err);
         else if (c->prec == HY_PREC_FP64)
             hipLaunchKernelGGL(hy::k_commit_force<double>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n,
-                               (const double*)c->gx, (const double*)c->gy, (const double*)c->gz, cx, cy, cz);
+                               (const double*)c->gx, (const double*)c->gy, (const double*)c->gz, cx, cy, cz, c->err);
         else
             hipLaunchKernelGGL(hy::k_commit_force<float>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n,
-                               (const float*)c->gx, (const float*)c->gy, (const float*)c->gz, cx, cy, cz);
+                               (const float*)c->gx, (const float*)c->gy, (const float*)c->gz, cx, cy, cz, c->err);
         launch_check("k_commit_force");
+        const auto st = fetch_status(c);
+        check_deposit(c, n, st);
+        raise_errors(st.err);
+        if (collect) {
+            c->last_potential_energy = c->hstatus->energy;
+            c->energy_valid = true;
+        }
         if (host) {
             hip_check(hipMemcpyAsync(ax, cx, n * 8, hipMemcpyDeviceToHost, c->stream), "d2h");
             hip_check(hipMemcpyAsync(ay, cy, n * 8, hipMemcpyDeviceToHost, c->stream), "d2h");
             hip_check(hipMemcpyAsync(az, cz, n * 8, hipMemcpyDeviceToHost, c->stream), "d2h");
+            hip_check(hipStreamSynchronize(c->stream), "sync");
         }
-        hip_check(hipStreamSynchronize(c->stream), "sync");
     });
 }
 
@@ -1553,63 +1560,77 @@ int hy_pm_kdk(hy_pm_ctx* c, uint64_t n, const double* x_in, const double* y_in, 
         // binary32 uniform-mass asynchronous steps carry deposit records, others keys
         const bool rec_out = has_next && !sync && !masses && c->rec_layout;
         c->keys_ready = c->rec_ready = false;
-        run_deposit(c, n, x_in, y_in, z_in, masses, uniform, M, sync, carried, carried_rec, rec_out);
-        // counts are consumed by the scan above; the gather below accumulates the
-        // next step's counts into the zeroed buffer
-        const bool make_keys = has_next;
-        if (make_keys) fill_u32(c, c->counts, c->nball);
-        if (rec_out) fill_u32(c, c->ovf_count, 1);
-        run_fft(c);
-        auto fill = [&](auto& a) {
-            a.g = c->geom; a.n = n;
-            a.x_in = x_in; a.y_in = y_in; a.z_in = z_in;
-            a.x_out = x_out ? x_out : const_cast<double*>(x_in);
-            a.y_out = y_out ? y_out : const_cast<double*>(y_in);
-            a.z_out = z_out ? z_out : const_cast<double*>(z_in);
-            a.acc_x = acc_x; a.acc_y = acc_y; a.acc_z = acc_z;
-            a.k_prev = k_prev; a.k_next = k_next; a.d_next = d_next;
-            a.has_prev = has_prev; a.has_next = has_next;
-            a.err = c->err;
-            if (make_keys) {
-                a.next_counts = c->counts;
-                a.next_keys = c->keys;
-                a.next_ranks = c->ranks;
+        // A synchronous call looks at the status once, at its end: the gather does
+        // nothing where the deposit failed, so a failed call leaves the state
+        // as it was.  Carried keys of changed positions fail that way, and the
+        // positions are routed afresh.
+        for (bool routed = carried;; routed = false) {
+            run_deposit(c, n, x_in, y_in, z_in, masses, uniform, M, false, routed, carried_rec, rec_out);
+            // counts are consumed by the scan above; the gather below accumulates the
+            // next step's counts into the zeroed buffer
+            const bool make_keys = has_next;
+            if (make_keys) fill_u32(c, c->counts, c->nball);
+            if (rec_out) fill_u32(c, c->ovf_count, 1);
+            run_fft(c);
+            auto fill = [&](auto& a) {
+                a.g = c->geom; a.n = n;
+                a.x_in = x_in; a.y_in = y_in; a.z_in = z_in;
+                a.x_out = x_out ? x_out : const_cast<double*>(x_in);
+                a.y_out = y_out ? y_out : const_cast<double*>(y_in);
+                a.z_out = z_out ? z_out : const_cast<double*>(z_in);
+                a.acc_x = acc_x; a.acc_y = acc_y; a.acc_z = acc_z;
+                a.k_prev = k_prev; a.k_next = k_next; a.d_next = d_next;
+                a.has_prev = has_prev; a.has_next = has_next;
+                a.err = c->err;
+                a.gate = sync ? 1 : 0;
+                if (make_keys) {
+                    a.next_counts = c->counts;
+                    a.next_keys = c->keys;
+                    a.next_ranks = c->ranks;
+                }
+            };
+            if (c->prec == HY_PREC_FP64) {
+                hy::GatherArgs<double, double> a{};
+                fill(a);
+                a.phi = static_cast<const double*>(c->R);
+                a.px_in = (const double*)px_in; a.py_in = (const double*)py_in; a.pz_in = (const double*)pz_in;
+                a.px_out = (double*)px_out; a.py_out = (double*)py_out; a.pz_out = (double*)pz_out;
+                launch_gather(c, a);
+            } else {
+                hy::GatherArgs<float, float> a{};
+                fill(a);
+                if (rec_out) {
+                    a.rec_start = c->cap_next;
+                    a.rec_out = c->rec;
+                    a.ovf_count = c->ovf_count;
+                    a.ovf_rec = c->ovf_rec;
+                }
+                a.phi = static_cast<const float*>(c->R);
+                a.px_in = (const float*)px_in; a.py_in = (const float*)py_in; a.pz_in = (const float*)pz_in;
+                a.px_out = (float*)px_out; a.py_out = (float*)py_out; a.pz_out = (float*)pz_out;
+                launch_gather(c, a);
             }
-        };
-        if (c->prec == HY_PREC_FP64) {
-            hy::GatherArgs<double, double> a{};
-            fill(a);
-            a.phi = static_cast<const double*>(c->R);
-            a.px_in = (const double*)px_in; a.py_in = (const double*)py_in; a.pz_in = (const double*)pz_in;
-            a.px_out = (double*)px_out; a.py_out = (double*)py_out; a.pz_out = (double*)pz_out;
-            launch_gather(c, a);
-        } else {
-            hy::GatherArgs<float, float> a{};
-            fill(a);
-            if (rec_out) {
-                a.rec_start = c->cap_next;
-                a.rec_out = c->rec;
-                a.ovf_count = c->ovf_count;
-                a.ovf_rec = c->ovf_rec;
-            }
-            a.phi = static_cast<const float*>(c->R);
-            a.px_in = (const float*)px_in; a.py_in = (const float*)py_in; a.pz_in = (const float*)pz_in;
-            a.px_out = (float*)px_out; a.py_out = (float*)py_out; a.pz_out = (float*)pz_out;
-            launch_gather(c, a);
-        }
-        mark(c, HY_STAGE_GATHER_KDK + 1);
-        end_call(c);
-        if (sync) {
+            mark(c, HY_STAGE_GATHER_KDK + 1);
+            if (!sync) break;
             const auto st = fetch_status(c);
+            if (routed && (st.err & hy::ERR_STALE_KEYS)) {
+                // coordinate errors of the stale routing are its artefacts
+                raise_errors(st.err & hy::ERR_POSITION_NONFINITE);
+                reset_status(c);
+                continue;
+            }
+            check_deposit(c, n, st);
             raise_errors(st.err);
+            break;
         }
+        end_call(c);
         if (rec_out) {
             c->rec_ready = true;
             c->rec_x = x_out ? x_out : x_in;
             c->rec_y = y_out ? y_out : y_in;
             c->rec_z = z_out ? z_out : z_in;
             c->rec_n = n;
-        } else if (make_keys) {
+        } else if (has_next) {
             c->keys_ready = true;
             c->keys_x = x_out ? x_out : x_in;
             c->keys_y = y_out ? y_out : y_in;

@@ -442,13 +442,15 @@ class LeapfrogIntegrator:
         out = self._spare if self._spare is not None else state.empty_like()
         self.solver.kdk(state, out, self.uniform_mass, self._pending_k2, None, None,
                         masses=self.masses, acc=acc, reuse_keys=state is self._last_out)
+        if self._pending_k2 is None:
+            # a call without a kick writes no state; one with a kick writes the
+            # positions too, unchanged
+            out.x.copy_(state.x)
+            out.y.copy_(state.y)
+            out.z.copy_(state.z)
         self._pending_k2 = None
         self._spare = state
         self._last_out = None
-        # positions are unchanged by a pure kick; copy them across
-        out.x.copy_(state.x)
-        out.y.copy_(state.y)
-        out.z.copy_(state.z)
         return out
 
     def run(self, state: ParticleState, stepper: TimeStepper, acc=None) -> ParticleState:
