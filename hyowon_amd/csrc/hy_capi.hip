@@ -173,6 +173,7 @@ struct hy_pm_ctx {
     void* adj_phi = nullptr;                         // adjoint workspace (allocated on first use)
     void* adj_a[3] = {nullptr, nullptr, nullptr};
     double* adj_max = nullptr;
+    double* hadj_max = nullptr;                      // pinned copy of adj_max
     int method = HY_METHOD_PURE_PM;
     double split_scale = 0.0;
     void* B2 = nullptr;          // TreePM long range: x-derivative spectrum
@@ -219,6 +220,7 @@ struct hy_pm_ctx {
         for (void* p : allocations) (void)hipFree(p);
         if (hstatus) (void)hipHostFree(hstatus);
         if (hmass) (void)hipHostFree(hmass);
+        if (hadj_max) (void)hipHostFree(hadj_max);
         if (own_stream && stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -1848,33 +1850,61 @@ int hy_pm_autotune_gather(hy_pm_ctx* c, uint64_t n, const double* x, const doubl
 
 namespace {
 
+template <typename T>
+void launch_adj_gather(hy_pm_ctx* c, const hy::AdjGatherArgs<T>& a) {
+    const bool o32 = (uint64_t)c->N * c->N * c->N * sizeof(T) <= (1ull << 32);
+    auto kern = o32 ? hy::k_adj_gather<T, true> : hy::k_adj_gather<T, false>;
+    hipLaunchKernelGGL(kern, dim3(blocks_for(a.n, 256)), dim3(256), 0, c->stream, a);
+    launch_check("k_adj_gather");
+}
+
+constexpr uint32_t ABS_MAX_BLOCKS = 256;
+
 void ensure_adjoint_workspace(hy_pm_ctx* c) {
     if (c->adj_phi) return;
     const size_t bytes = (size_t)c->N * c->N * c->N * c->real_bytes;
     c->adj_phi = c->alloc(bytes);
     for (auto& a : c->adj_a) a = c->alloc(bytes);
-    c->adj_max = (double*)c->alloc(1024 * sizeof(double));
+    c->adj_max = (double*)c->alloc(3 * ABS_MAX_BLOCKS * sizeof(double));
+    hip_check(hipHostMalloc((void**)&c->hadj_max, 3 * ABS_MAX_BLOCKS * sizeof(double), hipHostMallocDefault),
+              "hipHostMalloc");
 }
 
-// max |q| over n values (synchronises).
-double abs_max(hy_pm_ctx* c, uint64_t n, const double* q) {
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(blocks_for(n, 256), 1), 1024);
-    hipLaunchKernelGGL(hy::k_absmax, dim3(blocks), dim3(256), 0, c->stream, n, q, c->adj_max);
+// Runs f with the context's real mesh (deposit target, transform input and
+// output) replaced by mesh: results land where they are needed, uncopied.
+template <typename F>
+void with_mesh(hy_pm_ctx* c, void* mesh, F&& f) {
+    struct Restore {
+        hy_pm_ctx* c;
+        void* saved;
+        ~Restore() { c->R = saved; }
+    } restore{c, c->R};
+    c->R = mesh;
+    f();
+}
+
+// Launches the max |q| of three value arrays; read_abs_max sums up its blocks
+// after the stream has been waited for.
+uint32_t launch_abs_max(hy_pm_ctx* c, uint64_t n, const double* const q[3]) {
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(blocks_for(n, 256), 1), ABS_MAX_BLOCKS);
+    hipLaunchKernelGGL(hy::k_absmax, dim3(blocks, 3), dim3(256), 0, c->stream, n, q[0], q[1], q[2], c->adj_max);
     launch_check("k_absmax");
-    std::vector<double> h(blocks);
-    hip_check(hipMemcpyAsync(h.data(), c->adj_max, blocks * sizeof(double), hipMemcpyDeviceToHost, c->stream),
+    hip_check(hipMemcpyAsync(c->hadj_max, c->adj_max, 3 * blocks * sizeof(double), hipMemcpyDeviceToHost, c->stream),
               "d2h");
-    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    return blocks;
+}
+
+double read_abs_max(const hy_pm_ctx* c, uint32_t blocks, int d) {
     double m = 0.0;
-    for (double v : h) m = std::max(m, v);
+    for (uint32_t i = 0; i < blocks; ++i) m = std::max(m, c->hadj_max[d * blocks + i]);
     return m;
 }
 
-// Raw CIC deposit of signed per-particle values q at positions whose buckets
-// (and, for binary64, particle order) the last run_deposit left in place.
+// Raw CIC deposit into c->R of signed per-particle values q (unit their largest
+// magnitude) at positions whose buckets (and, for binary64, particle order) the
+// last run_deposit left in place.
 void deposit_values(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const double* z,
-                    const double* q, double uniform, double Min) {
-    const double unit = abs_max(c, n, q);
+                    const double* q, double unit, double uniform, double Min) {
     if (unit == 0.0 || !std::isfinite(unit)) {
         if (!std::isfinite(unit)) fail(HY_EOVERFLOW, "adjoint values are not finite");
         fill_u32(c, c->R, (uint64_t)c->N * c->N * c->N * (c->real_bytes / 4));
@@ -1924,24 +1954,26 @@ int hy_pm_kdk_vjp(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, co
             return;
         }
         // forward potential at x
-        run_deposit(c, n, x, y, z, nullptr, uniform, M, true);
-        run_fft(c);
-        const size_t bytes = (size_t)c->N * c->N * c->N * c->real_bytes;
-        hip_check(hipMemcpyAsync(c->adj_phi, c->R, bytes, hipMemcpyDeviceToDevice, c->stream), "copy phi");
+        with_mesh(c, c->adj_phi, [&] {
+            run_deposit(c, n, x, y, z, nullptr, uniform, M, false);
+            run_fft(c);
+        });
         // A_a = deposit of u_a, then div A into R, then chi = G div A
-        const double* u[3] = {lpx, lpy, lpz};
-        for (int d = 0; d < 3; ++d) {
-            deposit_values(c, n, x, y, z, u[d], uniform, M);
-            hip_check(hipMemcpyAsync(c->adj_a[d], c->R, bytes, hipMemcpyDeviceToDevice, c->stream), "copy A");
-        }
+        const double* const u[3] = {lpx, lpy, lpz};
+        const uint32_t blocks = launch_abs_max(c, n, u);
+        const auto dep = fetch_status(c);
+        check_deposit(c, n, dep);
+        raise_errors(dep.err);
+        for (int d = 0; d < 3; ++d)
+            with_mesh(c, c->adj_a[d], [&] { deposit_values(c, n, x, y, z, u[d], read_abs_max(c, blocks, d), uniform, M); });
         const uint64_t cells = (uint64_t)c->N * c->N * c->N;
         const double inv_2dx = 1.0 / (2.0 * c->geom.dx);
         if (c->prec == HY_PREC_FP64)
-            hipLaunchKernelGGL(hy::k_div_stencil<double>, dim3(blocks_for(cells, 256)), dim3(256), 0, c->stream,
+            hipLaunchKernelGGL(hy::k_div_stencil<double>, dim3(blocks_for(cells / 4, 256)), dim3(256), 0, c->stream,
                                (const double*)c->adj_a[0], (const double*)c->adj_a[1], (const double*)c->adj_a[2],
                                (double*)c->R, c->N, inv_2dx);
         else
-            hipLaunchKernelGGL(hy::k_div_stencil<float>, dim3(blocks_for(cells, 256)), dim3(256), 0, c->stream,
+            hipLaunchKernelGGL(hy::k_div_stencil<float>, dim3(blocks_for(cells / 4, 256)), dim3(256), 0, c->stream,
                                (const float*)c->adj_a[0], (const float*)c->adj_a[1], (const float*)c->adj_a[2],
                                (float*)c->R, c->N, inv_2dx);
         launch_check("k_div_stencil");
@@ -1958,8 +1990,7 @@ int hy_pm_kdk_vjp(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, co
             a.coef_b = ksum * uniform / dx3;
             a.lx = lx; a.ly = ly; a.lz = lz;
             a.err = c->err;
-            hipLaunchKernelGGL(hy::k_adj_gather<T>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, a);
-            launch_check("k_adj_gather");
+            launch_adj_gather(c, a);
         };
         if (c->prec == HY_PREC_FP64) gather(double{});
         else gather(float{});
@@ -1986,8 +2017,7 @@ int hy_pm_density_vjp(hy_pm_ctx* c, uint64_t n, const double* x, const double* y
             a.coef_b = coef * uniform;
             a.lx = lx; a.ly = ly; a.lz = lz;
             a.err = c->err;
-            hipLaunchKernelGGL(hy::k_adj_gather<T>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, a);
-            launch_check("k_adj_gather");
+            launch_adj_gather(c, a);
         };
         if (c->prec == HY_PREC_FP64) gather(double{});
         else gather(float{});

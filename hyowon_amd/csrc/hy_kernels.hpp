@@ -2374,16 +2374,12 @@ struct GatherArgs {
     int gate;                   // do nothing where err is already set
 };
 
-// Centred-gradient force at one particle: base cell (ix, iy, iz), corner weights
-// w[0] = 1 - f, w[1] = f per axis, phi its box's potential.  O32: the box's
-// mesh spans at most 2^32 bytes, so the stencil uses 32-bit byte offsets from
-// phi (a scalar base where phi is wave-uniform).  Returns whether a non-zero
-// product was lost.
+// Potential values of the 8 corners' centred differences around base cell
+// (ix, iy, iz).  O32: the box's mesh spans at most 2^32 bytes, so the stencil uses
+// 32-bit byte offsets from phi (a scalar base where phi is wave-uniform).
 template <typename T, bool O32>
-__device__ __forceinline__ bool stencil_force(const T* phi, const Geom& g, int ix, int iy, int iz,
-                                              const T (&wx)[2], const T (&wy)[2], const T (&wz)[2], T& gx, T& gy,
-                                              T& gz) {
-    const int N = g.N;
+__device__ __forceinline__ void load_stencil(const T* phi, int N, int ix, int iy, int iz, T (&X)[4][2][2],
+                                             T (&Y)[2][2][2], T (&Z)[2][2][2]) {
     // The 8 corners' centred differences touch 32 distinct potential
     // values: the x stencil X[k][b][c] at (ix-1+k, iy+b, iz+c), and the
     // y / z stencil ends Y[j][a][c] at (ix+a, iy-1 / iy+2, iz+c) and
@@ -2403,7 +2399,6 @@ __device__ __forceinline__ bool stencil_force(const T* phi, const Geom& g, int i
         yo[k] = (Off)wrap_cell(iy - 1 + k, N) * (Off)N * es;
         zo[k] = (Off)wrap_cell(iz - 1 + k, N) * es;
     }
-    T X[4][2][2], Y[2][2][2], Z[2][2][2];
     // The stencil as 12 z-contiguous runs: the (ix+a, iy+b) lines hold
     // iz-1..iz+2 (x and z stencils), the x-end and y-end lines
     // iz..iz+1.  A run that does not wrap in z is one vector load.
@@ -2445,6 +2440,17 @@ __device__ __forceinline__ bool stencil_force(const T* phi, const Geom& g, int i
     for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int u = 0; u < 2; ++u) run(xo[u + 1] + yo[j * 3], iz, Y[j][u], 2);
+}
+
+// Centred-gradient force at one particle: base cell (ix, iy, iz), corner weights
+// w[0] = 1 - f, w[1] = f per axis, phi its box's potential (load_stencil).
+// Returns whether a non-zero product was lost.
+template <typename T, bool O32>
+__device__ __forceinline__ bool stencil_force(const T* phi, const Geom& g, int ix, int iy, int iz,
+                                              const T (&wx)[2], const T (&wy)[2], const T (&wz)[2], T& gx, T& gy,
+                                              T& gz) {
+    T X[4][2][2], Y[2][2][2], Z[2][2][2];
+    load_stencil<T, O32>(phi, g.N, ix, iy, iz, X, Y, Z);
     // -(f+ - f-) / (2 dx); when dx is a power of two the quotient equals
     // the product with the exact reciprocal bit for bit
     const T two_dx = (T)(2.0 * g.dx);
@@ -2661,14 +2667,9 @@ __global__ void __launch_bounds__(256) k_gather_kdk(GatherArgs<T, PT> a) {
     }
 }
 
-// CIC interpolation of mesh f at base cell (ix, iy, iz), corner weights w[0] =
-// 1 - f, w[1] = f per axis (src/mesh/mass_assignment_gather.inc:95-181,
-// 402-451): the sum over the x, y, z corner offsets, in that order, of
-// f * ((wx * wy) * wz).  lost is set where a product of non-zero factors
-// rounds to zero.  O32: 32-bit byte offsets from f.
+// The 8 mesh values around base cell (ix, iy, iz).  O32: 32-bit byte offsets from f.
 template <typename T, bool O32>
-__device__ __forceinline__ T interp_mesh(const T* f, int N, int ix, int iy, int iz, const T (&wx)[2],
-                                         const T (&wy)[2], const T (&wz)[2], bool& lost) {
+__device__ __forceinline__ void load_cube(const T* f, int N, int ix, int iy, int iz, T (&F)[2][2][2]) {
     using Off = typename std::conditional<O32, uint32_t, uint64_t>::type;
     const Off es = O32 ? (Off)sizeof(T) : (Off)1;
     const Off NN = (Off)N * (Off)N;
@@ -2680,7 +2681,6 @@ __device__ __forceinline__ T interp_mesh(const T* f, int N, int ix, int iy, int 
     auto at = [&](Off o) -> const char* {
         return O32 ? reinterpret_cast<const char*>(f) + o : reinterpret_cast<const char*>(f + o);
     };
-    T F[2][2][2];
 #pragma unroll
     for (int ox = 0; ox < 2; ++ox)
 #pragma unroll
@@ -2695,6 +2695,18 @@ __device__ __forceinline__ T interp_mesh(const T* f, int N, int ix, int iy, int 
                 F[ox][oy][1] = *reinterpret_cast<const T*>(at(o + z1));
             }
         }
+}
+
+// CIC interpolation of mesh f at base cell (ix, iy, iz), corner weights w[0] =
+// 1 - f, w[1] = f per axis (src/mesh/mass_assignment_gather.inc:95-181,
+// 402-451): the sum over the x, y, z corner offsets, in that order, of
+// f * ((wx * wy) * wz).  lost is set where a product of non-zero factors
+// rounds to zero.
+template <typename T, bool O32>
+__device__ __forceinline__ T interp_mesh(const T* f, int N, int ix, int iy, int iz, const T (&wx)[2],
+                                         const T (&wy)[2], const T (&wz)[2], bool& lost) {
+    T F[2][2][2];
+    load_cube<T, O32>(f, N, ix, iy, iz, F);
     T v = (T)0;
 #pragma unroll
     for (int ox = 0; ox < 2; ++ox)
@@ -3059,7 +3071,9 @@ __global__ void k_adj_kick(uint64_t n, const double* __restrict__ lx, const doub
 }
 
 // max |q| over particles (per block, then over blocks): the signed deposit unit.
-__global__ void k_absmax(uint64_t n, const double* __restrict__ q, double* __restrict__ out) {
+__global__ void k_absmax(uint64_t n, const double* __restrict__ qx, const double* __restrict__ qy,
+                         const double* __restrict__ qz, double* __restrict__ out) {
+    const double* q = blockIdx.y == 0 ? qx : (blockIdx.y == 1 ? qy : qz);
     __shared__ double sh[256];
     double m = 0.0;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
@@ -3072,7 +3086,7 @@ __global__ void k_absmax(uint64_t n, const double* __restrict__ q, double* __res
         if ((int)threadIdx.x < k) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + k]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
+    if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = sh[0];
 }
 
 // Per-particle values q, scaled by inv_unit, into bucket order for the
@@ -3091,21 +3105,30 @@ __global__ void k_scatter_values(uint64_t n, const double* __restrict__ q, doubl
 
 // out = sum_a D_a A_a (periodic centred differences), one box.
 template <typename T>
-__global__ void k_div_stencil(const T* __restrict__ ax, const T* __restrict__ ay, const T* __restrict__ az,
-                              T* __restrict__ out, int N, double inv_2dx) {
+__global__ void __launch_bounds__(256) k_div_stencil(const T* __restrict__ ax, const T* __restrict__ ay,
+                                                     const T* __restrict__ az, T* __restrict__ out, int N,
+                                                     double inv_2dx) {
+    // four z-adjacent cells per thread (N is a multiple of 4)
+    typedef T V4 __attribute__((ext_vector_type(4)));
     const uint64_t NN = (uint64_t)N * N;
-    const uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t c = 4 * ((uint64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x);
     if (c >= NN * N) return;
     const int iz = (int)(c % N), iy = (int)((c / N) % N), ix = (int)(c / NN);
-    const uint64_t xp = (uint64_t)wrap_cell(ix + 1, N) * NN + (uint64_t)iy * N + iz;
-    const uint64_t xm = (uint64_t)wrap_cell(ix - 1, N) * NN + (uint64_t)iy * N + iz;
-    const uint64_t yp = (uint64_t)ix * NN + (uint64_t)wrap_cell(iy + 1, N) * N + iz;
-    const uint64_t ym = (uint64_t)ix * NN + (uint64_t)wrap_cell(iy - 1, N) * N + iz;
-    const uint64_t zp = (uint64_t)ix * NN + (uint64_t)iy * N + wrap_cell(iz + 1, N);
-    const uint64_t zm = (uint64_t)ix * NN + (uint64_t)iy * N + wrap_cell(iz - 1, N);
-    const double d = ((double)ax[xp] - (double)ax[xm]) + ((double)ay[yp] - (double)ay[ym]) +
-                     ((double)az[zp] - (double)az[zm]);
-    out[c] = (T)(d * inv_2dx);
+    auto at = [&](const T* f, int i, int j) {
+        return *reinterpret_cast<const V4*>(f + (uint64_t)wrap_cell(i, N) * NN + (uint64_t)wrap_cell(j, N) * N + iz);
+    };
+    const V4 xp = at(ax, ix + 1, iy), xm = at(ax, ix - 1, iy), yp = at(ay, ix, iy + 1), ym = at(ay, ix, iy - 1);
+    const V4 zc = at(az, ix, iy);
+    const T* zrow = az + (uint64_t)ix * NN + (uint64_t)iy * N;
+    const T z[6] = {zrow[wrap_cell(iz - 1, N)], zc.x, zc.y, zc.z, zc.w, zrow[wrap_cell(iz + 4, N)]};
+    V4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const double d = ((double)xp[j] - (double)xm[j]) + ((double)yp[j] - (double)ym[j]) +
+                         ((double)z[j + 2] - (double)z[j]);
+        o[j] = (T)(d * inv_2dx);
+    }
+    *reinterpret_cast<V4*>(out + c) = o;
 }
 
 template <typename T>
@@ -3128,10 +3151,13 @@ struct AdjGatherArgs {
     uint32_t* err;
 };
 
-template <typename T>
+// The potential and chi are read as z-contiguous vector runs, the 32 distinct
+// potential values once each (128^3 particles on 256^3, binary32: 196 us with
+// eight scalar 7-point stencils, 116 so).  Does nothing where err is set.
+template <typename T, bool O32>
 __global__ void __launch_bounds__(256) k_adj_gather(AdjGatherArgs<T> a) {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= a.n) return;
+    const uint64_t p = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (p >= a.n || *a.err) return;
     const Geom& g = a.g;
     const int N = g.N;
     int ix, iy, iz;
@@ -3143,35 +3169,37 @@ __global__ void __launch_bounds__(256) k_adj_gather(AdjGatherArgs<T> a) {
     const double inv_dx = 1.0 / g.dx;
     const double w[3][2] = {{1.0 - fx, fx}, {1.0 - fy, fy}, {1.0 - fz, fz}};
     const double dw[2] = {-inv_dx, inv_dx};
-    const uint64_t NN = (uint64_t)N * N;
-    const uint64_t boff = (uint64_t)box_of(p, g) * NN * N;
-    double ta[3] = {0.0, 0.0, 0.0}, tb[3] = {0.0, 0.0, 0.0};
     const bool with_a = a.ux != nullptr;
     const double u[3] = {with_a ? a.ux[p] : 0.0, with_a ? a.uy[p] : 0.0, with_a ? a.uz[p] : 0.0};
-    const double two_dx = 2.0 * g.dx;
+    T X[4][2][2], Y[2][2][2], Z[2][2][2], F[2][2][2];
+    load_cube<T, O32>(a.chi, N, ix, iy, iz, F);
+    if (with_a) load_stencil<T, O32>(a.phi, N, ix, iy, iz, X, Y, Z);
+    // -(f+ - f-) / (2 dx); with dx a power of two the product with the exact
+    // reciprocal has the quotient's bits
+    const double two_dx = 2.0 * g.dx, inv_two_dx = 0.5 * g.inv_dx;
+    const bool exact = g.inv_exact != 0;
+    auto grad = [&](T hi, T lo) {
+        const double d = (double)hi - (double)lo;
+        return exact ? -d * inv_two_dx : -d / two_dx;
+    };
+    double ta[3] = {0.0, 0.0, 0.0}, tb[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int ox = 0; ox < 2; ++ox) {
-        const int cx = wrap_cell(ix + ox, N);
 #pragma unroll
         for (int oy = 0; oy < 2; ++oy) {
-            const int cy = wrap_cell(iy + oy, N);
 #pragma unroll
             for (int oz = 0; oz < 2; ++oz) {
-                const int cz = wrap_cell(iz + oz, N);
-                const uint64_t c = boff + (uint64_t)cx * NN + (uint64_t)cy * N + cz;
                 // derivative of the corner weight along each axis
                 const double dwc[3] = {dw[ox] * w[1][oy] * w[2][oz], w[0][ox] * dw[oy] * w[2][oz],
                                        w[0][ox] * w[1][oy] * dw[oz]};
-                const double xv = (double)a.chi[c];
+                const double xv = (double)F[ox][oy][oz];
                 double s = 0.0;
                 if (with_a) {
-                    const T* phi = a.phi + boff;
-                    const double gx = -((double)phi[(uint64_t)wrap_cell(cx + 1, N) * NN + (uint64_t)cy * N + cz] -
-                                        (double)phi[(uint64_t)wrap_cell(cx - 1, N) * NN + (uint64_t)cy * N + cz]) / two_dx;
-                    const double gy = -((double)phi[(uint64_t)cx * NN + (uint64_t)wrap_cell(cy + 1, N) * N + cz] -
-                                        (double)phi[(uint64_t)cx * NN + (uint64_t)wrap_cell(cy - 1, N) * N + cz]) / two_dx;
-                    const double gz = -((double)phi[(uint64_t)cx * NN + (uint64_t)cy * N + wrap_cell(cz + 1, N)] -
-                                        (double)phi[(uint64_t)cx * NN + (uint64_t)cy * N + wrap_cell(cz - 1, N)]) / two_dx;
+                    const double gx = grad(X[ox + 2][oy][oz], X[ox][oy][oz]);
+                    const double gy = grad(oy == 0 ? X[ox + 1][1][oz] : Y[1][ox][oz],
+                                           oy == 0 ? Y[0][ox][oz] : X[ox + 1][0][oz]);
+                    const double gz = grad(oz == 0 ? X[ox + 1][oy][1] : Z[1][ox][oy],
+                                           oz == 0 ? Z[0][ox][oy] : X[ox + 1][oy][0]);
                     s = u[0] * gx + u[1] * gy + u[2] * gz;
                 }
 #pragma unroll
