@@ -775,14 +775,16 @@ void launch_gather(hy_pm_ctx* c, hy::GatherArgs<T, PT> a) {
     const uint64_t units = (uint64_t)a.lat.S * a.lat.S * a.lat.WC;
     const dim3 grid((uint32_t)(units ? blocks_for(units, 4) : blocks_for(a.n, 256))), block(256);
     const bool out = a.acc_x || a.g_x;
-    void (*kern)(hy::GatherArgs<T, PT>) =
-        out ? (o32 ? hy::k_gather_kdk<T, PT, true, false, true> : hy::k_gather_kdk<T, PT, false, false, true>)
-            : (o32 ? hy::k_gather_kdk<T, PT, true, false, false> : hy::k_gather_kdk<T, PT, false, false, false>);
+    auto pick = [&](auto rec, auto chunk) {
+        constexpr bool R = decltype(rec)::value, K = decltype(chunk)::value;
+        return out ? (o32 ? hy::k_gather_kdk<T, PT, true, R, true, K> : hy::k_gather_kdk<T, PT, false, R, true, K>)
+                   : (o32 ? hy::k_gather_kdk<T, PT, true, R, false, K> : hy::k_gather_kdk<T, PT, false, R, false, K>);
+    };
+    void (*kern)(hy::GatherArgs<T, PT>) = units ? pick(std::false_type{}, std::true_type{})
+                                                : pick(std::false_type{}, std::false_type{});
     if constexpr (std::is_same_v<T, float>) {
         if (a.rec_out)
-            kern = out ? (o32 ? hy::k_gather_kdk<T, PT, true, true, true> : hy::k_gather_kdk<T, PT, false, true, true>)
-                       : (o32 ? hy::k_gather_kdk<T, PT, true, true, false>
-                              : hy::k_gather_kdk<T, PT, false, true, false>);
+            kern = units ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{});
     }
     hipLaunchKernelGGL(kern, grid, block, 0, c->stream, a);
     launch_check("k_gather_kdk");
