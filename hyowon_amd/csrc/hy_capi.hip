@@ -695,22 +695,24 @@ void launch_interp(hy_pm_ctx* c, hy::InterpArgs<T> a) {
 }
 
 // Force of the n particles just deposited, in record order, over their force
-// records (binary32): the gradient of the potentials in R, or the force meshes
-// R, R2, R3 of the TreePM long range.
+// records (binary64: over the records' fractions): the gradient of the
+// potentials in R, or the force meshes R, R2, R3 of the TreePM long range.
+template <typename T>
 void launch_slot_force(hy_pm_ctx* c, uint64_t n, hy::ForceRecord* force) {
-    hy::SlotForceArgs a{};
+    hy::SlotForceArgs<T> a{};
     a.g = c->geom;
     a.n = n;
     a.rec = c->rec;
     a.force = force;
-    a.f[0] = static_cast<const float*>(c->R);
-    a.f[1] = static_cast<const float*>(c->R2);
-    a.f[2] = static_cast<const float*>(c->R3);
+    a.rec64 = c->rec64;
+    a.f[0] = static_cast<const T*>(c->R);
+    a.f[1] = static_cast<const T*>(c->R2);
+    a.f[2] = static_cast<const T*>(c->R3);
     a.err = c->err;
-    const bool o32 = c->nbox == 1 && (uint64_t)c->N * c->N * c->N * sizeof(float) <= (1ull << 32);
+    const bool o32 = c->nbox == 1 && (uint64_t)c->N * c->N * c->N * sizeof(T) <= (1ull << 32);
     const bool sg = c->method == HY_METHOD_TREEPM_LONG_RANGE;
-    auto kern = sg ? (o32 ? hy::k_slot_force<true, true> : hy::k_slot_force<true, false>)
-                   : (o32 ? hy::k_slot_force<false, true> : hy::k_slot_force<false, false>);
+    auto kern = sg ? (o32 ? hy::k_slot_force<T, true, true> : hy::k_slot_force<T, true, false>)
+                   : (o32 ? hy::k_slot_force<T, false, true> : hy::k_slot_force<T, false, false>);
     hipLaunchKernelGGL(kern, dim3((uint32_t)blocks_for(n, 256)), dim3(256), 0, c->stream, a);
     launch_check("k_slot_force");
 }
@@ -1452,10 +1454,9 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             dx_ = s; dy_ = s + c->cap; dz_ = s + 2 * c->cap;
         }
         reset_status(c);
-        // Binary32: the forces are gathered in record order, the force records
-        // behind the n records of the call (room for two per particle exists
-        // where the carried layout does).  Binary64 records hold the fractions
-        // of the deposit only, and gather in particle order.
+        // The forces are gathered in record order.  Binary32: the force records
+        // lie behind the n records of the call (room for two per particle exists
+        // where the carried layout does; else in particle order).
         hy::ForceRecord* slots = nullptr;
         static_assert(sizeof(hy::ForceRecord) == sizeof(hy::DepRecord), "force records behind the deposit records");
         if (c->rec_layout) slots = reinterpret_cast<hy::ForceRecord*>(c->rec + c->cap);
@@ -1464,33 +1465,31 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
         if (sg) run_fft_sg(c);
         else run_fft(c);
         if (collect) launch_potential_energy(c, n, dx_, dy_, dz_, dm, uniform);
-        auto gather = [&](auto tag) {
-            using T = decltype(tag);
-            if (sg) {
-                hy::InterpArgs<T> a{};
-                a.n = n;
-                a.x = dx_; a.y = dy_; a.z = dz_;
-                a.f[0] = static_cast<const T*>(c->R);
-                a.f[1] = static_cast<const T*>(c->R2);
-                a.f[2] = static_cast<const T*>(c->R3);
-                a.out[0] = static_cast<T*>(c->gx);
-                a.out[1] = static_cast<T*>(c->gy);
-                a.out[2] = static_cast<T*>(c->gz);
-                a.meshes = 3;
-                launch_interp(c, a);
-            } else {
-                hy::GatherArgs<T, T> a{};
-                a.g = c->geom; a.n = n;
-                a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
-                a.err = c->err;
-                a.phi = static_cast<const T*>(c->R);
-                a.g_x = (T*)c->gx; a.g_y = (T*)c->gy; a.g_z = (T*)c->gz;
-                launch_gather(c, a);
-            }
-        };
-        if (slots) launch_slot_force(c, n, slots);
-        else if (c->prec == HY_PREC_FP64) gather(double{});
-        else gather(float{});
+        if (c->prec == HY_PREC_FP64) {
+            launch_slot_force<double>(c, n, nullptr);
+        } else if (slots) {
+            launch_slot_force<float>(c, n, slots);
+        } else if (sg) {
+            hy::InterpArgs<float> a{};
+            a.n = n;
+            a.x = dx_; a.y = dy_; a.z = dz_;
+            a.f[0] = static_cast<const float*>(c->R);
+            a.f[1] = static_cast<const float*>(c->R2);
+            a.f[2] = static_cast<const float*>(c->R3);
+            a.out[0] = static_cast<float*>(c->gx);
+            a.out[1] = static_cast<float*>(c->gy);
+            a.out[2] = static_cast<float*>(c->gz);
+            a.meshes = 3;
+            launch_interp(c, a);
+        } else {
+            hy::GatherArgs<float, float> a{};
+            a.g = c->geom; a.n = n;
+            a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
+            a.err = c->err;
+            a.phi = static_cast<const float*>(c->R);
+            a.g_x = (float*)c->gx; a.g_y = (float*)c->gy; a.g_z = (float*)c->gz;
+            launch_gather(c, a);
+        }
         mark(c, HY_STAGE_GATHER_KDK + 1);
         end_call(c);
         if (collect)
@@ -1504,15 +1503,16 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             hip_check(hipMemcpyAsync(cy, ay, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             hip_check(hipMemcpyAsync(cz, az, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
         }
-        if (slots)
-            hipLaunchKernelGGL(hy::k_commit_slots, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, c->keys,
-                               c->ranks, c->offsets, slots, cx, cy, cz, c->err);
-        else if (c->prec == HY_PREC_FP64)
-            hipLaunchKernelGGL(hy::k_commit_force<double>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n,
-                               (const double*)c->gx, (const double*)c->gy, (const double*)c->gz, cx, cy, cz, c->err);
+        const dim3 grid(blocks_for(n, 256)), block(256);
+        if (c->prec == HY_PREC_FP64)
+            hipLaunchKernelGGL(hy::k_commit_slots<hy::DepRecord64>, grid, block, 0, c->stream, n, c->keys, c->ranks,
+                               c->offsets, c->rec64, cx, cy, cz, c->err);
+        else if (slots)
+            hipLaunchKernelGGL(hy::k_commit_slots<hy::ForceRecord>, grid, block, 0, c->stream, n, c->keys, c->ranks,
+                               c->offsets, slots, cx, cy, cz, c->err);
         else
-            hipLaunchKernelGGL(hy::k_commit_force<float>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n,
-                               (const float*)c->gx, (const float*)c->gy, (const float*)c->gz, cx, cy, cz, c->err);
+            hipLaunchKernelGGL(hy::k_commit_force, grid, block, 0, c->stream, n, (const float*)c->gx,
+                               (const float*)c->gy, (const float*)c->gz, cx, cy, cz, c->err);
         launch_check("k_commit_force");
         const auto st = fetch_status(c);
         check_deposit(c, n, st);

@@ -309,7 +309,8 @@ __global__ void k_cap_apply(CapScan s) {
 
 // The whole scan in one workgroup, for up to SMALL_SCAN_MAX buckets (a 192^3 mesh
 // has 13824): one launch and no round trip through block_sums; 16 -> 6 us for
-// the 4096 buckets of a 128^3 mesh.  Each thread owns a run of buckets.
+// the 4096 buckets of a 128^3 mesh, even (15 us) at 13824, where it still saves
+// two launches.  Each thread owns a run of buckets.
 constexpr int SMALL_SCAN_THREADS = 1024;
 constexpr uint64_t SMALL_SCAN_MAX = 16 * SMALL_SCAN_THREADS;
 
@@ -401,9 +402,12 @@ __global__ void k_scatter_checked(uint64_t n, const double* __restrict__ x, cons
     order[offsets[k] + ranks[p]] = (uint32_t)p;
 }
 
-// Binary64 deposit record: tile-local base cell, the particle index (the
-// reference's per-cell summation order is by index) and the binary64
-// fractions.
+// Binary64 deposit record: tile-local base cell (12 bits) and above it the tile
+// in its box, the particle index (the reference's per-cell summation order is
+// by index) and the binary64 fractions; after the slot-order force kernel, the
+// force instead of the fractions.
+constexpr int REC_CELL_BITS = 12;  // tile edges up to 16; tiles of a 1024^3 box: 18 bits
+
 struct DepRecord64 {
     uint32_t cell;
     uint32_t index;
@@ -454,6 +458,7 @@ __global__ void k_scatter_records(uint64_t n, const double* __restrict__ x, cons
     R r;
     r.cell = record_cell(bx, by, bz, g);
     if constexpr (sizeof(R) == sizeof(DepRecord64)) {
+        r.cell |= (k % buckets_per_box(g)) >> 3 << REC_CELL_BITS;
         r.index = (uint32_t)p;
         r.fx = fx;
         r.fy = fy;
@@ -1225,7 +1230,7 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
     // bucket says (ERR_COORDINATE; also a slot a failed scatter left unwritten).
     constexpr uint32_t DEP_NOWHERE = 0x7fff;
     auto base_cell = [&](const DepRecord64& rec, int d) -> uint32_t {
-        const uint32_t c = rec.cell;
+        const uint32_t c = rec.cell & ((1u << REC_CELL_BITS) - 1u);
         const int cz = (int)(c % (uint32_t)TT), cy = (int)((c / (uint32_t)TT) % (uint32_t)TT),
                   cx = (int)(c / (uint32_t)(TT * TT));
         if (cx >= TT || ((d & 4) && cx != TT - 1) || ((d & 2) && cy != TT - 1) || ((d & 1) && cz != TT - 1) ||
@@ -2774,71 +2779,105 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<T> a) {
     if (bad) atomicOr(a.err, ERR_FORCE_NONFINITE);
 }
 
-// Binary32 force of the particles in deposit-record order (slot s of the
-// bucket layout), the result over the slot's force record.  Consecutive slots
+// Force of the particles in deposit-record order (slot s of the bucket layout),
+// the result over the slot's force record (binary64: over the fractions).  Consecutive slots
 // share a 16^3 tile, so the stencil lines stay in L1 and L2 whatever the order
 // of the particle arrays; in particle order a shuffled set fetches 12 to 16
 // lines per particle from beyond L2 (20M shuffled particles on 512^3: 4.43 ms
 // in particle order, 0.78 here, with 0.28 more in the scatter and 0.33 more in
-// the commit).  On lattice order it is even: TreePM, 16.8M on 512^3, 1.23 ->
+// the commit; binary64, 3M on 192^3: 0.51 ->
+// 0.12, with 0.03 more in the commit).  On lattice order it is even: TreePM, 16.8M on 512^3, 1.23 ->
 // 0.90, with 0.14 + 0.06 more around it.  FORCE_SG false: centred gradient of
 // f[0] (one potential per box); true: interpolation of the force meshes f[0..2].
+template <typename T>
 struct SlotForceArgs {
     Geom g;
     uint64_t n;
-    const DepRecord* rec;
+    const DepRecord* rec;  // binary32
     ForceRecord* force;
-    const float* f[3];
+    DepRecord64* rec64;    // binary64
+    const T* f[3];
     uint32_t* err;
 };
 
-template <bool FORCE_SG, bool O32>
-__global__ void __launch_bounds__(256) k_slot_force(SlotForceArgs a) {
+template <typename T, bool FORCE_SG, bool O32>
+__global__ void __launch_bounds__(256) k_slot_force(SlotForceArgs<T> a) {
     const uint64_t s = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     // a failed deposit (a particle without a slot) leaves records unwritten
     if (s >= a.n || *a.err) return;
     const Geom& g = a.g;
-    const int T = g.T;
-    const DepRecord r = a.rec[s];
-    ForceRecord q = a.force[s];
+    const int E = g.T;
     const uint32_t nT = (uint32_t)g.nT, ntiles = nT * nT * nT;
-    const uint32_t box = O32 ? 0u : q.tile / ntiles;  // O32: one box
-    const uint32_t tile = O32 ? q.tile : q.tile % ntiles;
-    const int cz = T == 16 ? (int)(r.cell & 15u) : (int)r.cell % T;
-    const int cxy = T == 16 ? (int)(r.cell >> 4) : (int)r.cell / T;
-    const int cy = T == 16 ? cxy & 15 : cxy % T, cx = T == 16 ? cxy >> 4 : cxy / T;
-    const int ix = (int)(tile / (nT * nT)) * T + cx, iy = (int)(tile / nT % nT) * T + cy, iz = (int)(tile % nT) * T + cz;
-    const float wx[2] = {q.wx, r.fx}, wy[2] = {q.wy, r.fy}, wz[2] = {q.wz, r.fz};
-    float v[3];
+    uint32_t cell, tile, box;  // O32: one box
+    T wx[2], wy[2], wz[2];
+    if constexpr (sizeof(T) == 4) {
+        const DepRecord r = a.rec[s];
+        const ForceRecord q = a.force[s];
+        cell = r.cell;
+        box = O32 ? 0u : q.tile / ntiles;
+        tile = O32 ? q.tile : q.tile % ntiles;
+        wx[0] = q.wx; wx[1] = r.fx;
+        wy[0] = q.wy; wy[1] = r.fy;
+        wz[0] = q.wz; wz[1] = r.fz;
+    } else {
+        const DepRecord64 r = a.rec64[s];
+        cell = r.cell & ((1u << REC_CELL_BITS) - 1u);
+        tile = r.cell >> REC_CELL_BITS;
+        box = O32 ? 0u : box_of(r.index, g);
+        wx[0] = 1.0 - r.fx; wx[1] = r.fx;
+        wy[0] = 1.0 - r.fy; wy[1] = r.fy;
+        wz[0] = 1.0 - r.fz; wz[1] = r.fz;
+    }
+    const int cz = E == 16 ? (int)(cell & 15u) : (int)cell % E;
+    const int cxy = E == 16 ? (int)(cell >> 4) : (int)cell / E;
+    const int cy = E == 16 ? cxy & 15 : cxy % E, cx = E == 16 ? cxy >> 4 : cxy / E;
+    const int ix = (int)(tile / (nT * nT)) * E + cx, iy = (int)(tile / nT % nT) * E + cy, iz = (int)(tile % nT) * E + cz;
+    T v[3];
     bool lost = false;
     if constexpr (FORCE_SG) {
 #pragma unroll
-        for (int m = 0; m < 3; ++m) v[m] = interp_mesh<float, O32>(a.f[m], g.N, ix, iy, iz, wx, wy, wz, lost);
+        for (int m = 0; m < 3; ++m) v[m] = interp_mesh<T, O32>(a.f[m], g.N, ix, iy, iz, wx, wy, wz, lost);
     } else {
-        const float* phi = a.f[0] + (uint64_t)box * (uint64_t)g.N * (uint64_t)g.N * (uint64_t)g.N;
-        lost = stencil_force<float, O32>(phi, g, ix, iy, iz, wx, wy, wz, v[0], v[1], v[2]);
+        const T* phi = a.f[0] + (uint64_t)box * (uint64_t)g.N * (uint64_t)g.N * (uint64_t)g.N;
+        lost = stencil_force<T, O32>(phi, g, ix, iy, iz, wx, wy, wz, v[0], v[1], v[2]);
     }
     if (lost) atomicOr(a.err, FORCE_SG ? ERR_INTERP_UNDERFLOW : ERR_GATHER_UNDERFLOW);
     if (!isfinite(v[0]) || !isfinite(v[1]) || !isfinite(v[2])) atomicOr(a.err, ERR_FORCE_NONFINITE);
-    q.wx = v[0];
-    q.wy = v[1];
-    q.wz = v[2];
-    a.force[s] = q;
+    if constexpr (sizeof(T) == 4) {
+        a.force[s] = {v[0], v[1], v[2], 0u};
+    } else {
+        a.rec64[s].fx = v[0];
+        a.rec64[s].fy = v[1];
+        a.rec64[s].fz = v[2];
+    }
 }
 
 // acc += g for every particle, its force read from its slot, where no error is set.
+__device__ __forceinline__ void slot_value(const ForceRecord& q, double v[3]) {
+    v[0] = q.wx;
+    v[1] = q.wy;
+    v[2] = q.wz;
+}
+__device__ __forceinline__ void slot_value(const DepRecord64& q, double v[3]) {
+    v[0] = q.fx;
+    v[1] = q.fy;
+    v[2] = q.fz;
+}
+
+template <typename R>
 __global__ void __launch_bounds__(256) k_commit_slots(uint64_t n, const uint32_t* __restrict__ keys,
                                                       const uint32_t* __restrict__ ranks,
                                                       const uint32_t* __restrict__ offsets,
-                                                      const ForceRecord* __restrict__ force, double* __restrict__ ax,
+                                                      const R* __restrict__ force, double* __restrict__ ax,
                                                       double* __restrict__ ay, double* __restrict__ az,
                                                       const uint32_t* __restrict__ err) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n || *err) return;
-    const ForceRecord q = force[offsets[keys[p]] + ranks[p]];
-    ax[p] += (double)q.wx;
-    ay[p] += (double)q.wy;
-    az[p] += (double)q.wz;
+    double v[3];
+    slot_value(force[offsets[keys[p]] + ranks[p]], v);
+    ax[p] += v[0];
+    ay[p] += v[1];
+    az[p] += v[2];
 }
 
 // Potential-energy diagnostic: sum_p m_p phi(x_p) with phi CIC-interpolated
@@ -3037,9 +3076,8 @@ __global__ void __launch_bounds__(256) k_lpt_update(const double* __restrict__ p
 
 // Transactional commit for the reference-shaped force entry: acc += g where no
 // error is set.
-template <typename T>
-__global__ void k_commit_force(uint64_t n, const T* __restrict__ gx, const T* __restrict__ gy,
-                               const T* __restrict__ gz, double* __restrict__ ax,
+__global__ void k_commit_force(uint64_t n, const float* __restrict__ gx, const float* __restrict__ gy,
+                               const float* __restrict__ gz, double* __restrict__ ax,
                                double* __restrict__ ay, double* __restrict__ az,
                                const uint32_t* __restrict__ err) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
