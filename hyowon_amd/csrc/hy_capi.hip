@@ -537,8 +537,9 @@ void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, const uint32_t* start 
     const uint64_t waves = c->ntiles * hy::SA_WAVES_PER_TILE;
     // 2048 records per workgroup: the workgroups of a box meet at its few digit
     // words and its ticket, so fewer are faster (64 boxes of 192^3, 54 -> 7
-    // workgroups each: 243 -> 89 us)
-    const dim3 rgrid((uint32_t)std::min<uint64_t>(64, blocks_for(waves, 2048)), c->nbox);
+    // workgroups each: 243 -> 89 us); up to 256, one per CU, where the records
+    // themselves (32 MB for 1024^3) take longer
+    const dim3 rgrid((uint32_t)std::min<uint64_t>(256, blocks_for(waves, 2048)), c->nbox);
     if (c->prec == HY_PREC_FP64)
         hipLaunchKernelGGL(hy::k_mass_finish, rgrid, dim3(256), 0, c->stream, c->mass_waves, waves, c->mass_digits,
                            c->tickets, c->mass_total, chk);

@@ -1,7 +1,7 @@
 // HIP kernels of the MI355X particle-mesh gravity step (gfx950, wave64).
 //
 // Stage map (reference hot path, file:line relative to the reference tree):
-//   k_bucket_key / k_scan_* / k_scatter  stable bucketing of particles that
+//   k_bucket_key / k_scan_*, k_cap_* / k_scatter  stable bucketing of particles that
 //        feeds the deterministic deposit (reference x-plane counting sort,
 //        src/mesh/mass_assignment_workspace.inc:264-374, generalised to
 //        tile buckets; determinism restored by k_deposit's index sort).
@@ -9,10 +9,10 @@
 //        to src/mesh/mass_assignment_deposit.inc:193-240 (bin X with weight
 //        1-f, then bin X-1 with weight f, particles in index order, oy outer,
 //        oz inner), density contrast as src/gravity/pm_solver.cpp:700-759.
-//   k_fft_*      (hy_fft_passes.hpp) r2c / Green / c2r Poisson solve (src/mesh/fft_backend.cpp,
+//   k_tl_*       (hy_fft_passes.hpp) r2c / Green / c2r Poisson solve (src/mesh/fft_backend.cpp,
 //        src/mesh/green_function.cpp:165-241).
-//   k_gather_kdk fused centered-gradient CIC gather
-//        (src/mesh/mass_assignment_gradient.cpp:117-206) with the K2 kick,
+//   k_gather_kdk, k_slot_force  centered-gradient CIC gather
+//        (src/mesh/mass_assignment_gradient.cpp:117-206); k_gather_kdk with the K2 kick,
 //        the next K1 kick and the periodic drift
 //        (include/cosmo_nbody/time/particle_update.hpp:20-116).
 #pragma once
