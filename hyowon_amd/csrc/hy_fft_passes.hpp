@@ -440,8 +440,12 @@ __device__ __forceinline__ void tl_x_green_body(FftArgs<T> a) {
     }
 }
 
+// The spectral-gradient pass with a length-24 level sits at 256 registers in
+// binary64: asked for two waves per SIMD it stays there (one wave: 384^3 force
+// meshes 2.95 -> 3.16 ms); lengths 16 and 32 are left to the compiler.
 template <typename T, int N, int V, int SG = 0>
-__global__ void __launch_bounds__((TLCfg<T, N, (N / 2 + 1) * N, V>::THREADS)) k_tl_x_green(FftArgs<T> a) {
+__global__ void __launch_bounds__((TLCfg<T, N, (N / 2 + 1) * N, V>::THREADS))
+__attribute__((amdgpu_waves_per_eu(SG == 1 && TwoLevel<N>::B == 24 ? 2 : 1))) k_tl_x_green(FftArgs<T> a) {
     tl_x_green_body<T, N, V, SG>(a);
 }
 
