@@ -156,6 +156,8 @@ struct hy_pm_ctx {
     uint64_t scratch_cap = 0;
     unsigned long long* scratch_cursor = nullptr;
     uint32_t* err = nullptr;
+    uint32_t* late = nullptr;      // error bits of the kernels that act only where err is clear: a word of
+                                   // its own, so that a failing particle stops none of the others
     void* gx = nullptr;
     void* gy = nullptr;
     void* gz = nullptr;
@@ -191,7 +193,8 @@ struct hy_pm_ctx {
     // pinned host mirror of the status words
     struct Status {
         uint32_t err;
-        uint32_t total;
+        uint32_t late;
+        uint64_t total;
         double mass;
         double mass_in[2];  // sum and maximum of explicit masses
         double energy;      // potential energy of the call
@@ -400,14 +403,16 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
     }
 }
 
-void reset_status(hy_pm_ctx* c) { fill_u32(c, c->err, 1); }
+void reset_status(hy_pm_ctx* c) { fill_u32(c, c->err, 2); }
 
-// Copy err / grand total / deposited mass to the host and synchronise.
+// Copy err / late / grand total / deposited mass to the host and synchronise;
+// err holds the bits of both words.
 hy_pm_ctx::Status fetch_status(hy_pm_ctx* c) {
-    // err, grand_total and the first box's mass are adjacent: one copy
+    // the words and the first box's mass are adjacent: one copy
     hip_check(hipMemcpyAsync(c->hstatus, c->err, offsetof(hy_pm_ctx::Status, mass_in), hipMemcpyDeviceToHost,
                              c->stream), "status");
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    c->hstatus->err |= c->hstatus->late;
     return *c->hstatus;
 }
 
@@ -709,7 +714,8 @@ void launch_slot_force(hy_pm_ctx* c, uint64_t n, hy::ForceRecord* force) {
     a.f[0] = static_cast<const T*>(c->R);
     a.f[1] = static_cast<const T*>(c->R2);
     a.f[2] = static_cast<const T*>(c->R3);
-    a.err = c->err;
+    a.gate = c->err;
+    a.err = c->late;
     const bool o32 = c->nbox == 1 && (uint64_t)c->N * c->N * c->N * sizeof(T) <= (1ull << 32);
     const bool sg = c->method == HY_METHOD_TREEPM_LONG_RANGE;
     auto kern = sg ? (o32 ? hy::k_slot_force<T, true, true> : hy::k_slot_force<T, true, false>)
@@ -1150,11 +1156,13 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         }
         const uint64_t wave_words = c->prec == HY_PREC_FP64 ? hy::SA_WAVE_WORDS : 2;  // window, or digit-sum pair
         c->mass_waves = (unsigned long long*)c->alloc(wave_words * hy::SA_WAVES_PER_TILE * c->ntiles * c->nbox * 8);
-        // status words as Status mirrors them: err, grand_total, then the masses
-        const size_t status_bytes = 8 + (size_t)c->nbox * 8;
+        // status words as Status mirrors them: err, late, grand_total (64 bits, the
+        // upper ones 0), then the masses
+        const size_t status_bytes = 16 + (size_t)c->nbox * 8;
         c->err = (uint32_t*)c->alloc(status_bytes);
-        c->grand_total = c->err + 1;
-        c->mass_total = reinterpret_cast<double*>(c->err + 2);
+        c->late = c->err + 1;
+        c->grand_total = c->err + 2;
+        c->mass_total = reinterpret_cast<double*>(c->err + 4);
         c->scratch_cap = 2 * cap + (1u << 16);
         c->scratch = (uint64_t*)c->alloc(c->scratch_cap * 8);
         c->scratch_cursor = (unsigned long long*)c->alloc(16);
@@ -1555,7 +1563,7 @@ int hy_pm_kdk(hy_pm_ctx* c, uint64_t n, const double* x_in, const double* y_in, 
         if (masses && c->nbox > 1) fail(HY_EINVAL, "explicit masses take a single-box context");
         const double M = input_mass(c, nper, masses, uniform);
         if (sync) reset_status(c);
-            // keys (or records) of the previous fused step are valid for exactly its
+        // keys (or records) of the previous fused step are valid for exactly its
         // output positions
         const bool reuse = (flags & HY_REUSE_KEYS) != 0;
         const bool carried = reuse && c->keys_ready && c->keys_n == n && c->keys_x == x_in && c->keys_y == y_in &&
@@ -1566,9 +1574,10 @@ int hy_pm_kdk(hy_pm_ctx* c, uint64_t n, const double* x_in, const double* y_in, 
         const bool rec_out = has_next && !sync && !masses && c->rec_layout;
         c->keys_ready = c->rec_ready = false;
         // A synchronous call looks at the status once, at its end: the gather does
-        // nothing where the deposit failed, so a failed call leaves the state
-        // as it was.  Carried keys of changed positions fail that way, and the
-        // positions are routed afresh.
+        // nothing where the deposit or the transform failed, so such a call leaves
+        // the state as it was.  (A particle that fails in the gather itself keeps
+        // its state, all others are updated.)  Carried keys of changed positions
+        // fail in the deposit, and the positions are routed afresh.
         for (bool routed = carried;; routed = false) {
             run_deposit(c, n, x_in, y_in, z_in, masses, uniform, M, false, routed, carried_rec, rec_out);
             // counts are consumed by the scan above; the gather below accumulates the
@@ -1586,8 +1595,8 @@ int hy_pm_kdk(hy_pm_ctx* c, uint64_t n, const double* x_in, const double* y_in, 
                 a.acc_x = acc_x; a.acc_y = acc_y; a.acc_z = acc_z;
                 a.k_prev = k_prev; a.k_next = k_next; a.d_next = d_next;
                 a.has_prev = has_prev; a.has_next = has_next;
-                a.err = c->err;
-                a.gate = sync ? 1 : 0;
+                a.gate = sync ? c->err : nullptr;
+                a.err = sync ? c->late : c->err;
                 if (make_keys) {
                     a.next_counts = c->counts;
                     a.next_keys = c->keys;
@@ -1992,7 +2001,8 @@ int hy_pm_kdk_vjp(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, co
             a.coef_a = ksum;
             a.coef_b = ksum * uniform / dx3;
             a.lx = lx; a.ly = ly; a.lz = lz;
-            a.err = c->err;
+            a.gate = c->err;
+            a.err = c->late;
             launch_adj_gather(c, a);
         };
         if (c->prec == HY_PREC_FP64) gather(double{});
@@ -2019,7 +2029,8 @@ int hy_pm_density_vjp(hy_pm_ctx* c, uint64_t n, const double* x, const double* y
             a.chi = static_cast<const T*>(u_mesh);
             a.coef_b = coef * uniform;
             a.lx = lx; a.ly = ly; a.lz = lz;
-            a.err = c->err;
+            a.gate = c->err;
+            a.err = c->late;
             launch_adj_gather(c, a);
         };
         if (c->prec == HY_PREC_FP64) gather(double{});

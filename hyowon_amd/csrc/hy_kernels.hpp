@@ -2376,7 +2376,7 @@ struct GatherArgs {
     int has_prev;
     int has_next;
     uint32_t* err;
-    int gate;                   // do nothing where err is already set
+    const uint32_t* gate;       // do nothing where this word is set (another than err), or null
 };
 
 // Potential values of the 8 corners' centred differences around base cell
@@ -2517,7 +2517,7 @@ __device__ __forceinline__ bool stencil_force(const T* phi, const Geom& g, int i
 template <typename T, typename PT, bool O32, bool REC, bool OUT, bool CHUNK>
 __global__ void __launch_bounds__(256) k_gather_kdk(GatherArgs<T, PT> a) {
     if constexpr (!REC) {  // records are carried by asynchronous steps only
-        if (a.gate && *a.err) return;
+        if (a.gate && *a.gate) return;
     }
     // each XCD walks a contiguous particle range (spatially compact for
     // lattice-ordered particles), so potential lines are reused in its L2
@@ -2797,6 +2797,7 @@ struct SlotForceArgs {
     ForceRecord* force;
     DepRecord64* rec64;    // binary64
     const T* f[3];
+    const uint32_t* gate;  // do nothing where this word is set
     uint32_t* err;
 };
 
@@ -2804,7 +2805,7 @@ template <typename T, bool FORCE_SG, bool O32>
 __global__ void __launch_bounds__(256) k_slot_force(SlotForceArgs<T> a) {
     const uint64_t s = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     // a failed deposit (a particle without a slot) leaves records unwritten
-    if (s >= a.n || *a.err) return;
+    if (s >= a.n || *a.gate) return;
     const Geom& g = a.g;
     const int E = g.T;
     const uint32_t nT = (uint32_t)g.nT, ntiles = nT * nT * nT;
@@ -2852,7 +2853,8 @@ __global__ void __launch_bounds__(256) k_slot_force(SlotForceArgs<T> a) {
     }
 }
 
-// acc += g for every particle, its force read from its slot, where no error is set.
+// acc += g for every particle, its force read from its slot, where no error is
+// set (status: the error words of the deposit and transform and of the force).
 __device__ __forceinline__ void slot_value(const ForceRecord& q, double v[3]) {
     v[0] = q.wx;
     v[1] = q.wy;
@@ -2870,9 +2872,9 @@ __global__ void __launch_bounds__(256) k_commit_slots(uint64_t n, const uint32_t
                                                       const uint32_t* __restrict__ offsets,
                                                       const R* __restrict__ force, double* __restrict__ ax,
                                                       double* __restrict__ ay, double* __restrict__ az,
-                                                      const uint32_t* __restrict__ err) {
+                                                      const uint32_t* __restrict__ status) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n || *err) return;
+    if (p >= n || (status[0] | status[1])) return;
     double v[3];
     slot_value(force[offsets[keys[p]] + ranks[p]], v);
     ax[p] += v[0];
@@ -3079,9 +3081,9 @@ __global__ void __launch_bounds__(256) k_lpt_update(const double* __restrict__ p
 __global__ void k_commit_force(uint64_t n, const float* __restrict__ gx, const float* __restrict__ gy,
                                const float* __restrict__ gz, double* __restrict__ ax,
                                double* __restrict__ ay, double* __restrict__ az,
-                               const uint32_t* __restrict__ err) {
+                               const uint32_t* __restrict__ status) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n || *err) return;
+    if (p >= n || (status[0] | status[1])) return;
     ax[p] += (double)gx[p];
     ay[p] += (double)gy[p];
     az[p] += (double)gz[p];
@@ -3190,16 +3192,17 @@ struct AdjGatherArgs {
     double* lx;
     double* ly;
     double* lz;
+    const uint32_t* gate;  // do nothing where this word is set
     uint32_t* err;
 };
 
 // The potential and chi are read as z-contiguous vector runs, the 32 distinct
 // potential values once each (128^3 particles on 256^3, binary32: 196 us with
-// eight scalar 7-point stencils, 116 so).  Does nothing where err is set.
+// eight scalar 7-point stencils, 116 so).
 template <typename T, bool O32>
 __global__ void __launch_bounds__(256) k_adj_gather(AdjGatherArgs<T> a) {
     const uint64_t p = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (p >= a.n || *a.err) return;
+    if (p >= a.n || *a.gate) return;
     const Geom& g = a.g;
     const int N = g.N;
     int ix, iy, iz;
