@@ -425,7 +425,8 @@ struct ForceRecord {
 
 // Scatter into bucket order, writing the particle index and its deposit
 // record (and, where force is set, its force record at the same slot).  The bucket is recomputed from the current position and must equal
-// the stored key (keys carried over from the previous step are checked here).
+// the stored key (keys carried over from the previous step are checked here; a
+// mismatch also sets stale, a word of pinned host memory, where given).
 // R = DepRecord (binary32 fractions, masses / mass unit) or DepRecord64
 // (binary64 fractions and particle index, masses as given).
 template <typename R, typename MT>
@@ -435,7 +436,7 @@ __global__ void k_scatter_records(uint64_t n, const double* __restrict__ x, cons
                                   const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ offsets,
                                   uint32_t* __restrict__ order, R* __restrict__ rec,
                                   MT* __restrict__ rec_mass, uint32_t* __restrict__ err, double shift,
-                                  ForceRecord* __restrict__ force) {
+                                  ForceRecord* __restrict__ force, uint32_t* __restrict__ stale) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const uint32_t k = keys[p];
@@ -450,7 +451,12 @@ __global__ void k_scatter_records(uint64_t n, const double* __restrict__ x, cons
         return;
     }
     if (k == 0xffffffffu || box_of(p, g) * buckets_per_box(g) + bucket_of(bx, by, bz, g) != k) {
-        atomicOr(err, ERR_STALE_KEYS);
+        // one atomic per wave, one store to the host in all (2M of them took 2 ms)
+        if (__ffsll((unsigned long long)__ballot(1)) - 1 == (int)lane_id()) {
+            const uint32_t old = atomicOr(err, ERR_STALE_KEYS);
+            if (stale && !(old & ERR_STALE_KEYS))
+                __hip_atomic_store(stale, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         return;
     }
     const uint32_t dst = offsets[k] + ranks[p];
