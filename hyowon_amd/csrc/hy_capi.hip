@@ -507,6 +507,19 @@ long double mass_tol_factor(const hy_pm_ctx* c, uint64_t n) {
     return f;
 }
 
+// Whether the binary64 deposit's first launch takes its wide kernel (1024 records,
+// two workgroups per CU) or its narrow one (736, three): wide where the mean
+// records per tile say that tiles fit the one and not the other.  Density calls
+// on 256^3, ms, narrow / wide: 0.33 / 0.36 at 614 records, 0.37 / 0.40 at 705, 0.47 /
+// 0.38 at 737, 0.57 / 0.41 at 786, 0.63 / 0.47 at 988; even from 1070, where
+// no tile fits either; with explicit masses 0.45 / 0.45, 0.49 / 0.49, 0.60 / 0.47,
+// 0.69 / 0.51, 0.76 / 0.57.  The counts spread by about their square root.
+bool wide_deposit(const hy_pm_ctx* c, uint64_t n) {
+    const double edge = c->geom.T + 1.0, cells = (double)c->N * c->N * c->N * c->nbox;
+    const double mean = (double)n / cells * edge * edge * edge, spread = std::sqrt(mean);
+    return mean + spread > hy::DEP_CAP && mean - spread <= hy::DEP_CAP_WIDE;
+}
+
 // Also evaluates the routing identity and the mass bound on the device (error
 // bits reported by the synchronous check or hy_pm_check).
 // Binary32: the records lie in the layout start (dense offsets unless
@@ -521,12 +534,16 @@ void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, const uint32_t* start 
         };
         const uint64_t tiles = c->ntiles * c->nbox, jobs = std::min<uint64_t>(c->even_cap, 512);
         const bool t16 = c->geom.T == 16;
+        constexpr int CAP = hy::DEP_CAP, WIDE = hy::DEP_CAP_WIDE;
+        const bool wide = wide_deposit(c, P.n);
         if (P.masses) {
-            launch(t16 ? hy::k_deposit<16, true, false> : hy::k_deposit<0, true, false>, tiles);
-            launch(t16 ? hy::k_deposit<16, true, true> : hy::k_deposit<0, true, true>, jobs);
+            if (wide) launch(t16 ? hy::k_deposit<16, true, false, WIDE> : hy::k_deposit<0, true, false, WIDE>, tiles);
+            else launch(t16 ? hy::k_deposit<16, true, false, CAP> : hy::k_deposit<0, true, false, CAP>, tiles);
+            launch(t16 ? hy::k_deposit<16, true, true, CAP> : hy::k_deposit<0, true, true, CAP>, jobs);
         } else {
-            launch(t16 ? hy::k_deposit<16, false, false> : hy::k_deposit<0, false, false>, tiles);
-            launch(t16 ? hy::k_deposit<16, false, true> : hy::k_deposit<0, false, true>, jobs);
+            if (wide) launch(t16 ? hy::k_deposit<16, false, false, WIDE> : hy::k_deposit<0, false, false, WIDE>, tiles);
+            else launch(t16 ? hy::k_deposit<16, false, false, CAP> : hy::k_deposit<0, false, false, CAP>, tiles);
+            launch(t16 ? hy::k_deposit<16, false, true, CAP> : hy::k_deposit<0, false, true, CAP>, jobs);
         }
     } else {
         hy::DepFxParams Q{P, c->mass_unit, std::ldexp(c->mass_unit, -32), c->rec,

@@ -937,24 +937,28 @@ __device__ __forceinline__ void wg_exclusive_scan_lds(uint32_t* a, int count, ui
 //     its word counts, in time linear in its length; then the terms are formed
 //     64 at a time and added in order with lane reads, so a dense cell costs
 //     one addition latency per entry.
-// A tile with more than DEP_CAP records, or with a list for a wave, becomes 1 to
-// 64 jobs (boxes of the tile, one workgroup each) of a second launch; a job that still exceeds the
-// LDS lists its records in the scratch (when it has room) and halves its box
-// along the longest edge until the records fit.  A single cell with more than
-// DEP_CAP sources sorts its particle indices by themselves, in index ranges
-// that fit the LDS.
+// A tile with more than CAP records, or with a list for a wave, becomes jobs
+// (boxes of the tile, one workgroup each) of a second launch: as many as the
+// plan of its records makes, or 1 to 64 equal ones where it makes none.  A job
+// that still exceeds the LDS lists its records in the scratch (when it has
+// room) and halves its box along the longest edge until the records fit.  A
+// single cell with more than DEP_CAP sources sorts its particle indices by
+// themselves, in index ranges that fit the LDS.
 //
 // Bound by LDS latency (the chain counter -> scan -> entry -> record) and by
-// the 150 or so instructions per cell; DEP_CAP = 736 records (the 1/8
-// particles per cell of a mesh twice the lattice give about 614) keep the
-// workgroup's LDS at 53 KB, three per CU.  Measured against one thread per cell
+// the 150 or so instructions per cell.  CAP = 736 records (the 1/8 particles per
+// cell of a mesh twice the lattice give about 614) keep the workgroup's LDS at
+// 53 KB, three per CU (59 KB and two with masses); CAP = 1024, 66 KB and two, is
+// for loads whose tiles need it (the host's rule): with 736 alone 0.16 to 0.2
+// particles per cell went through the second launch and were 5 to 8% slower than
+// the kernel that this one replaced.  Measured against one thread per cell
 // merging four index-sorted source lists (and a whole-tile sort in global
 // memory above 1024 records): 16.8M lattice particles on 512^3 1.33 -> 0.85 ms,
 // 3M clustered particles with masses on 192^3 16.8 -> 2.2 ms, 8192 on 32^3
 // 162 -> 36 us.
 // ---------------------------------------------------------------------------
-constexpr int DEP_CAP = 736;
-constexpr int DEP_PER = (DEP_CAP + DEP_THREADS - 1) / DEP_THREADS;
+constexpr int DEP_CAP = 736;        // records of a job, and of a tile in the first launch's narrow kernel
+constexpr int DEP_CAP_WIDE = 1024;  // records of a tile in its wide kernel
 constexpr int DEP_SERIAL = 16;  // entries one thread sorts (its network's size) in the second launch ...
 constexpr int DEP_COMMON = 8;   // ... and in the first, whose 80 registers hold no larger network
 constexpr int DEP_JOB_RECORDS = 256;  // a tile of M records makes at most M / DEP_JOB_RECORDS jobs
@@ -962,18 +966,19 @@ constexpr int DEP_MAX_CELLS = DEP_MAX_T * DEP_MAX_T * DEP_MAX_T;
 constexpr int DEP_HEAVY = 8 * DEP_CAP / (DEP_SERIAL + 1) + 1;  // most lists longer than DEP_SERIAL
 constexpr int DEP_STACK = 16;                                   // boxes waiting (at most one per halving, 12)
 constexpr int DEP_BITS = 2 * ((DEP_CAP + 31) / 32);  // words of a list's bitmap: both x offsets
-static_assert(8 * DEP_CAP <= 65535 && DEP_CAP <= 8192, "16-bit list entries");
+static_assert(8 * DEP_CAP_WIDE <= 65535, "16-bit list entries");
 static_assert(DEP_BITS <= 64 && DEP_CAP % 16 == 0, "one lane per bitmap word; padded index scans");
 
 // LDS of the workgroup as one block (also the key array of a hot cell).
+template <int CAP>
 struct DepLds {
-    double fx[DEP_CAP], fy[DEP_CAP], fz[DEP_CAP];
+    double fx[CAP], fy[CAP], fz[CAP];
     uint32_t start[DEP_MAX_CELLS + 1];
-    alignas(16) uint32_t idx[DEP_CAP];  // particle index
-    uint16_t ent[8 * DEP_CAP]; // slot * 8 + corner (ox, oy, oz bits 2, 1, 0)
-    uint16_t cell[DEP_CAP];    // base cell in the tile, each axis + 1 in 5 bits; then ranks by particle index
+    alignas(16) uint32_t idx[CAP];  // particle index
+    uint16_t ent[8 * CAP]; // slot * 8 + corner (ox, oy, oz bits 2, 1, 0)
+    uint16_t cell[CAP];    // base cell in the tile, each axis + 1 in 5 bits; then ranks by particle index
 };
-constexpr uint32_t DEP_HOT_LDS = sizeof(DepLds) / sizeof(uint64_t);
+constexpr uint32_t DEP_HOT_LDS = sizeof(DepLds<DEP_CAP>) / sizeof(uint64_t);
 
 // Halvings (x, y, z in turn) of a tile of M > DEP_CAP records: uniform boxes
 // then hold 340 to 750 records.
@@ -1062,7 +1067,7 @@ __device__ __forceinline__ double wave_ordered_add(double sum, double term, int 
 constexpr int DEP_PLAN_EXT = (DEP_MAX_T + 1) * (DEP_MAX_T + 1) * (DEP_MAX_T + 1);
 constexpr uint32_t DEP_FRONTIER = 1024, DEP_LEAVES = 2048;
 constexpr int DEP_PLAN_LDS = DEP_PLAN_EXT + 2 * (int)DEP_FRONTIER + (int)DEP_LEAVES + 4;
-static_assert(DEP_PLAN_LDS * sizeof(uint32_t) <= sizeof(DepLds), "the plan fits the deposit's LDS");
+static_assert(DEP_PLAN_LDS * sizeof(uint32_t) <= sizeof(DepLds<DEP_CAP>), "the plan fits the deposit's LDS");
 
 template <typename BaseCell, typename SlotOf>
 __device__ __forceinline__ bool dep_plan_jobs(const DepParams& P, int T, uint32_t M, uint32_t gtile,
@@ -1167,11 +1172,13 @@ __device__ __forceinline__ bool dep_plan_jobs(const DepParams& P, int T, uint32_
 // list.  DENSE = true: the workgroups walk that list (the box
 // splitting and the hot cells in the common kernel would take its registers
 // from 80 to 145, three workgroups per CU to one).
-template <int TE, bool MASS, bool DENSE>
-__global__ void __launch_bounds__(DEP_THREADS) __attribute__((amdgpu_waves_per_eu(DENSE || MASS ? 4 : 6)))
+template <int TE, bool MASS, bool DENSE, int CAP>
+__global__ void __launch_bounds__(DEP_THREADS) __attribute__((amdgpu_waves_per_eu(DENSE || MASS || CAP > DEP_CAP ? 4 : 6)))
 k_deposit(DepParams P, double* __restrict__ mesh0) {
-    __shared__ __align__(16) DepLds S;
-    __shared__ double sh_m[MASS ? DEP_CAP : 1];
+    static_assert(!DENSE || CAP == DEP_CAP, "jobs hold DEP_CAP records");
+    constexpr int PER = (CAP + DEP_THREADS - 1) / DEP_THREADS;  // records per thread
+    __shared__ __align__(16) DepLds<CAP> S;
+    __shared__ double sh_m[MASS ? CAP : 1];
     __shared__ uint32_t sh_rs[DEP_NRANGES], sh_rc[DEP_NRANGES + 1];
     __shared__ uint8_t sh_rd[DEP_NRANGES], sh_rcls[DEP_NRANGES];
     __shared__ uint32_t sh_part[DEP_THREADS / 64];
@@ -1258,7 +1265,7 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
     };
 
     if constexpr (!DENSE) {
-        if (M > (uint32_t)DEP_CAP) {
+        if (M > (uint32_t)CAP) {
             if (!dep_plan_jobs(P, TT, M, gtile, base_cell, slot_of, reinterpret_cast<uint32_t*>(&S), &sh_nheavy)) leave(dep_split(M));
             if (lane == 0) wave_out[0] = ~0ull;
             return;
@@ -1350,11 +1357,11 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
             for (int i = tid; i <= cells; i += DEP_THREADS) S.start[i] = 0u;
             if constexpr (!DENSE) {
                 // both records of a thread in flight together
-                DepRecord64 rec[DEP_PER];
-                uint32_t slot[DEP_PER];
-                int d[DEP_PER];
+                DepRecord64 rec[PER];
+                uint32_t slot[PER];
+                int d[PER];
 #pragma unroll
-                for (int j = 0; j < DEP_PER; ++j) {
+                for (int j = 0; j < PER; ++j) {
                     const uint32_t v = (uint32_t)(tid + j * DEP_THREADS);
                     if (v < M) {
                         slot[j] = slot_of(v, d[j]);
@@ -1362,7 +1369,7 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
                     }
                 }
 #pragma unroll
-                for (int j = 0; j < DEP_PER; ++j) {
+                for (int j = 0; j < PER; ++j) {
                     const uint32_t v = (uint32_t)(tid + j * DEP_THREADS);
                     if (v < M) keep(v, slot[j], rec[j], base_cell(rec[j], d[j]));
                 }
@@ -1479,11 +1486,11 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
         // counting sort of the contributions by destination cell: corner o of a
         // record is cell c0 + ox sx + oy ez + oz of the box where it lies in it
         const int sx = ey * ez;
-        uint32_t rank[DEP_PER][4];  // two 16-bit ranks per word (a list holds at most DEP_CAP)
-        int cell0[DEP_PER];
-        uint32_t corners[DEP_PER];  // bit o: corner o lies in the box
+        uint32_t rank[PER][4];  // two 16-bit ranks per word (a list holds at most CAP)
+        int cell0[PER];
+        uint32_t corners[PER];  // bit o: corner o lies in the box
 #pragma unroll
-        for (int j = 0; j < DEP_PER; ++j) {
+        for (int j = 0; j < PER; ++j) {
             const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
             corners[j] = 0u;
             cell0[j] = 0;
@@ -1508,13 +1515,13 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
         __syncthreads();
         if constexpr (!DENSE) {
             if (sh_nheavy) {  // lists for whole waves
-                leave(0);
+                leave(M > (uint32_t)DEP_CAP ? dep_split(M) : 0);
                 return;
             }
         }
         wg_exclusive_scan_lds(S.start, cells + 1, sh_part);
 #pragma unroll
-        for (int j = 0; j < DEP_PER; ++j) {
+        for (int j = 0; j < PER; ++j) {
             const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
 #pragma unroll
             for (int o = 0; o < 8; ++o) {
@@ -1526,7 +1533,7 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
         }
         __syncthreads();
         auto term_of = [&](uint16_t e) -> double {
-            const uint32_t s = min((uint32_t)e >> 3, (uint32_t)DEP_CAP - 1u);  // empty network entries: any record
+            const uint32_t s = min((uint32_t)e >> 3, (uint32_t)CAP - 1u);  // empty network entries: any record
             const double fx = S.fx[s], fy = S.fy[s], fz = S.fz[s];
             double mm = P.uniform_mass;
             if constexpr (MASS) mm = sh_m[s];
@@ -1576,8 +1583,8 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
                     // read whether or not the entry exists (within the arrays): the
                     // reads of all entries go out together
                     const uint32_t at = at0 + (uint32_t)i;
-                    const uint32_t v = S.ent[min(at, 8u * DEP_CAP - 1u)];
-                    const uint32_t index = S.idx[min(v >> 3, (uint32_t)DEP_CAP - 1u)];
+                    const uint32_t v = S.ent[min(at, 8u * CAP - 1u)];
+                    const uint32_t index = S.idx[min(v >> 3, (uint32_t)CAP - 1u)];
                     const uint32_t top = 0x00100000u | (at >= b1 ? 1u << 18 : 0u) | ((v & 4u) << 14) | (index >> 16);
                     const uint64_t key = ((uint64_t)((uint32_t)i < n ? top : 0x7fe00000u) << 32) | (index << 16) | v;
                     k[i] = __longlong_as_double((long long)key);
@@ -1652,9 +1659,9 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
             const uint32_t m16 = (m + 15u) & ~15u;
             if ((uint32_t)tid < m16 - m) S.idx[m + (uint32_t)tid] = 0xffffffffu;
             __syncthreads();
-            uint32_t mine[DEP_PER], r[DEP_PER];
+            uint32_t mine[PER], r[PER];
 #pragma unroll
-            for (int j = 0; j < DEP_PER; ++j) {
+            for (int j = 0; j < PER; ++j) {
                 const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
                 mine[j] = s < m ? S.idx[s] : 0u;
                 r[j] = 0u;
@@ -1666,12 +1673,12 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
 #pragma unroll
-                    for (int j = 0; j < DEP_PER; ++j)
+                    for (int j = 0; j < PER; ++j)
                         r[j] += (q[k].x < mine[j] ? 1u : 0u) + (q[k].y < mine[j] ? 1u : 0u) +
                                 (q[k].z < mine[j] ? 1u : 0u) + (q[k].w < mine[j] ? 1u : 0u);
             }
 #pragma unroll
-            for (int j = 0; j < DEP_PER; ++j) {
+            for (int j = 0; j < PER; ++j) {
                 const uint32_t s = (uint32_t)(tid + j * DEP_THREADS);
                 if (s < m) S.cell[s] = (uint16_t)r[j];
             }
