@@ -141,6 +141,7 @@ struct hy_pm_ctx {
     uint32_t* offsets = nullptr;
     uint32_t* block_sums = nullptr;
     uint32_t* grand_total = nullptr;
+    uint32_t* groups = nullptr;    // distinct buckets of the probed waves (OrderProbe)
     uint32_t* xcounts = nullptr;   // x-plane bins (N)
     uint32_t* xoffsets = nullptr;  // N+1
     unsigned long long* mass_digits = nullptr;  // per box: exact deposited-mass digit counters
@@ -194,14 +195,16 @@ struct hy_pm_ctx {
     struct Status {
         uint32_t err;
         uint32_t late;
-        uint64_t total;
+        uint32_t total;
+        uint32_t groups;    // distinct keys of the probed waves (OrderProbe)
         double mass;
         double mass_in[2];  // sum and maximum of explicit masses
         double energy;      // potential energy of the call
         uint32_t stale;     // written by the scatter itself where a carried key is stale
+        uint32_t order;     // written by the scatter: groups
     };
     Status* hstatus = nullptr;
-    hipEvent_t scattered = nullptr;  // end of a scatter whose stale keys the host waits for
+    hipEvent_t scattered = nullptr;  // end of a scatter whose verdict the host waits for
 
     std::vector<void*> allocations;
 
@@ -357,11 +360,11 @@ void cap_scan(hy_pm_ctx* c, const uint32_t* cur, uint32_t* dense, uint32_t* capn
 void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const double* z, int mode,
                uint32_t* counts, uint32_t* offsets, uint64_t nb, uint32_t* order, bool carried = false,
                const double* masses = nullptr, uint32_t* capn = nullptr, double shift = 0.0,
-               hy::ForceRecord* force = nullptr, uint32_t* stale = nullptr) {
+               hy::ForceRecord* force = nullptr, uint32_t* stale = nullptr, hy::OrderProbe probe = {}) {
     if (!carried) {
         fill_u32(c, counts, nb);
         hipLaunchKernelGGL(hy::k_bucket_key, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y, z,
-                           c->geom, mode, c->keys, c->ranks, counts, c->err, shift);
+                           c->geom, mode, c->keys, c->ranks, counts, c->err, shift, probe);
         launch_check("k_bucket_key");
     }
     if (mode == 0 && c->prec == HY_PREC_FP32_MIXED && c->rec_layout) {
@@ -387,12 +390,12 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
     if (mode == 0 && c->prec == HY_PREC_FP32_MIXED) {
         hipLaunchKernelGGL((hy::k_scatter_records<hy::DepRecord, float>), dim3(blocks_for(n, 256)), dim3(256), 0,
                            c->stream, n, x, y, z, masses, 1.0 / c->mass_unit, c->geom, c->keys, c->ranks, offsets,
-                           order, c->rec, c->rec_mass, c->err, shift, force, stale);
+                           order, c->rec, c->rec_mass, c->err, shift, force, stale, probe);
         launch_check("k_scatter_records");
     } else if (mode == 0) {
         hipLaunchKernelGGL((hy::k_scatter_records<hy::DepRecord64, double>), dim3(blocks_for(n, 256)), dim3(256), 0,
                            c->stream, n, x, y, z, masses, 1.0, c->geom, c->keys, c->ranks, offsets, order,
-                           c->rec64, c->rec_mass64, c->err, shift, (hy::ForceRecord*)nullptr, stale);
+                           c->rec64, c->rec_mass64, c->err, shift, (hy::ForceRecord*)nullptr, stale, probe);
         launch_check("k_scatter_records");
     } else if (carried) {
         hipLaunchKernelGGL(hy::k_scatter_checked, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y,
@@ -405,7 +408,7 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
     }
 }
 
-void reset_status(hy_pm_ctx* c) { fill_u32(c, c->err, 2); }
+void reset_status(hy_pm_ctx* c) { fill_u32(c, c->err, 4); }
 
 // Copy err / late / grand total / deposited mass to the host and synchronise;
 // err holds the bits of both words.
@@ -743,6 +746,33 @@ void launch_slot_force(hy_pm_ctx* c, uint64_t n, hy::ForceRecord* force) {
     launch_check("k_slot_force");
 }
 
+// Probe of the particles' order for a force of n particles, whose result chooses
+// between the particle-order gather (or, sg, interpolation) and the one in record
+// order.  The measure is the number of distinct buckets among a wave's 64
+// particles, over about a thousand waves: near 8 per mean spacing in cells on
+// a lattice, which grows as its particles leave it, 64 in a shuffled set.  Both
+// sides, ms per call (particle / record order), lattices with displacements of
+// 1, 2 and 4 spacings (16.0, 17.0 and 18.8 buckets on 512^3 at half that side):
+//   binary32 512^3    2.53 / 2.83, 2.76 / 2.94, 3.08 / 3.05, shuffled 6.78 / 4.18
+//   binary32 1024^3   18.8 / 21.5 (14.9 buckets), 4 spacings 23.1 / 23.3 (17.4)
+//   TreePM 512^3      3.73 / 4.06, 4.07 / 4.21, 4.78 / 4.39, shuffled 8.16 / 5.56
+//   binary64 512^3    4.97 / 5.19, 6.49 / 6.51, 7.98 / 7.73, shuffled 9.52 / 6.52
+// Sets sorted by 4 or 16 cells (6 and 4 buckets) are 2 to 8% faster in particle
+// order.  The sides cross at 8.1 to 9.3 times the spacing in binary32 and at 8.1 to
+// 8.6 in binary64 and TreePM.  Below 2^20 particles the two are within 3%, the wait for
+// the probe not counted: record order, unprobed.
+hy::OrderProbe order_probe(hy_pm_ctx* c, uint64_t n, bool sg) {
+    hy::OrderProbe p{};
+    if (n < (1ull << 20)) return p;
+    const double spacing = std::cbrt((double)c->N * c->N * c->N * c->nbox / (double)n);
+    const uint64_t blocks = blocks_for(n, 256);
+    p.stride = (uint32_t)std::max<uint64_t>(1, blocks / 1024);
+    p.limit = (uint32_t)((c->prec == HY_PREC_FP32_MIXED && !sg ? 8.7 : 8.25) * spacing * (double)blocks_for(blocks, p.stride));
+    p.groups = c->groups;
+    p.host = &c->hstatus->order;
+    return p;
+}
+
 void require_pure_pm(const hy_pm_ctx* c, const char* what) {
     if (c->method != HY_METHOD_PURE_PM)
         fail(HY_EINVAL, std::string(what) + " takes a pure-PM context (the TreePM long-range force needs the "
@@ -877,12 +907,12 @@ void check_deposit(hy_pm_ctx* c, uint64_t n, const hy_pm_ctx::Status& st) {
 // also lay out the capacities of the records this step's gather writes.
 // shift: deposit the positions x - shift (the power spectrum's interlacing
 // partner), routed and wrapped as the reference's shifted copy would be.
-// stale: pinned word that the scatter sets where a carried key is stale; the event
-// scattered follows it.
+// stale: pinned word that the scatter sets where a carried key is stale; probe:
+// measures the order of the particles.  The event scattered follows either.
 void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const double* z,
                  const double* masses, double uniform, double Min, bool sync, bool carried = false,
                  bool carried_rec = false, bool rec_out = false, double shift = 0.0,
-                 hy::ForceRecord* force = nullptr, uint32_t* stale = nullptr) {
+                 hy::ForceRecord* force = nullptr, uint32_t* stale = nullptr, hy::OrderProbe probe = {}) {
     mark(c, 0);
     // the binary32 deposit reads records only: no particle order is written
     uint32_t* order = nullptr;
@@ -904,8 +934,8 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
         ovf = c->ovf_start;
     } else {
         bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, carried, masses, capn, shift, force,
-                  stale);
-        if (stale) hip_check(hipEventRecord(c->scattered, c->stream), "hipEventRecord");
+                  stale, probe);
+        if (stale || probe.groups) hip_check(hipEventRecord(c->scattered, c->stream), "hipEventRecord");
     }
     mark(c, HY_STAGE_BUCKET + 1);
     auto plan = plan_deposit(c, n, x, y, z, masses, uniform, Min, shift);
@@ -1179,12 +1209,13 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         }
         const uint64_t wave_words = c->prec == HY_PREC_FP64 ? hy::SA_WAVE_WORDS : 2;  // window, or digit-sum pair
         c->mass_waves = (unsigned long long*)c->alloc(wave_words * hy::SA_WAVES_PER_TILE * c->ntiles * c->nbox * 8);
-        // status words as Status mirrors them: err, late, grand_total (64 bits, the
-        // upper ones 0), then the masses
+        // status words as Status mirrors them: err, late, grand_total, groups, then
+        // the masses
         const size_t status_bytes = 16 + (size_t)c->nbox * 8;
         c->err = (uint32_t*)c->alloc(status_bytes);
         c->late = c->err + 1;
         c->grand_total = c->err + 2;
+        c->groups = c->err + 3;
         c->mass_total = reinterpret_cast<double*>(c->err + 4);
         c->scratch_cap = 2 * cap + (1u << 16);
         c->scratch = (uint64_t*)c->alloc(c->scratch_cap * 8);
@@ -1487,42 +1518,54 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             dx_ = s; dy_ = s + c->cap; dz_ = s + 2 * c->cap;
         }
         reset_status(c);
-        // The forces are gathered in record order.  Binary32: the force records
-        // lie behind the n records of the call (room for two per particle exists
-        // where the carried layout does; else in particle order).
+        // The forces are gathered in record order, or in particle order where the
+        // probed waves say that it keeps to the buckets; the same bits either way.  Binary32: the force
+        // records lie behind the n records of the call (room for two per particle
+        // exists where the carried layout does; else in particle order).
         hy::ForceRecord* slots = nullptr;
         static_assert(sizeof(hy::ForceRecord) == sizeof(hy::DepRecord), "force records behind the deposit records");
         if (c->rec_layout) slots = reinterpret_cast<hy::ForceRecord*>(c->rec + c->cap);
-        run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, false, false, false, false, 0.0, slots);
         const bool sg = c->method == HY_METHOD_TREEPM_LONG_RANGE;
+        const bool records = slots || c->prec == HY_PREC_FP64;
+        const hy::OrderProbe probe = records ? order_probe(c, n, sg) : hy::OrderProbe{};
+        run_deposit(c, n, dx_, dy_, dz_, dm, uniform, M, false, false, false, false, 0.0, slots, nullptr, probe);
         if (sg) run_fft_sg(c);
         else run_fft(c);
         if (collect) launch_potential_energy(c, n, dx_, dy_, dz_, dm, uniform);
-        if (c->prec == HY_PREC_FP64) {
-            launch_slot_force<double>(c, n, nullptr);
-        } else if (slots) {
-            launch_slot_force<float>(c, n, slots);
-        } else if (sg) {
-            hy::InterpArgs<float> a{};
-            a.n = n;
-            a.x = dx_; a.y = dy_; a.z = dz_;
-            a.f[0] = static_cast<const float*>(c->R);
-            a.f[1] = static_cast<const float*>(c->R2);
-            a.f[2] = static_cast<const float*>(c->R3);
-            a.out[0] = static_cast<float*>(c->gx);
-            a.out[1] = static_cast<float*>(c->gy);
-            a.out[2] = static_cast<float*>(c->gz);
-            a.meshes = 3;
-            launch_interp(c, a);
-        } else {
-            hy::GatherArgs<float, float> a{};
-            a.g = c->geom; a.n = n;
-            a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
-            a.err = c->err;
-            a.phi = static_cast<const float*>(c->R);
-            a.g_x = (float*)c->gx; a.g_y = (float*)c->gy; a.g_z = (float*)c->gz;
-            launch_gather(c, a);
+        bool in_order = !records;
+        if (probe.groups) {
+            hip_check(hipEventSynchronize(c->scattered), "hipEventSynchronize");
+            in_order = *const_cast<const volatile uint32_t*>(&c->hstatus->order) <= probe.limit;
         }
+        auto force = [&](auto tag) {
+            using T = decltype(tag);
+            if (!in_order) {
+                launch_slot_force<T>(c, n, slots);
+            } else if (sg) {
+                hy::InterpArgs<T> a{};
+                a.n = n;
+                a.x = dx_; a.y = dy_; a.z = dz_;
+                a.f[0] = static_cast<const T*>(c->R);
+                a.f[1] = static_cast<const T*>(c->R2);
+                a.f[2] = static_cast<const T*>(c->R3);
+                a.out[0] = static_cast<T*>(c->gx);
+                a.out[1] = static_cast<T*>(c->gy);
+                a.out[2] = static_cast<T*>(c->gz);
+                a.meshes = 3;
+                launch_interp(c, a);
+            } else {
+                hy::GatherArgs<T, T> a{};
+                a.g = c->geom; a.n = n;
+                a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
+                a.gate = c->err;
+                a.err = c->late;
+                a.phi = static_cast<const T*>(c->R);
+                a.g_x = (T*)c->gx; a.g_y = (T*)c->gy; a.g_z = (T*)c->gz;
+                launch_gather(c, a);
+            }
+        };
+        if (c->prec == HY_PREC_FP64) force(double{});
+        else force(float{});
         mark(c, HY_STAGE_GATHER_KDK + 1);
         end_call(c);
         if (collect)
@@ -1536,16 +1579,20 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
             hip_check(hipMemcpyAsync(cy, ay, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
             hip_check(hipMemcpyAsync(cz, az, n * 8, hipMemcpyHostToDevice, c->stream), "h2d");
         }
-        const dim3 grid(blocks_for(n, 256)), block(256);
-        if (c->prec == HY_PREC_FP64)
-            hipLaunchKernelGGL(hy::k_commit_slots<hy::DepRecord64>, grid, block, 0, c->stream, n, c->keys, c->ranks,
-                               c->offsets, c->rec64, cx, cy, cz, c->err);
-        else if (slots)
-            hipLaunchKernelGGL(hy::k_commit_slots<hy::ForceRecord>, grid, block, 0, c->stream, n, c->keys, c->ranks,
-                               c->offsets, slots, cx, cy, cz, c->err);
-        else
-            hipLaunchKernelGGL(hy::k_commit_force, grid, block, 0, c->stream, n, (const float*)c->gx,
-                               (const float*)c->gy, (const float*)c->gz, cx, cy, cz, c->err);
+        auto commit = [&](auto tag) {
+            using T = decltype(tag);
+            using R = std::conditional_t<sizeof(T) == 4, hy::ForceRecord, hy::DepRecord64>;
+            const dim3 grid(blocks_for(n, 256)), block(256);
+            const void* rec = sizeof(T) == 4 ? (const void*)slots : (const void*)c->rec64;
+            if (in_order)
+                hipLaunchKernelGGL(hy::k_commit_force<T>, grid, block, 0, c->stream, n, (const T*)c->gx,
+                                   (const T*)c->gy, (const T*)c->gz, cx, cy, cz, c->err);
+            else
+                hipLaunchKernelGGL(hy::k_commit_slots<R>, grid, block, 0, c->stream, n, c->keys, c->ranks, c->offsets,
+                                   static_cast<const R*>(rec), cx, cy, cz, c->err);
+        };
+        if (c->prec == HY_PREC_FP64) commit(double{});
+        else commit(float{});
         launch_check("k_commit_force");
         const auto st = fetch_status(c);
         check_deposit(c, n, st);

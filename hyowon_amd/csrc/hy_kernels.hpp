@@ -50,10 +50,12 @@ __device__ __forceinline__ uint32_t record_cell(int bx, int by, int bz, const Ge
 // Wave-aggregated integer atomic: lanes with equal keys reserve consecutive
 // slots.  Groups are found with ballots first; then every group leader issues
 // its atomic in the same instruction, so a wave pays one atomic round trip.
-// Returns this lane's rank (slot) within its bucket.
-__device__ __forceinline__ uint32_t aggregated_rank(uint32_t* counts, uint32_t key, bool valid) {
+// Returns this lane's rank (slot) within its bucket; groups: the wave's number of
+// distinct keys.
+__device__ __forceinline__ uint32_t aggregated_rank(uint32_t* counts, uint32_t key, bool valid, uint32_t& groups) {
     const uint32_t lane = lane_id();
     uint64_t remaining = __ballot(valid);
+    groups = 0;
     int my_leader = (int)lane;
     uint64_t my_mask = 0;
     while (remaining) {
@@ -65,6 +67,7 @@ __device__ __forceinline__ uint32_t aggregated_rank(uint32_t* counts, uint32_t k
             my_mask = mask;
         }
         remaining &= ~mask;
+        ++groups;
     }
     uint32_t old = 0;
     if (valid && (int)lane == my_leader) old = atomicAdd(&counts[key], (uint32_t)__popcll(my_mask));
@@ -75,10 +78,19 @@ __device__ __forceinline__ uint32_t aggregated_rank(uint32_t* counts, uint32_t k
 // mode 0: deposit buckets; mode 1: reference x-plane bins (key = base x).
 // shift: positions are routed as x - shift (the interlacing partner of the
 // power-spectrum estimator; 0 otherwise, where x - 0 is x exactly).
+// probe: how well the order of the particles keeps to the buckets (OrderProbe).
+struct OrderProbe {
+    uint32_t* groups;   // distinct keys of the probed waves, added up (null: not probed)
+    uint32_t* host;     // their sum in pinned host memory, written by the scatter
+    uint32_t stride;    // the first wave of every stride-th workgroup is probed
+    uint32_t limit;     // groups above it: the order does not keep to the buckets
+};
+
 __global__ void k_bucket_key(uint64_t n, const double* __restrict__ x, const double* __restrict__ y,
                              const double* __restrict__ z, Geom g, int mode,
                              uint32_t* __restrict__ keys, uint32_t* __restrict__ ranks,
-                             uint32_t* __restrict__ counts, uint32_t* __restrict__ err, double shift) {
+                             uint32_t* __restrict__ counts, uint32_t* __restrict__ err, double shift,
+                             OrderProbe probe) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool in = p < n;
     uint32_t key = 0;
@@ -91,7 +103,9 @@ __global__ void k_bucket_key(uint64_t n, const double* __restrict__ x, const dou
         if (ok) key = mode == 0 ? box_of(p, g) * buckets_per_box(g) + bucket_of(bx, by, bz, g) : (uint32_t)bx;
         else atomicOr(err, ERR_POSITION_NONFINITE);
     }
-    const uint32_t rank = aggregated_rank(counts, key, in && ok);
+    uint32_t groups;
+    const uint32_t rank = aggregated_rank(counts, key, in && ok, groups);
+    if (probe.groups && blockIdx.x % probe.stride == 0 && threadIdx.x == 0) atomicAdd(probe.groups, groups);
     if (in && !ok) key = 0xffffffffu;
     if (in) {
         keys[p] = key;
@@ -424,7 +438,8 @@ struct ForceRecord {
 };
 
 // Scatter into bucket order, writing the particle index and its deposit
-// record (and, where force is set, its force record at the same slot).  The bucket is recomputed from the current position and must equal
+// record (and, where force is set and a probe has not found the particles in
+// order, its force record at the same slot).  The bucket is recomputed from the current position and must equal
 // the stored key (keys carried over from the previous step are checked here; a
 // mismatch also sets stale, a word of pinned host memory, where given).
 // R = DepRecord (binary32 fractions, masses / mass unit) or DepRecord64
@@ -436,9 +451,15 @@ __global__ void k_scatter_records(uint64_t n, const double* __restrict__ x, cons
                                   const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ offsets,
                                   uint32_t* __restrict__ order, R* __restrict__ rec,
                                   MT* __restrict__ rec_mass, uint32_t* __restrict__ err, double shift,
-                                  ForceRecord* __restrict__ force, uint32_t* __restrict__ stale) {
+                                  ForceRecord* __restrict__ force, uint32_t* __restrict__ stale,
+                                  OrderProbe probe) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
+    if (probe.groups) {
+        const uint32_t groups = *probe.groups;
+        if (p == 0) __hip_atomic_store(probe.host, groups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (groups <= probe.limit) force = nullptr;
+    }
     const uint32_t k = keys[p];
     int bx, by, bz;
     double fx, fy, fz;
@@ -2655,7 +2676,8 @@ __global__ void __launch_bounds__(256) k_gather_kdk(GatherArgs<T, PT> a) {
                 s0 = a.rec_start[next_key];
                 s1 = a.rec_start[next_key + 1];
             }
-            const uint32_t rank = aggregated_rank(a.next_counts, next_key, have);
+            uint32_t groups;
+            const uint32_t rank = aggregated_rank(a.next_counts, next_key, have, groups);
             uint32_t slot = 0;
             bool over = false;
             if (have) {
@@ -2680,7 +2702,8 @@ __global__ void __launch_bounds__(256) k_gather_kdk(GatherArgs<T, PT> a) {
                 }
             }
         } else {
-            const uint32_t rank = aggregated_rank(a.next_counts, next_key, have);
+            uint32_t groups;
+            const uint32_t rank = aggregated_rank(a.next_counts, next_key, have, groups);
             if (live) {
                 __builtin_nontemporal_store(key_ok ? next_key : 0xffffffffu, &a.next_keys[p]);
                 __builtin_nontemporal_store(rank, &a.next_ranks[p]);
@@ -2793,14 +2816,15 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<T> a) {
 }
 
 // Force of the particles in deposit-record order (slot s of the bucket layout),
-// the result over the slot's force record (binary64: over the fractions).  Consecutive slots
-// share a 16^3 tile, so the stencil lines stay in L1 and L2 whatever the order
-// of the particle arrays; in particle order a shuffled set fetches 12 to 16
-// lines per particle from beyond L2 (20M shuffled particles on 512^3: 4.43 ms
-// in particle order, 0.78 here, with 0.28 more in the scatter and 0.33 more in
-// the commit; binary64, 3M on 192^3: 0.51 ->
-// 0.12, with 0.03 more in the commit).  On lattice order it is even: TreePM, 16.8M on 512^3, 1.23 ->
-// 0.90, with 0.14 + 0.06 more around it.  FORCE_SG false: centred gradient of
+// the result over the slot's force record (binary64: over the fractions).
+// Consecutive slots share a 16^3 tile, so the stencil lines stay in L1 and L2
+// whatever the order of the particle arrays; in particle order a shuffled set
+// fetches 12 to 16 lines per particle from beyond L2 (20M shuffled particles on
+// 512^3: 4.43 ms in particle order, 0.78 here, with 0.28 more in the scatter and
+// 0.33 more in the commit; binary64, 3M on 192^3: 0.51 -> 0.12, with 0.03 more in
+// the commit).  Where the order keeps to the buckets it is slower (16.8M on 512^3
+// near their lattice: 0.42 -> 0.70, with 0.14 and 0.07 more around it); the host
+// chooses by a probe of the order (order_probe).  FORCE_SG false: centred gradient of
 // f[0] (one potential per box); true: interpolation of the force meshes f[0..2].
 template <typename T>
 struct SlotForceArgs {
@@ -3091,8 +3115,9 @@ __global__ void __launch_bounds__(256) k_lpt_update(const double* __restrict__ p
 
 // Transactional commit for the reference-shaped force entry: acc += g where no
 // error is set.
-__global__ void k_commit_force(uint64_t n, const float* __restrict__ gx, const float* __restrict__ gy,
-                               const float* __restrict__ gz, double* __restrict__ ax,
+template <typename T>
+__global__ void k_commit_force(uint64_t n, const T* __restrict__ gx, const T* __restrict__ gy,
+                               const T* __restrict__ gz, double* __restrict__ ax,
                                double* __restrict__ ay, double* __restrict__ az,
                                const uint32_t* __restrict__ status) {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
