@@ -136,7 +136,6 @@ struct hy_pm_ctx {
     // particles
     uint32_t* keys = nullptr;
     uint32_t* ranks = nullptr;
-    uint32_t* order = nullptr;
     uint32_t* counts = nullptr;
     uint32_t* offsets = nullptr;
     uint32_t* block_sums = nullptr;
@@ -397,10 +396,6 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
                            c->stream, n, x, y, z, masses, 1.0, c->geom, c->keys, c->ranks, offsets, order,
                            c->rec64, c->rec_mass64, c->err, shift, (hy::ForceRecord*)nullptr, stale, probe);
         launch_check("k_scatter_records");
-    } else if (carried) {
-        hipLaunchKernelGGL(hy::k_scatter_checked, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y,
-                           z, c->geom, c->keys, c->ranks, offsets, order, c->err);
-        launch_check("k_scatter_checked");
     } else {
         hipLaunchKernelGGL(hy::k_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, c->keys,
                            c->ranks, offsets, order);
@@ -460,7 +455,6 @@ DepositPlan plan_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double
     P.uniform_mass = uniform;
     P.pos_shift = shift;
     P.offsets = c->offsets;
-    P.order = c->order;
     P.rec64 = c->rec64;
     P.rec_mass64 = c->rec_mass64;
     P.n = n;
@@ -468,7 +462,6 @@ DepositPlan plan_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double
     P.inv_volume = inv_volume;
     P.total_mass = Min;
     P.cells_real = cells;
-    P.centred_scale = inv_volume * (1.0 / cells);
     {
         // 1/(N_c dx^3) as the reference forms it: (((1/N_c)/dx)/dx)/dx in long double
         long double S = 1.0L;
@@ -914,8 +907,6 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
                  bool carried_rec = false, bool rec_out = false, double shift = 0.0,
                  hy::ForceRecord* force = nullptr, uint32_t* stale = nullptr, hy::OrderProbe probe = {}) {
     mark(c, 0);
-    // the binary32 deposit reads records only: no particle order is written
-    uint32_t* order = nullptr;
     uint32_t* capn = rec_out ? c->cap_next : nullptr;
     const uint32_t* start = nullptr;
     const uint32_t* ovf = nullptr;
@@ -933,7 +924,7 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
         start = c->cap_cur;
         ovf = c->ovf_start;
     } else {
-        bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, order, carried, masses, capn, shift, force,
+        bucketize(c, n, x, y, z, 0, c->counts, c->offsets, c->nball, nullptr, carried, masses, capn, shift, force,
                   stale, probe);
         if (stale || probe.groups) hip_check(hipEventRecord(c->scattered, c->stream), "hipEventRecord");
     }
@@ -1184,7 +1175,6 @@ int hy_pm_create(const hy_pm_desc* desc, hy_pm_ctx** out) {
         const uint64_t cap = std::max<uint64_t>(c->cap, 1);
         c->keys = (uint32_t*)c->alloc(cap * 4);
         c->ranks = (uint32_t*)c->alloc(cap * 4);
-        c->order = (uint32_t*)c->alloc(cap * 4);
         c->ntiles = (uint64_t)c->geom.nT * c->geom.nT * c->geom.nT;
         c->nb = c->ntiles * 8;
         c->nball = c->nb * c->nbox;

@@ -393,29 +393,6 @@ __global__ void k_place_overflow(const uint32_t* __restrict__ ovf_count, const u
     }
 }
 
-// Scatter with keys made by an earlier call: each key is checked against the
-// bucket of the current position first (ERR_STALE_KEYS on a mismatch).
-__global__ void k_scatter_checked(uint64_t n, const double* __restrict__ x, const double* __restrict__ y,
-                                  const double* __restrict__ z, Geom g, const uint32_t* __restrict__ keys,
-                                  const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ offsets,
-                                  uint32_t* __restrict__ order, uint32_t* __restrict__ err) {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const uint32_t k = keys[p];
-    int bx, by, bz;
-    double f;
-    const bool ok = cic_axis(x[p], g, bx, f) && cic_axis(y[p], g, by, f) && cic_axis(z[p], g, bz, f);
-    if (!ok) {
-        atomicOr(err, ERR_POSITION_NONFINITE);
-        return;
-    }
-    if (k == 0xffffffffu || box_of(p, g) * buckets_per_box(g) + bucket_of(bx, by, bz, g) != k) {
-        atomicOr(err, ERR_STALE_KEYS);
-        return;
-    }
-    order[offsets[k] + ranks[p]] = (uint32_t)p;
-}
-
 // Binary64 deposit record: tile-local base cell (12 bits) and above it the tile
 // in its box, the particle index (the reference's per-cell summation order is
 // by index) and the binary64 fractions; after the slot-order force kernel, the
@@ -588,7 +565,6 @@ k_canonicalize(uint64_t nb, const uint32_t* __restrict__ offsets, uint32_t* __re
 // ===========================================================================
 constexpr int DEP_THREADS = 512;
 constexpr int DEP_MAX_T = 16;
-constexpr int DEP_EXT = (DEP_MAX_T + 1) * (DEP_MAX_T + 1) * (DEP_MAX_T + 1);  // 4913
 constexpr int DEP_NRANGES = 20;
 
 // ---------------------------------------------------------------------------
@@ -797,15 +773,13 @@ struct DepParams {
     double uniform_mass;
     double pos_shift;         // positions are deposited as x - pos_shift (0: as given)
     const uint32_t* offsets;  // bucket offsets (nb+1)
-    const uint32_t* order;    // bucketed particle indices
     const DepRecord64* rec64; // binary64 deposit records in bucket order
     const double* rec_mass64; // binary64 masses in bucket order (explicit masses, or signed adjoint values)
-    uint64_t n;               // particle count (bound of every order entry)
+    uint64_t n;               // particle count (bound of every record's index)
     double mean_mass;         // M / N_cells
     double inv_volume;        // 1 / dx^3
     double total_mass;        // M (exact input mass)
     double cells_real;        // N_cells as double
-    double centred_scale;     // inv_volume / N_cells (normalize path, unused)
     uint64_t norm_mant;       // 1/(N_cells dx^3) as a 64-bit mantissa ...
     int norm_exp;             // ... times 2^norm_exp (the reference holds it in long double)
     int direct;               // 1: (m - mean) * inv_volume ; 0: fma-centred path
@@ -1027,11 +1001,6 @@ __device__ __forceinline__ uint32_t dep_box(int T, int levels, uint32_t j) {
         code |= ((uint32_t)lo << (4 * a)) | ((uint32_t)(e - 1) << (12 + 4 * a));
     }
     return code;
-}
-
-// Order of a list entry: the x offset (reference's phase), then the particle index.
-__device__ __forceinline__ uint64_t dep_entry_key(uint16_t e, const uint32_t* idx) {
-    return ((uint64_t)(e & 4u) << 30) | idx[e >> 3];
 }
 
 // Minimum and maximum of ordinary binary64 numbers as the bare instructions
