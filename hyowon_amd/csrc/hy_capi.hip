@@ -36,7 +36,9 @@ struct HyError {
 [[noreturn]] void fail(int code, const std::string& what) { throw HyError{code, what}; }
 
 void hip_check(hipError_t e, const char* what) {
-    if (e != hipSuccess) fail(HY_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
+    if (e == hipSuccess) return;
+    (void)hipGetLastError();  // reported here: not again by the next launch's check
+    fail(HY_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
 template <typename F>
@@ -185,6 +187,7 @@ struct hy_pm_ctx {
     void* kd = nullptr;          // k component per index, 0 on the Nyquist index
     void* ic_kc = nullptr;       // binary64 k tables of the 1LPT displacements (allocated on first use)
     void* ic_kd = nullptr;
+    bool ic_ready = false;
     void* pk_aux = nullptr;      // interlaced partner spectrum (allocated on first use)
     double* pk_tab = nullptr;    // k components, windows, alias factors (3N), shell edges
     double* pk_part = nullptr;   // workgroup shell partials
@@ -938,10 +941,8 @@ void run_deposit(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, con
 
 // Device staging of host-pointer calls: positions and masses (4 * cap), accelerations (3 * cap).
 void ensure_host_staging(hy_pm_ctx* c) {
-    if (!c->hpos) {
-        c->hpos = (double*)c->alloc(c->cap * 4 * sizeof(double));
-        c->hacc = (double*)c->alloc(c->cap * 3 * sizeof(double));
-    }
+    if (!c->hpos) c->hpos = (double*)c->alloc(c->cap * 4 * sizeof(double));
+    if (!c->hacc) c->hacc = (double*)c->alloc(c->cap * 3 * sizeof(double));
 }
 
 // Device copy of a host-pointer call's masses.
@@ -1358,17 +1359,18 @@ int hy_ic_lpt(hy_pm_ctx* c, uint64_t n_side, const void* delta_k, double p_facto
             fail(HY_EINVAL, "1LPT particle lattice must divide the IC mesh");
         if (!std::isfinite(p_factor)) fail(HY_EINVAL, "Invalid start-scaled LPT normalization");
         set_device(c);
-        if (!c->ic_kc) {
+        if (!c->ic_ready) {
             std::vector<double> kc(N), kd(N);
             for (uint64_t m = 0; m < N; ++m) {
                 const int64_t mode = m <= N / 2 ? (int64_t)m : (int64_t)m - (int64_t)N;
                 kc[m] = 2.0 * std::numbers::pi * (double)mode / c->geom.L;
                 kd[m] = (N % 2 == 0 && m == N / 2) ? 0.0 : kc[m];
             }
-            c->ic_kc = c->alloc(N * sizeof(double));
-            c->ic_kd = c->alloc(N * sizeof(double));
+            if (!c->ic_kc) c->ic_kc = c->alloc(N * sizeof(double));
+            if (!c->ic_kd) c->ic_kd = c->alloc(N * sizeof(double));
             hip_check(hipMemcpy(c->ic_kc, kc.data(), N * sizeof(double), hipMemcpyHostToDevice), "upload");
             hip_check(hipMemcpy(c->ic_kd, kd.data(), N * sizeof(double), hipMemcpyHostToDevice), "upload");
+            c->ic_ready = true;
         }
         reset_status(c);
         const uint64_t NH = N / 2 + 1;
@@ -1948,14 +1950,17 @@ void launch_adj_gather(hy_pm_ctx* c, const hy::AdjGatherArgs<T>& a) {
 
 constexpr uint32_t ABS_MAX_BLOCKS = 256;
 
+// Each buffer by itself: a call that ran out of memory half way leaves the rest to
+// the next one.
 void ensure_adjoint_workspace(hy_pm_ctx* c) {
-    if (c->adj_phi) return;
     const size_t bytes = (size_t)c->N * c->N * c->N * c->real_bytes;
-    c->adj_phi = c->alloc(bytes);
-    for (auto& a : c->adj_a) a = c->alloc(bytes);
-    c->adj_max = (double*)c->alloc(3 * ABS_MAX_BLOCKS * sizeof(double));
-    hip_check(hipHostMalloc((void**)&c->hadj_max, 3 * ABS_MAX_BLOCKS * sizeof(double), hipHostMallocDefault),
-              "hipHostMalloc");
+    if (!c->adj_phi) c->adj_phi = c->alloc(bytes);
+    for (auto& a : c->adj_a)
+        if (!a) a = c->alloc(bytes);
+    if (!c->adj_max) c->adj_max = (double*)c->alloc(3 * ABS_MAX_BLOCKS * sizeof(double));
+    if (!c->hadj_max)
+        hip_check(hipHostMalloc((void**)&c->hadj_max, 3 * ABS_MAX_BLOCKS * sizeof(double), hipHostMallocDefault),
+                  "hipHostMalloc");
 }
 
 // Runs f with the context's real mesh (deposit target, transform input and
