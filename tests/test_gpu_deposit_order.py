@@ -1,7 +1,8 @@
 """The binary64 deposit's work splits, bit for bit against the oracle: tiles
-whose records exceed the workgroup's LDS (halved into boxes), long cell lists
-(one wave each), single cells hotter than the LDS list and than the LDS key
-array, tiles that are not 16 cells wide, explicit masses."""
+whose records exceed the workgroup's LDS (jobs planned from their record counts;
+where no plan fits: test_gpu_deposit_fallback.py), long cell lists (one wave each),
+single cells hotter than the LDS list and than the LDS key array, tiles that are
+not 16 cells wide, explicit masses."""
 import numpy as np
 import pytest
 
@@ -21,8 +22,10 @@ SPLITS = [
     (8, 8.0, 500, 5000, 1.0),        # tile edge 8, periodic neighbours are the tile itself
     (32, 32.0, 4000, 3000, 0.4),     # cells above the LDS list
     (32, 40.0, 4000, 30000, 0.3),    # cells above the LDS key array
-    (16, 16.0, 1, 767, 0.05),        # 768 records: the largest single box
-    (16, 16.0, 1, 768, 0.05),        # 769
+    # one cell's neighbourhood, 1124 and 1126 records with the periodic duplicates: planned
+    # (record counts at the kernels' capacities: test_gpu_deposit_capacity.py)
+    (16, 16.0, 1, 767, 0.05),
+    (16, 16.0, 1, 768, 0.05),
 ]
 
 
