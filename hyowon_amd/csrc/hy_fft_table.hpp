@@ -24,7 +24,7 @@ struct FftKernels {
     FftPass<T> x_fwd;  // forward-only x pass of the spectral estimators (in place on B)
     FftPass<T> z_fwd;  // z r2c pass of the spectral estimators (stores kz <= mode_limit only)
     FftPass<T> x_inv;  // inverse-only x pass of the IC displacements (in place on B)
-    FftPass<T> sg[3];  // spectral-gradient x, y^-1 and z^-1 passes (TreePM long range; variant 0)
+    FftPass<T> sg[3];  // spectral-gradient x (fft_x_variant), y^-1 and z^-1 passes (variant 0; TreePM long range)
     bool sg_x_dual = false;  // sg[0] writes the -i k_x and the plain inverse from one read of B
     FftPass<T> sg_y_dual;    // y^-1 pass writing the -i k_y and the plain inverse from one read of B (or none)
     int variants = 0;  // launch variants compiled for this size
@@ -34,15 +34,35 @@ struct FftKernels {
 // Sizes below this have one launch variant (their passes are latency-bound and
 // the variants collapse onto the same row counts).
 constexpr int kFftTunedFrom = 192;
-// Variant of the x passes that come in one (spectral gradient, forward or
-// inverse only) from that size up.
-constexpr int kFftXVariant = 3;
 
 // Defined in hy_fft_f32.hip / hy_fft_f64.hip; false for an unsupported size.
 bool lookup_fft(int N, FftKernels<float>& out);
 bool lookup_fft(int N, FftKernels<double>& out);
 
 #ifdef HY_FFT_INSTANTIATE
+// Variant of the x passes with a Green multiply (the others of theirs are the
+// autotuner's): they need LDS for the exchange only, so small workgroups keep more
+// of them resident: 20 KB on 2^a meshes, as long as that makes a whole wave (at
+// 1024 in binary64 it holds one row, 32 threads: 5.79 ms, the spectral gradient
+// 11.0), else 40 KB.  Against 80 KB: 512^3 binary32 0.39 -> 0.28 ms, binary64
+// 0.71 -> 0.60; 1024^3 binary32 1.91 -> 1.61, binary64 3.77 -> 3.41, its spectral
+// gradient 6.48 -> 6.40; 384^3 binary32 0.126 -> 0.107, its spectral gradient 0.28 ->
+// 0.19, binary64 0.34 and 0.34.
+template <typename T, int N>
+constexpr int fft_x_variant() {
+    if (N < kFftTunedFrom) return 0;
+    return (N & (N - 1)) == 0 && TLCfg<T, N, (N / 2 + 1) * N, 3>::THREADS >= 64 ? 3 : 1;
+}
+
+// ... and of the forward or inverse x passes, one transform each, which hold half the
+// registers: 20 KB also where that is half a wave (1024^3 binary64 3.23 ms, 3.41 with
+// 80 KB), but 80 KB on the large binary32 meshes (1024^3 1.45 ms, 1.52 with 20 KB).
+template <typename T, int N>
+constexpr int fft_x_dft_variant() {
+    if (N < kFftTunedFrom || (N >= 512 && sizeof(T) == 4)) return 0;
+    return (N & (N - 1)) == 0 ? 3 : 1;
+}
+
 template <typename T, int N, int V>
 void fill_variant(FftKernels<T>& k) {
     using RZ = TLCfg<T, N / 2, N, V>;
@@ -53,9 +73,11 @@ void fill_variant(FftKernels<T>& k) {
     k.pass[FFT_X_GREEN][V] = {k_tl_x_green<T, N, V>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
     k.pass[FFT_Y_BWD][V] = {k_tl_y_bwd<T, N, V>, RY::ROWS, RY::THREADS, RY::LDS_BYTES};
     k.pass[FFT_Z_C2R][V] = {k_tl_z_c2r<T, N, V>, RZ::ROWS, RZ::THREADS, RZ::LDS_BYTES};
-    if constexpr (V == (N >= kFftTunedFrom ? kFftXVariant : 0)) {
+    if constexpr (V == fft_x_dft_variant<T, N>()) {
         k.x_fwd = {k_tl_x_dft<T, N, V, -1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
         k.x_inv = {k_tl_x_dft<T, N, V, +1>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
+    }
+    if constexpr (V == fft_x_variant<T, N>()) {
         if constexpr (sizeof(T) == 4) {
             // binary32: the second held column fits the register file
             k.sg[0] = {k_tl_x_green_dual<T, N, V>, RX::ROWS, RX::THREADS, RX::X_LDS_BYTES};
@@ -74,17 +96,15 @@ void fill_variant(FftKernels<T>& k) {
 }
 
 // Variants a context starts with, from the measured times of all four:
-//   x + Green: the pass needs LDS for its exchange only, so small workgroups
-//     keep more of them resident: 20 KB on 2^a meshes (512^3 binary32 0.39 ->
-//     0.28 ms, binary64 0.71 -> 0.60), 40 KB on 3*2^a (384^3 0.126 -> 0.107);
+//   x + Green: fft_x_variant;
 //   256^3 y and y^-1: 40 KB (0.025 -> 0.021 ms);
-//   192^3 z c2r: 64 rows in binary32 (64 boxes 1.06 -> 0.70 ms), and 16 in
-//     binary64 with z r2c (0.023 -> 0.019, 0.022 -> 0.017 ms).
+//   192^3 z c2r: 64 rows in binary32 (one box 0.0165 -> 0.0152 ms, 64 boxes 1.06 ->
+//     0.70), and 16 in binary64 with z r2c (one box 0.022 -> 0.017 and 0.022 ->
+//     0.019 ms, 64 boxes 1.28 -> 1.27 and 1.27 -> 1.23).
 template <typename T, int N>
 constexpr int fft_plan(int pass) {
-    constexpr bool pow2 = (N & (N - 1)) == 0;
     if (N < kFftTunedFrom) return 0;
-    if (pass == FFT_X_GREEN) return pow2 ? 3 : 1;
+    if (pass == FFT_X_GREEN) return fft_x_variant<T, N>();
     if (N == 256 && (pass == FFT_Y_FWD || pass == FFT_Y_BWD)) return 1;
     if (N == 192 && sizeof(T) == 4 && pass == FFT_Z_C2R) return 2;
     if (N == 192 && sizeof(T) == 8 && (pass == FFT_Z_R2C || pass == FFT_Z_C2R)) return 1;
