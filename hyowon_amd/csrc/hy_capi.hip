@@ -365,7 +365,7 @@ void bucketize(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, const
                hy::ForceRecord* force = nullptr, uint32_t* stale = nullptr, hy::OrderProbe probe = {}) {
     if (!carried) {
         fill_u32(c, counts, nb);
-        hipLaunchKernelGGL(hy::k_bucket_key, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y, z,
+        hipLaunchKernelGGL(probe.groups ? hy::k_bucket_key<true> : hy::k_bucket_key<false>, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, x, y, z,
                            c->geom, mode, c->keys, c->ranks, counts, c->err, shift, probe);
         launch_check("k_bucket_key");
     }
@@ -1549,8 +1549,7 @@ int hy_pm_force(hy_pm_ctx* c, uint64_t n, const double* x, const double* y, cons
                 hy::GatherArgs<T, T> a{};
                 a.g = c->geom; a.n = n;
                 a.x_in = dx_; a.y_in = dy_; a.z_in = dz_;
-                a.gate = c->err;
-                a.err = c->late;
+                a.err = c->late;  // no gate: the commit has one
                 a.phi = static_cast<const T*>(c->R);
                 a.g_x = (T*)c->gx; a.g_y = (T*)c->gy; a.g_z = (T*)c->gz;
                 launch_gather(c, a);

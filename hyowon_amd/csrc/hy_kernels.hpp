@@ -78,7 +78,7 @@ __device__ __forceinline__ uint32_t aggregated_rank(uint32_t* counts, uint32_t k
 // mode 0: deposit buckets; mode 1: reference x-plane bins (key = base x).
 // shift: positions are routed as x - shift (the interlacing partner of the
 // power-spectrum estimator; 0 otherwise, where x - 0 is x exactly).
-// probe: how well the order of the particles keeps to the buckets (OrderProbe).
+// PROBE: counts how well the order of the particles keeps to the buckets.
 struct OrderProbe {
     uint32_t* groups;   // distinct keys of the probed waves, added up (null: not probed)
     uint32_t* host;     // their sum in pinned host memory, written by the scatter
@@ -86,6 +86,7 @@ struct OrderProbe {
     uint32_t limit;     // groups above it: the order does not keep to the buckets
 };
 
+template <bool PROBE>
 __global__ void k_bucket_key(uint64_t n, const double* __restrict__ x, const double* __restrict__ y,
                              const double* __restrict__ z, Geom g, int mode,
                              uint32_t* __restrict__ keys, uint32_t* __restrict__ ranks,
@@ -105,7 +106,9 @@ __global__ void k_bucket_key(uint64_t n, const double* __restrict__ x, const dou
     }
     uint32_t groups;
     const uint32_t rank = aggregated_rank(counts, key, in && ok, groups);
-    if (probe.groups && blockIdx.x % probe.stride == 0 && threadIdx.x == 0) atomicAdd(probe.groups, groups);
+    if constexpr (PROBE) {
+        if (blockIdx.x % probe.stride == 0 && threadIdx.x == 0) atomicAdd(probe.groups, groups);
+    }
     if (in && !ok) key = 0xffffffffu;
     if (in) {
         keys[p] = key;
