@@ -70,9 +70,9 @@ def step_alg_bytes(n_p: int, N: int, real: int) -> float:
 
 
 STAGE_KERNEL = {"bucket": "hy::k_cap_apply", "deposit": "void hy::k_deposit_fixed<16>",
-                "gather_kdk": "void hy::k_gather_kdk<float, float, true, true, false"}  # name prefixes
-FFT_KERNEL = {"fft_z_r2c": "k_fft_z_r2c", "fft_y_fwd": "k_fft_y_fwd", "fft_x_green": "k_fft_x_green",
-              "fft_y_bwd": "k_fft_y_bwd", "fft_z_c2r": "k_fft_z_c2r"}
+                "gather_kdk": "void hy::k_gather_kdk<float, float, true, true, false, false>"}
+FFT_KERNEL = {"fft_z_r2c": "k_tl_z_r2c", "fft_y_fwd": "k_tl_y_fwd", "fft_x_green": "k_tl_x_green",
+              "fft_y_bwd": "k_tl_y_bwd", "fft_z_c2r": "k_tl_z_c2r"}
 
 
 def measured_traffic(stage: str, n_side: int, N: int, prec: str, plan: dict):
@@ -85,11 +85,12 @@ def measured_traffic(stage: str, n_side: int, N: int, prec: str, plan: dict):
         prof = json.load(f)
     if stage in FFT_KERNEL:
         v = plan["variant"][stage[4:]]
-        sg = ", 0" if stage in ("fft_x_green", "fft_y_bwd", "fft_z_c2r") else ""  # spectral-gradient flag
-        name = f"void hy::{FFT_KERNEL[stage].replace('k_fft_', 'k_tl_')}<float, {N}, {v}{sg}>"
+        # spectral-gradient flag of the x, y^-1 and z^-1 passes, pruning flag of z r2c
+        flag = {"fft_x_green": ", 0", "fft_y_bwd": ", 0", "fft_z_c2r": ", 0", "fft_z_r2c": ", false"}.get(stage, "")
+        name = f"void hy::{FFT_KERNEL[stage]}<float, {N}, {v}{flag}>"
     else:
         name = STAGE_KERNEL.get(stage)
-    k = next((v for n, v in prof.get("kernels", {}).items() if n.startswith(name)), None)
+    k = prof.get("kernels", {}).get(name)  # the exact instantiation: another one's bytes are not this stage's
     return (k["traffic_bytes"] if k else None), os.path.relpath(path, ROOT)
 
 
