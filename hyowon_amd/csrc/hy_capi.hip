@@ -561,7 +561,8 @@ void launch_deposit(hy_pm_ctx* c, const hy::DepParams& P, const uint32_t* start 
     // 2048 records per workgroup: the workgroups of a box meet at its few digit
     // words and its ticket, so fewer are faster (64 boxes of 192^3, 54 -> 7
     // workgroups each: 243 -> 89 us); up to 256, one per CU, where the records
-    // themselves (32 MB for 1024^3) take longer
+    // themselves take longer (32 MB for 1024^3: 65 us with 64 workgroups, 44 with
+    // 128, 40 with 256, binary64 145, 88 and 82; 512^3 16 and 18, 24 and 21)
     const dim3 rgrid((uint32_t)std::min<uint64_t>(256, blocks_for(waves, 2048)), c->nbox);
     if (c->prec == HY_PREC_FP64)
         hipLaunchKernelGGL(hy::k_mass_finish, rgrid, dim3(256), 0, c->stream, c->mass_waves, waves, c->mass_digits,
@@ -1637,9 +1638,9 @@ int hy_pm_kdk(hy_pm_ctx* c, uint64_t n, const double* x_in, const double* y_in, 
         c->keys_ready = c->rec_ready = false;
         // A synchronous call looks at the status once, at its end: the gather does
         // nothing where the deposit or the transform failed, so such a call leaves
-        // the state as it was.  (A particle that fails in the gather itself keeps
-        // its state, all others are updated.)  Carried keys of changed positions
-        // fail in the deposit, and the positions are routed afresh.
+        // the state as it was, and costs a transform.  (A particle that fails in the
+        // gather itself keeps its state, all others are updated.)  Carried keys of
+        // changed positions fail in the scatter, and the positions are routed afresh.
         for (bool routed = carried;; routed = false) {
             // From 2^24 cells up the host looks at the keys' verdict while the deposit
             // runs, so stale keys do not cost a transform (512^3 binary32 4.75 ->

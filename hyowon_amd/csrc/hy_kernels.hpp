@@ -959,7 +959,7 @@ constexpr int DEP_CAP = 736;        // records of a job, and of a tile in the fi
 constexpr int DEP_CAP_WIDE = 1024;  // records of a tile in its wide kernel
 constexpr int DEP_SERIAL = 16;  // entries one thread sorts (its network's size) in the second launch ...
 constexpr int DEP_COMMON = 8;   // ... and in the first, whose 80 registers hold no larger network
-constexpr int DEP_JOB_RECORDS = 256;  // a tile of M records makes at most M / DEP_JOB_RECORDS jobs
+constexpr int DEP_JOB_RECORDS = 256;  // a tile of M records is cut evenly into at most M / DEP_JOB_RECORDS jobs
 constexpr int DEP_MAX_CELLS = DEP_MAX_T * DEP_MAX_T * DEP_MAX_T;
 constexpr int DEP_HEAVY = 8 * DEP_CAP / (DEP_SERIAL + 1) + 1;  // most lists longer than DEP_SERIAL
 constexpr int DEP_STACK = 16;                                   // boxes waiting (at most one per halving, 12)
@@ -1270,9 +1270,12 @@ k_deposit(DepParams P, double* __restrict__ mesh0) {
     int depth = 1;
     while (depth > 0) {
         // The box stack written at the end of the last trip, and that box's LDS
-        // reads.  The wait is explicit: at this loop header the compiler left
-        // the barrier's own lgkmcnt wait out, and a wave that read the stack
-        // ahead of its write went through other barriers than the rest.
+        // reads.  The wait is explicit: with one thread's LDS write on a path that
+        // ended in continue and no barrier behind it, the compiler left the wait
+        // of the header's barrier out, and a wave that read the stack ahead of its
+        // write went through other barriers than the rest.  Such a write has its
+        // barrier before the continue here, and every barrier of the compiled
+        // kernels an LDS wait on all paths to it.
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         __syncthreads();
         --depth;
@@ -2151,10 +2154,10 @@ __global__ void __launch_bounds__(256) k_mass_finish(const unsigned long long* _
     }
 }
 
-// Binary32: the waves' digit-sum pairs (s0, s1) added up per workgroup (below
-// 2^54 each: at most 2^13 waves of under 2^41 per thread at the grid's 2^16
-// threads per box and a mesh of 4096^3), and the workgroup's exact total
-// (s0 + s1 2^32) * unit * 2^-32 added to the box's counters as digits.
+// Binary32: the waves' digit-sum pairs (s0, s1) added up per workgroup (a 1024^3
+// mesh has 2^21 waves of under 2^41 each, so any grid's sums stay below 2^62), and
+// the workgroup's exact total (s0 + s1 2^32) * unit * 2^-32 added to the box's counters
+// as digits.
 __global__ void __launch_bounds__(256) k_mass_finish_fixed(const unsigned long long* __restrict__ waves,
                                                            uint64_t waves_per_box, double unit,
                                                            unsigned long long* digits, uint32_t* tickets,
@@ -2212,9 +2215,10 @@ __global__ void __launch_bounds__(256) k_mass_finish_fixed(const unsigned long l
 // identity of src/gravity/pm_solver.cpp:120-130, rounded once.  Each mass is
 // three 32-bit digits from its limb; a thread keeps six digit sums from one
 // limb below its first mass, which takes masses within a factor 2^64 of each
-// other, and other masses go to LDS counters.  Bound by the read of the
-// masses (8 B each); the host pass that it replaces copied them and took
-// about 3 ns per mass (3M masses: 9.4 ms -> 0.03 ms).
+// other, and other masses go to LDS counters.  Bound by the atomics, not by the
+// read: 256 threads meet at the same few LDS words after about eleven masses each,
+// and the workgroups at the same few global ones (3M masses 75 us, 0.32 TB/s; the
+// host pass that it replaces copied them and took 9.4 ms).
 __global__ void __launch_bounds__(256) k_input_mass(uint64_t n, const double* __restrict__ m,
                                                     unsigned long long* digits, unsigned long long* max_bits,
                                                     uint32_t* ticket, double* __restrict__ out) {

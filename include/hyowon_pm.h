@@ -19,8 +19,12 @@
  *    other streams must be ordered by the caller (or pass that stream).
  *  - One context owns one HIP stream and its mesh workspace; calls on a
  *    context must be serialised (as PMSolver, include/cosmo_nbody/mesh/
- *    mass_assignment.hpp:44-45).  All device memory is allocated by
- *    hy_pm_create; the force and step entry points allocate nothing.
+ *    mass_assignment.hpp:44-45).  hy_pm_create allocates the device memory of
+ *    steps, device-pointer forces, densities and transforms.  Allocated on a
+ *    context's first use, and kept: the partial sums of HY_COLLECT_POTENTIAL, the
+ *    staging of HY_HOST_POINTERS calls, the adjoint workspace of hy_pm_kdk_vjp
+ *    (four meshes), the shell sums of hy_pm_power_spectrum and the partner
+ *    spectrum of an interlaced one, the tables of hy_ic_lpt.
  */
 #ifndef HYOWON_PM_H
 #define HYOWON_PM_H
@@ -255,7 +259,8 @@ int hy_pm_autotune(hy_pm_ctx* ctx, uint32_t reps, hy_fft_tuning* out);
 
 /* Gather schedule.  The fused gather walks particle arrays held in Lagrangian
  * lattice order (n = S^3, S a multiple of 256 or rows that fill at least 7/8 of
- * their 64-particle chunks) in column tiles of TX x TY lattice rows, so the blocks resident on one XCD share that XCD's L2.
+ * their 64-particle chunks) in column tiles of TX x TY lattice rows, so the blocks
+ * resident on one XCD share that XCD's L2.
  * hy_pm_autotune_gather deposits and solves for the given positions (single
  * box, pure PM, uniform mass), times the gather under each candidate number
  * of rows per tile (0 = particle order, 16, 64, 256, 1024; ms_out[5] receives
@@ -391,8 +396,8 @@ typedef struct {
  * CIC deposit and r2c transform on the context's mesh and workspace, then the
  * shell sums on the device.  masses == NULL selects the uniform mass.  bins
  * (host memory) receives opts->num_bins shells.  Single-box contexts only.
- * An interlaced estimate allocates a partner spectrum and staging for the
- * shifted positions on first use.  Synchronous. */
+ * An interlaced estimate allocates a partner spectrum on first use.
+ * Synchronous. */
 int hy_pm_power_spectrum(hy_pm_ctx* ctx, uint64_t n, const double* x, const double* y, const double* z,
                          const double* masses, double uniform_mass, const hy_pk_options* opts,
                          hy_pk_bin* bins, uint32_t flags);
