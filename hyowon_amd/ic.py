@@ -11,7 +11,8 @@ rescaled by the growth table's (D1(a_start)/D1(1))^2 and interpolated as a
 natural cubic spline in ln k -- all evaluated by libhyowon_pm (hy_linear_power,
 hy_ic_mode_variance, hy_growth).  The table written here is the synthetic BBKS
 spectrum P(k) = A k^n_s T(k)^2 (Bardeen et al. 1986, q = k/Gamma) over
-1e-4..1e2 h/Mpc, A normalised to sigma_8 at z = 0.
+1e-4..1e2 h/Mpc, A normalised to sigma_8 at z = 0; the default cosmology's is
+the file beside this module.
 
 rng="philox" draws the reference's mode-keyed Philox field
 (src/ic/random_field.cpp); rng="torch" draws real-space white noise with
@@ -21,6 +22,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import os
 from dataclasses import dataclass
 from functools import lru_cache
 
@@ -115,6 +117,16 @@ def _bbks_amplitude(n_s: float, gamma: float, sigma8: float) -> float:
 
 @lru_cache(maxsize=8)
 def _bbks_table(c: Cosmology, k_min: float = 1e-4, k_max: float = 1e2, per_decade: int = 100) -> str:
+    # numpy's pow and log1p differ by a few last places between hosts with and
+    # without AVX-512, so the default cosmology's rows are read, not computed:
+    # the same seed then gives the same ICs, bit for bit, on every host
+    if (c, k_min, k_max, per_decade) == (Cosmology(), 1e-4, 1e2, 100):
+        with open(os.path.join(os.path.dirname(__file__), "bbks_default_table.txt"), encoding="ascii") as f:
+            return f.read()
+    return _bbks_rows(c, k_min, k_max, per_decade)
+
+
+def _bbks_rows(c: Cosmology, k_min: float, k_max: float, per_decade: int) -> str:
     decades = math.log10(k_max / k_min)
     n = int(round(decades * per_decade)) + 1
     k = k_min * 10.0 ** (np.arange(n) * (decades / (n - 1)))

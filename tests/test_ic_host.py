@@ -138,6 +138,22 @@ def test_product_bbks_table_is_the_golden_one():
     assert ic.Cosmology().table() == str(g["table"])
 
 
+def test_default_bbks_table_is_the_closed_form():
+    """The default cosmology's stored rows are those the closed form gives: the
+    header and every number to 1e-13, some thirty times the few last places by
+    which hosts differ in pow and log1p."""
+    from hyowon_amd import ic
+    c = ic.Cosmology()
+    stored, rows = (t.splitlines() for t in (c.table(), ic._bbks_rows(c, 1e-4, 1e2, 100)))
+    assert len(stored) == len(rows)
+    for a, b in zip(stored, rows):
+        if a.startswith("#") and "A=" not in a:
+            assert a == b
+        else:
+            u, v = (np.array(t.split("A=")[-1].split(), float) for t in (a, b))
+            assert np.allclose(u, v, rtol=1e-13, atol=0)
+
+
 def test_linear_power_growth_rescaling_and_header_checks(L):
     """P(k, z) / P(k, 0) = (D1(a)/D1(1))^2 up to the spline's rounding, at the
     knots exactly interpolated; a header that disagrees with the cosmology is
